@@ -37,13 +37,13 @@ namespace {
 // (femx_mesh_upload cuts tet4 meshes into <= 256-element blocks, hexa8 into <= 128)
 template <int NPE>
 constexpr int threads_for() { return NPE == 4 ? 256 : 128; }
-constexpr int RING = 64; // per-step diagnostic rows kept on the device
 
 // diagnostic row layout: 0..5 min/max u v w, 6,7 min/max tau, 8,9 min/max
 // lambda, 10 v-CFL max, 11 a-CFL max, 12 l-CFL max, 13,14 min/max E,
-// 15,16 min/max nu, 17 max |u|^2 (the log columns of :1601-1630)
+// 15,16 min/max nu, 17 max |u|^2 (the log columns of :1601-1630).  The log row
+// holds the step it belongs to in one more column.
 enum { D_UMIN = 0, D_TAU = 6, D_LAM = 8, D_VCFL = 10, D_ACFL = 11, D_LCFL = 12, D_E = 13, D_NU = 15, D_UMOD = 17,
-       D_COLS = 18 };
+       D_COLS = 18, D_STEP = 18, D_ROW = 19 };
 __host__ __device__ constexpr bool d_is_min(int c) {
   return c == 0 || c == 2 || c == 4 || c == D_TAU || c == D_LAM || c == D_E || c == D_NU;
 }
@@ -149,8 +149,8 @@ struct SupgArgs {
   int *err;
   double *eblk;              // [nblk][D_COLS] per-block rows: node extrema, element diagnostics (DIAG)
   int *halt;                 // INT_MAX or the step that exceeded EXITCOND
-  const double *prev_row;    // previous step's diagnostic row (exit check), or null
   int step_id;
+  int want_row;              // the step's log row is made: write the block's row
   SupgConst k;
 };
 
@@ -176,7 +176,15 @@ __device__ __forceinline__ void lpos_load(const uint16_t *lpos, int e, int ps[NP
   }
 }
 
-__device__ __forceinline__ bool halted(const int *halt) { return __builtin_nontemporal_load(halt) != INT_MAX; }
+// The exit condition (:1635-1643): the workgroups that form the new states of
+// step `step` and see |u|^2 above the threshold put the step into *halt; the
+// rest of that step still runs, every later step's work is skipped.  It
+// replaces a test of the previous step's reduced maximum, so a step needs no
+// reduction unless its log row is asked for.
+__device__ __forceinline__ bool halted(const int *halt, int step) { return __builtin_nontemporal_load(halt) < step; }
+__device__ __forceinline__ void exit_check(double m2, const SupgConst &k, int *halt, int step) {
+  if (m2 > k.exit2) atomicMin(halt, step);
+}
 
 // SUPG node update of one node (:1510-1514 update, :1519-1521 BCs,
 // :1527-1561 fixed DOFs): returns nothing, writes sol_p of the next step.
@@ -216,15 +224,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
   __shared__ double pu[PSEP ? 256 : 1], pv[PSEP ? 256 : 1], pw[PSEP ? 256 : 1];
   __shared__ T sres[DYN ? 3 * NPE * SB : 1];
   const int tid = threadIdx.x;
-  if (halted(a.halt)) return;
-  if (DYN && a.prev_row) {
-    // exit condition of the previous step (:1635-1643), decided identically by every block
-    const double m2 = a.prev_row[D_UMOD];
-    if (m2 > a.k.exit2) {
-      if (tid == 0) atomicMin(a.halt, a.step_id - 1);
-      return;
-    }
-  }
+  if (halted(a.halt, a.step_id)) return;
   const int n0 = a.node_off[blk], nn = a.node_off[blk + 1] - n0;
   const int e0 = a.elem_off[blk], ne = a.elem_off[blk + 1] - e0;
   const bool has_e = tid < ne;
@@ -704,7 +704,8 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         static_cast<double4 *>(a.partials)[psl] = make_double4(F[0], F[1], F[2], 0.0);
     }
   }
-  block_node_store<SB>(nv, nm2[0], a.eblk + (long)row * D_COLS);
+  exit_check(nm2[0], a.k, a.halt, a.step_id);
+  if (a.want_row) block_node_store<SB>(nv, nm2[0], a.eblk + (long)row * D_COLS);
 }
 
 template <typename T, int NPE, bool BHAT, bool DYN, bool PRESS, bool PSEP, bool DIAG>
@@ -713,30 +714,31 @@ __global__ __launch_bounds__(threads_for<NPE>(), 2) void supg_block(SupgArgs<T> 
 }
 
 
-// Reduce the per-block rows into this step's ring row (one workgroup).
-// Reduction of the per-block rows to the step's log row, in two stages: 32
-// workgroups each fold a strided share of the rows, all columns at once in
-// registers, into one partial row; one wave folds the partial rows with all
-// of its loads in flight together.
+// The log row of one step, made for the last step of a call (and for every
+// step while the element diagnostics are on: the l-CFL column is a running
+// maximum since the first step, the reference sets l_CFL_max once before its
+// time loop, :996, and resets only the v- and a-CFL maxima per step,
+// :1078-1079; it is carried in *lcfl).  Reduction of the per-workgroup rows
+// in two stages: 32 workgroups each fold a strided share of the rows, all
+// columns at once in registers, into one partial row; one wave folds the
+// partial rows with all of its loads in flight together.  Up to
+// DIAG_ONE_PASS rows one workgroup does both.  A separate launch after the
+// fix-up: folded by the fix-up's last workgroup instead, each of its
+// workgroups paid a device-scope fence (22 us against 6 us at 85k hexa).
 constexpr int DIAG_PARTS = 32;
-constexpr int DIAG_ONE_PASS = 2048;  // up to this many rows, one workgroup and one launch
-// The l-CFL column is a running maximum since the first step (the reference
-// sets l_CFL_max once before its time loop, :996, and resets only the v- and
-// a-CFL maxima per step, :1078-1079): the kernel that writes the step's row
-// folds in the previous step's row (prev, null on the first step).
-// One workgroup of 256 threads folds the rows of workgroups part, part +
-// nparts, ... into out[0 .. D_COLS).  AT: the fix-up's rows (nblk) were
-// written by other workgroups of the running kernel, so they are read with
-// device-scope atomic loads (coherent across the XCDs' L2 caches); the
-// element blocks' rows come from the previous kernel.
-template <bool AT>
-__device__ __forceinline__ double ld_row(const double *p) {
-  if constexpr (AT) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else return *p;
+constexpr int DIAG_ONE_PASS = 2048;
+__device__ __forceinline__ void row_store(int c, double v, double *row, double *lcfl, int step) {
+  if (c == D_LCFL) {
+    v = fmax(v, *lcfl);
+    *lcfl = v;
+  }
+  row[c] = v;
+  if (c == 0) row[D_STEP] = (double)step;
 }
-template <bool AT>
+// One workgroup of 256 threads folds the rows of workgroups part, part +
+// nparts, ... into out[0 .. D_COLS), or into the log row (lcfl not null).
 __device__ __forceinline__ void diag_fold(const double *eblk, int ne_blk, const double *nblk, int nn_blk,
-                                          int with_elem, double *out, const double *prev, int part, int nparts) {
+                                          int with_elem, double *out, double *lcfl, int step, int part, int nparts) {
   double m[D_COLS];
 #pragma unroll
   for (int c = 0; c < D_COLS; c++) m[c] = d_identity(c);
@@ -747,7 +749,7 @@ __device__ __forceinline__ void diag_fold(const double *eblk, int ne_blk, const 
 #pragma unroll
     for (int c = 0; c < D_COLS; c++)
       if (c < 6 || c == D_UMOD) {
-        const double x = ld_row<AT>(nblk + (long)b * D_COLS + c);
+        const double x = nblk[(long)b * D_COLS + c];
         m[c] = d_is_min(c) ? fmin(m[c], x) : fmax(m[c], x);
       }
   }
@@ -773,22 +775,22 @@ __device__ __forceinline__ void diag_fold(const double *eblk, int ne_blk, const 
     const int c = threadIdx.x;
     double v = red[0][c];
     for (int w = 1; w < 4; w++) v = d_is_min(c) ? fmin(v, red[w][c]) : fmax(v, red[w][c]);
-    if (c == D_LCFL && prev) v = fmax(v, prev[D_LCFL]);
-    out[c] = v;
+    if (lcfl) row_store(c, v, out, lcfl, step);
+    else out[c] = v;
   }
 }
 
 __global__ __launch_bounds__(256) void supg_diag_partial(const double *eblk, int ne_blk, const double *nblk,
-                                                         int nn_blk, int with_elem, double *part, const int *halt,
-                                                         const double *prev) {
-  if (halted(halt)) return;
-  diag_fold<false>(eblk, ne_blk, nblk, nn_blk, with_elem, part + (long)blockIdx.x * D_COLS, prev, blockIdx.x,
-                   gridDim.x);
+                                                         int nn_blk, int with_elem, double *part, double *lcfl,
+                                                         const int *halt, int step) {
+  if (halted(halt, step)) return;
+  diag_fold(eblk, ne_blk, nblk, nn_blk, with_elem, lcfl ? part : part + (long)blockIdx.x * D_COLS, lcfl, step,
+            blockIdx.x, gridDim.x);
 }
 
-__global__ __launch_bounds__(64) void supg_diag_final(const double *part, int np, double *row, const int *halt,
-                                                      const double *prev) {
-  if (halted(halt)) return;
+__global__ __launch_bounds__(64) void supg_diag_final(const double *part, int np, double *row, double *lcfl,
+                                                      const int *halt, int step) {
+  if (halted(halt, step)) return;
   if (threadIdx.x < D_COLS) {
     const int c = threadIdx.x;
     double x[DIAG_PARTS];
@@ -797,9 +799,19 @@ __global__ __launch_bounds__(64) void supg_diag_final(const double *part, int np
     double v = d_identity(c);
 #pragma unroll
     for (int q = 0; q < DIAG_PARTS; q++) v = d_is_min(c) ? fmin(v, x[q]) : fmax(v, x[q]);
-    if (c == D_LCFL && prev) v = fmax(v, prev[D_LCFL]);
-    row[c] = v;
+    row_store(c, v, row, lcfl, step);
   }
+}
+
+// The rows of a state's velocity extrema from the state itself (the log row
+// of a step that the exit condition made the last one of its call).
+__global__ __launch_bounds__(256) void supg_state_rows(int N, const double4 *U, double *nblk) {
+  double nv[6], m2 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 6; i++) nv[i] = d_identity(D_UMIN + i);
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n < N) node_extrema(U[n], nv, m2);
+  block_node_store<256>(nv, m2, nblk + (long)blockIdx.x * D_COLS);
 }
 
 struct SupgFix {
@@ -817,51 +829,33 @@ struct SupgFix {
   const int *row_off;
   const double4 *rows;
   int *err;
-  const int *halt;
+  int *halt;
+  int step_id;
+  int want_row;  // the step's log row is made: write the workgroup's row
   double *nblk;  // [workgroups][D_COLS]: node columns of each workgroup's row
-  // few rows: the fix-up's last workgroup folds this step's rows into the
-  // log row (NULL: a separate reduction does)
-  double *fold_row;
-  const double *fold_prev, *eblk;
-  int ne_blk, with_elem;
-  unsigned *fold_count;  // workgroups done, reset by the last one
   SupgConst k;
 };
 
 template <typename T>
 __device__ __forceinline__ void fixup_node(const SupgFix &a, int s, double nv[6], double &nm2);
 
-// Fix-up workgroup wg of nwg of one mesh.
+// Fix-up workgroup wg of one mesh.
 template <typename T>
-__device__ __forceinline__ void supg_fixup_run(const SupgFix &a, const int wg, const int nwg) {
-  if (halted(a.halt)) return;
+__device__ __forceinline__ void supg_fixup_run(const SupgFix &a, const int wg) {
+  if (halted(a.halt, a.step_id)) return;
   const int s = wg * 256 + (int)threadIdx.x;
   double nv[6], nm2[1] = {0.0};
 #pragma unroll
   for (int i = 0; i < 6; i++) nv[i] = d_identity(D_UMIN + i);
   if (s < a.n_sh) fixup_node<T>(a, s, nv, nm2[0]);
+  exit_check(nm2[0], a.k, a.halt, a.step_id);
   // this workgroup's row of velocity extrema and max |u|^2 (:604-655)
-  block_node_store<256>(nv, nm2[0], a.nblk + (long)wg * D_COLS);
-  if (a.fold_row) {
-    // the last workgroup to finish folds every row (its own and the
-    // others', made visible by their fences before they counted)
-    __shared__ bool last;
-    if (threadIdx.x == 0) {
-      __threadfence();
-      last = atomicAdd(a.fold_count, 1u) == (unsigned)nwg - 1u;
-    }
-    __syncthreads();
-    if (last) {
-      __threadfence();
-      diag_fold<true>(a.eblk, a.ne_blk, a.nblk, nwg, a.with_elem, a.fold_row, a.fold_prev, 0, 1);
-      if (threadIdx.x == 0) *a.fold_count = 0u;
-    }
-  }
+  if (a.want_row) block_node_store<256>(nv, nm2[0], a.nblk + (long)wg * D_COLS);
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void supg_fixup(SupgFix a) {
-  supg_fixup_run<T>(a, blockIdx.x, gridDim.x);
+  supg_fixup_run<T>(a, blockIdx.x);
 }
 
 template <typename T>
@@ -985,10 +979,9 @@ struct femx_supg {
   DevBuf<double> sh_m;  // per shared node: lumped mass
   DevBuf<int> sh_rec;   // per shared node: BC record or -1
   DevBuf<double> lam, regime, pres, scratch;
-  DevBuf<double> ring, eblk, nblk;  // [RING][D_COLS] reduced rows; per-block rows
+  DevBuf<double> row, eblk, nblk;   // [D_ROW] log row, then the running l-CFL maximum; per-block rows
   DevBuf<double> dpart;             // [DIAG_PARTS][D_COLS] partial rows of the reduction
   DevBuf<int> halt;
-  DevBuf<unsigned> fold_count;      // the fix-up's workgroups done (its fold of the log row)
   int cur = 0;
   long loop_time = 0;
   double time = 0.0;
@@ -1059,8 +1052,8 @@ SupgArgs<T> supg_args(femx_supg *s, bool euler_step, double t) {
   a.err = s->bc.err.p;
   a.eblk = s->eblk.p;
   a.halt = s->halt.p;
-  a.prev_row = nullptr;
   a.step_id = (int)s->loop_time;
+  a.want_row = 0;
   a.k = supg_const(s, t, euler_step);
   return a;
 }
@@ -1107,32 +1100,24 @@ double supg_bytes(const femx_supg *s) {
   return E * (3.0 * s->mesh->npe + 32.0) + N * (32.0 + 32.0 + 32.0 + 32.0);
 }
 
-femx_status launch_supg(femx_supg *s, bool dyn, bool press, bool euler_step, double t, long step_id,
-                        const double *prev_row) {
+femx_status launch_supg(femx_supg *s, bool dyn, bool press, bool euler_step, double t, bool want_row) {
   const char *name = dyn ? (press ? "supg_block_press" : "supg_block") : "supg_press";
   TimedLaunch tl(s->timer, s->timer.kind(name, supg_bytes(s)), s->st);
   if (f32_elem(s->p.precision)) {
     SupgArgs<float> a = supg_args<float>(s, euler_step, t);
-    a.prev_row = prev_row;
-    a.step_id = (int)step_id;
+    a.want_row = want_row;
     launch_supg_npe<float>(s, a, dyn, press, s->diag_enabled);
   } else {
     SupgArgs<double> a = supg_args<double>(s, euler_step, t);
-    a.prev_row = prev_row;
-    a.step_id = (int)step_id;
+    a.want_row = want_row;
     launch_supg_npe<double>(s, a, dyn, press, s->diag_enabled);
   }
   FEMX_HIP(hipGetLastError());
   return FEMX_OK;
 }
 
-femx_status launch_fix(femx_supg *s, bool euler_step, double t, double *fold_row = nullptr,
-                       const double *fold_prev = nullptr) {
+SupgFix fix_args(femx_supg *s, bool euler_step, double t) {
   Blocks &b = s->mesh->blk;
-  if (b.n_sh == 0) return FEMX_OK;
-  const bool f32p = f32_sum(s->p.precision);  // float4 partial records
-  const double rec_bytes = f32p ? 16.0 : 32.0;  // one partial slot record, written and read
-  TimedLaunch tl(s->timer, s->timer.kind("supg_fixup", b.sh_off[b.n_sh] * rec_bytes * 2 + b.n_sh * 200.0), s->st);
   SupgFix a;
   a.n_sh = b.n_sh;
   a.sh_node = b.d_sh_node.p;
@@ -1151,23 +1136,47 @@ femx_status launch_fix(femx_supg *s, bool euler_step, double t, double *fold_row
   a.rows = s->bc.rows.p;
   a.err = s->bc.err.p;
   a.halt = s->halt.p;
+  a.step_id = (int)s->loop_time;
+  a.want_row = 0;
   a.nblk = s->nblk.p;
-  a.fold_row = fold_row;
-  a.fold_prev = fold_prev;
-  a.eblk = s->eblk.p;
-  a.ne_blk = b.nb;
-  a.with_elem = s->diag_enabled ? 1 : 0;
-  a.fold_count = s->fold_count.p;
   a.k = supg_const(s, t, euler_step);
+  return a;
+}
+
+femx_status launch_fix(femx_supg *s, bool euler_step, double t, bool want_row) {
+  Blocks &b = s->mesh->blk;
+  if (b.n_sh == 0) return FEMX_OK;
+  const bool f32p = f32_sum(s->p.precision);  // float4 partial records
+  const double rec_bytes = f32p ? 16.0 : 32.0;  // one partial slot record, written and read
+  TimedLaunch tl(s->timer, s->timer.kind("supg_fixup", b.sh_off[b.n_sh] * rec_bytes * 2 + b.n_sh * 200.0), s->st);
+  SupgFix a = fix_args(s, euler_step, t);
+  a.want_row = want_row;
   if (f32p) supg_fixup<float><<<grid_for(b.n_sh, 256), 256, 0, s->st>>>(a);
   else supg_fixup<double><<<grid_for(b.n_sh, 256), 256, 0, s->st>>>(a);
   FEMX_HIP(hipGetLastError());
   return FEMX_OK;
 }
 
+// Workgroups whose rows (nblk) a step's fix-up writes.
+int fix_rows(const femx_supg *s) { return s->mesh->blk.n_sh ? grid_for(s->mesh->blk.n_sh, 256) : 0; }
+
+// The log row of step `step` from ne element-block rows and nn rows of nblk.
+femx_status launch_row(femx_supg *s, int ne, int nn, bool with_elem, int step) {
+  double *row = s->row.p, *lcfl = s->row.p + D_ROW;
+  if (ne + nn <= DIAG_ONE_PASS) {
+    supg_diag_partial<<<1, 256, 0, s->st>>>(s->eblk.p, ne, s->nblk.p, nn, with_elem, row, lcfl, s->halt.p, step);
+  } else {
+    supg_diag_partial<<<DIAG_PARTS, 256, 0, s->st>>>(s->eblk.p, ne, s->nblk.p, nn, with_elem, s->dpart.p, nullptr,
+                                                     s->halt.p, step);
+    supg_diag_final<<<1, 64, 0, s->st>>>(s->dpart.p, DIAG_PARTS, row, lcfl, s->halt.p, step);
+  }
+  FEMX_HIP(hipGetLastError());
+  return FEMX_OK;
+}
+
 femx_status flush_pressure(femx_supg *s) {
   if (!s->press_pending) return FEMX_OK;
-  femx_status r = launch_supg(s, false, true, true, s->time, s->loop_time, nullptr);
+  femx_status r = launch_supg(s, false, true, true, s->time, false);
   if (r != FEMX_OK) return r;
   s->press_pending = false;
   return FEMX_OK;
@@ -1216,14 +1225,11 @@ extern "C" femx_status femx_supg_create(femx_mesh *mh, const femx_bc_desc *bc, c
   if ((r = s->partials.alloc(std::max(nparts, 1))) != FEMX_OK) return fail(r);
   if ((r = s->lam.alloc(m.E)) != FEMX_OK || (r = s->regime.alloc(m.E)) != FEMX_OK || (r = s->pres.alloc(m.E)) != FEMX_OK)
     return fail(r);
-  if ((r = s->ring.alloc((size_t)RING * D_COLS)) != FEMX_OK || (r = s->halt.alloc(1)) != FEMX_OK ||
-      (r = s->fold_count.alloc(1)) != FEMX_OK)
-    return fail(r);
-  if (hipMemsetAsync(s->fold_count.p, 0, sizeof(unsigned), s->st) != hipSuccess) return fail(FEMX_ERR_HIP);
+  if ((r = s->row.alloc(D_ROW + 1)) != FEMX_OK || (r = s->halt.alloc(1)) != FEMX_OK) return fail(r);
   if ((r = s->eblk.alloc((size_t)m.blk.nb * D_COLS)) != FEMX_OK) return fail(r);
   if ((r = s->nblk.alloc((size_t)grid_for(m.N, 256) * D_COLS)) != FEMX_OK) return fail(r);
   if ((r = s->dpart.alloc((size_t)DIAG_PARTS * D_COLS)) != FEMX_OK) return fail(r);
-  if (hipMemsetAsync(s->ring.p, 0, (size_t)RING * D_COLS * sizeof(double), s->st) != hipSuccess) return fail(FEMX_ERR_HIP);
+  if (hipMemsetAsync(s->row.p, 0, (D_ROW + 1) * sizeof(double), s->st) != hipSuccess) return fail(FEMX_ERR_HIP);
   if (m.npe == 8)
     supg_mass<8><<<grid_for(m.N, 256), 256, 0, s->st>>>(m.N, m.g_off.p, m.g_slot.p, m.conn.p, m.xyz.p, p->rho, s->xyzm.p);
   else
@@ -1276,6 +1282,7 @@ extern "C" femx_status femx_supg_set_state(femx_supg *s, const double *sol) {
   FEMX_HIP(hipMemsetAsync(s->lam.p, 0, m.E * sizeof(double), s->st));  // el_lam = 0 at the initial pressure (:896)
   FEMX_HIP(hipMemsetAsync(s->regime.p, 0, m.E * sizeof(double), s->st));
   FEMX_HIP(hipMemsetAsync(s->Fprev.p, 0, m.N * sizeof(double4), s->st));
+  FEMX_HIP(hipMemsetAsync(s->row.p, 0, (D_ROW + 1) * sizeof(double), s->st));
   s->press_pending = true;
   femx_status r = check_bc_err(s);
   FEMX_HIP(hipStreamSynchronize(s->st));
@@ -1295,30 +1302,16 @@ femx_status supg_enqueue(femx_supg *s, int nsteps) {
     s->loop_time++;
     s->time += s->p.dt;  // currentTime += timeStep (:1041)
     const bool euler_step = s->p.use_euler || s->loop_time == 1;
-    double *row = s->ring.p + (s->loop_time % RING) * D_COLS;
-    const double *prev = s->loop_time > 1 ? s->ring.p + ((s->loop_time - 1) % RING) * D_COLS : nullptr;
-    femx_status r = launch_supg(s, true, s->press_pending, euler_step, s->time, s->loop_time, prev);
+    // the log row: per step with the element diagnostics on, else the one of
+    // the call's last step
+    const bool row = s->diag_enabled || k == nsteps - 1;
+    femx_status r = launch_supg(s, true, s->press_pending, euler_step, s->time, row);
     if (r != FEMX_OK) return r;
-    // node extrema rows: one per fix-up workgroup (nblk) and one per element
-    // block (node columns of eblk), written where the new states are formed;
-    // with few rows, the fix-up's last workgroup folds them into the log row
-    const int nnb = s->mesh->blk.n_sh ? grid_for(s->mesh->blk.n_sh, 256) : 0;
-    const bool fold = nnb > 0 && nnb + s->mesh->blk.nb <= DIAG_ONE_PASS;
-    if ((r = launch_fix(s, euler_step, s->time, fold ? row : nullptr, fold ? prev : nullptr)) != FEMX_OK) return r;
+    if ((r = launch_fix(s, euler_step, s->time, row)) != FEMX_OK) return r;
     s->cur ^= 1;
     s->press_pending = true;
-    if (fold) {
-      // folded by the fix-up
-    } else if (nnb + s->mesh->blk.nb <= DIAG_ONE_PASS) {
-      // few rows and no fix-up: one workgroup folds them into the log row
-      supg_diag_partial<<<1, 256, 0, s->st>>>(s->eblk.p, s->mesh->blk.nb, s->nblk.p, nnb, s->diag_enabled ? 1 : 0,
-                                              row, s->halt.p, prev);
-    } else {
-      supg_diag_partial<<<DIAG_PARTS, 256, 0, s->st>>>(s->eblk.p, s->mesh->blk.nb, s->nblk.p, nnb,
-                                                       s->diag_enabled ? 1 : 0, s->dpart.p, s->halt.p, nullptr);
-      supg_diag_final<<<1, 64, 0, s->st>>>(s->dpart.p, DIAG_PARTS, row, s->halt.p, prev);
-    }
-    FEMX_HIP(hipGetLastError());
+    if (row && (r = launch_row(s, s->mesh->blk.nb, fix_rows(s), s->diag_enabled, (int)s->loop_time)) != FEMX_OK)
+      return r;
     s->pend_n++;
   }
   return FEMX_OK;
@@ -1334,20 +1327,11 @@ femx_status supg_finish(femx_supg *s, int *steps_done) {
   s->pend_n = 0;
   if (steps_done) *steps_done = 0;
   int halt = INT_MAX;
-  double last[D_COLS];
   FEMX_HIP(hipMemcpyAsync(&halt, s->halt.p, sizeof(int), hipMemcpyDeviceToHost, s->st));
-  FEMX_HIP(hipMemcpyAsync(last, s->ring.p + (s->loop_time % RING) * D_COLS, sizeof(last), hipMemcpyDeviceToHost,
-                          s->st));
-  FEMX_HIP(hipStreamSynchronize(s->st));
   femx_status r = check_bc_err(s);
   if (r != FEMX_OK) return r;
-  long stop = -1;
   if (halt != INT_MAX) {
-    stop = halt;
-  } else if (nsteps > 0 && last[D_UMOD] > s->p.exit_condition * s->p.exit_condition) {
-    stop = s->loop_time;
-  }
-  if (stop >= 0) {
+    const long stop = halt;
     // rewind the host counters to the step that exceeded the threshold
     const long done = stop - first;
     s->loop_time = stop;
@@ -1356,6 +1340,16 @@ femx_status supg_finish(femx_supg *s, int *steps_done) {
     s->cur = (int)((cur0 + done) & 1);
     if (steps_done) *steps_done = (int)done;
     s->halted = true;
+    // a step inside a call has no log row of its own: make it from the state
+    double step = 0.0;
+    FEMX_HIP(hipMemcpyAsync(&step, s->row.p + D_STEP, sizeof(double), hipMemcpyDeviceToHost, s->st));
+    FEMX_HIP(hipStreamSynchronize(s->st));
+    if (step != (double)stop) {
+      const int nwg = grid_for(s->mesh->N, 256);
+      supg_state_rows<<<nwg, 256, 0, s->st>>>(s->mesh->N, s->U[s->cur].p, s->nblk.p);
+      FEMX_HIP(hipGetLastError());
+      if ((r = launch_row(s, 0, nwg, false, (int)stop)) != FEMX_OK) return r;
+    }
     set_error("ERROR: Maximum velocity module larger than admissible threshold.");
     return FEMX_EXIT_CONDITION;
   }
@@ -1444,7 +1438,7 @@ extern "C" femx_status femx_supg_get_log(femx_supg *s, double *cols19) {
     if (f != FEMX_OK && f != FEMX_EXIT_CONDITION) return f;
   }
   double k[D_COLS];
-  FEMX_HIP(hipMemcpyAsync(k, s->ring.p + (s->loop_time % RING) * D_COLS, sizeof(k), hipMemcpyDeviceToHost, s->st));
+  FEMX_HIP(hipMemcpyAsync(k, s->row.p, sizeof(k), hipMemcpyDeviceToHost, s->st));
   FEMX_HIP(hipStreamSynchronize(s->st));
   cols19[0] = (double)s->loop_time;
   cols19[1] = s->time;
@@ -1502,10 +1496,10 @@ struct SupgDyn {
 };
 
 struct SupgMember {
-  SupgArgs<float> a;  // per step: U, Upress, Un, k.t, step_id, prev_row
-  SupgFix f;          // per step: U, Un, k.t (the tick folds the log row)
+  SupgArgs<float> a;  // per step: U, Upress, Un, k.t, step_id, want_row
+  SupgFix f;          // per step: U, Un, k.t, step_id, want_row
   double4 *Ub[2];
-  double *ring;
+  double *row;
   SupgDyn *dyn;
   double dt;
   int nwg;  // fix-up workgroups
@@ -1518,14 +1512,12 @@ __device__ __forceinline__ void args_to_global(SupgArgs<float> &a) {
   to_global(a.Upress), to_global(a.Un), to_global(a.Unp), to_global(a.Fprev), to_global(a.partials);
   to_global(a.lam), to_global(a.regime), to_global(a.pres), to_global(a.node_rec), to_global(a.rec);
   to_global(a.row_off), to_global(a.rows), to_global(a.err), to_global(a.eblk), to_global(a.halt);
-  to_global(a.prev_row);
 }
 __device__ __forceinline__ void args_to_global(SupgFix &a) {
   to_global(a.sh_node), to_global(a.sh_off), to_global(a.sh_slot), to_global(a.sh_first4);
   to_global(a.partials), to_global(a.sh_m), to_global(a.sh_rec), to_global(a.U), to_global(a.Un);
   to_global(a.Unp), to_global(a.Fprev), to_global(a.rec), to_global(a.row_off), to_global(a.rows);
-  to_global(a.err), to_global(a.halt), to_global(a.nblk), to_global(a.fold_row), to_global(a.fold_prev);
-  to_global(a.eblk), to_global(a.fold_count);
+  to_global(a.err), to_global(a.halt), to_global(a.nblk);
 }
 
 __device__ __forceinline__ int supg_member_of(const int *off, int nm, int g) {
@@ -1539,13 +1531,14 @@ __device__ __forceinline__ int supg_member_of(const int *off, int nm, int g) {
 }
 
 __global__ __launch_bounds__(threads_for<8>(), 2) void supg_block_union(const SupgMember *mem, const int *blk_off,
-                                                                        int nm, int ntot) {
+                                                                        int nm, int ntot, int last) {
   const int g = xcd_block(blockIdx.x, ntot);
   const int h = supg_member_of(blk_off, nm, g);
   const SupgMember &me = mem[h];
   SupgDyn *dyn = me.dyn;
   to_global(dyn);
-  if (uni(dyn->left) <= 0) return;
+  const int left = uni(dyn->left);
+  if (left <= 0) return;
   const int par = uni(dyn->par), lt = uni(dyn->lt) + 1;
   SupgArgs<float> a = me.a;
   a.U = me.Ub[par];
@@ -1553,44 +1546,48 @@ __global__ __launch_bounds__(threads_for<8>(), 2) void supg_block_union(const Su
   a.Un = me.Ub[par ^ 1];
   a.k.t = uni(dyn->t) + me.dt;  // currentTime += timeStep (:1041)
   a.step_id = lt;
-  a.prev_row = lt > 1 ? me.ring + (long)((lt - 1) % RING) * D_COLS : nullptr;
+  a.want_row = last || left == 1;
   args_to_global(a);
   const int blk = g - uni(blk_off[h]);
   supg_block_run<float, 8, true, true, true, false, false>(a, blk, blk);
 }
 
-__global__ __launch_bounds__(256) void supg_fixup_union(const SupgMember *mem, const int *fx_off, int nm) {
+__global__ __launch_bounds__(256) void supg_fixup_union(const SupgMember *mem, const int *fx_off, int nm, int last) {
   const int g = blockIdx.x;
   const int h = supg_member_of(fx_off, nm, g);
   const SupgMember &me = mem[h];
   SupgDyn *dyn = me.dyn;
   to_global(dyn);
-  if (uni(dyn->left) <= 0) return;
+  const int left = uni(dyn->left);
+  if (left <= 0) return;
   const int par = uni(dyn->par);
   SupgFix f = me.f;
+  f.step_id = uni(dyn->lt) + 1;
+  f.want_row = last || left == 1;
   f.U = me.Ub[par];
   f.Un = me.Ub[par ^ 1];
   f.k.t = uni(dyn->t) + me.dt;
   args_to_global(f);
-  supg_fixup_run<double>(f, g - uni(fx_off[h]), me.nwg);
+  supg_fixup_run<double>(f, g - uni(fx_off[h]));
 }
 
-// End of a union step, one workgroup per member with steps left: the step's
-// rows (element blocks and fix-up, both written by the previous kernels)
-// folded into its log row, then the member moves on by one step.
-__global__ __launch_bounds__(256) void supg_union_tick(const SupgMember *mem) {
+// End of a union step, one workgroup per member with steps left: the log row
+// of the member's last step, or of the call's last step (last), from the
+// step's rows (element blocks and fix-up, both written by the previous
+// kernels), then the member moves on by one step.
+__global__ __launch_bounds__(256) void supg_union_tick(const SupgMember *mem, int last) {
   const SupgMember &me = mem[blockIdx.x];
   SupgDyn *d = me.dyn;
   to_global(d);
-  if (uni(d->left) <= 0) return;
+  const int left = uni(d->left);
+  if (left <= 0) return;
   const int lt = uni(d->lt) + 1;
   const int *halt = me.a.halt;
-  const double *eblk = me.f.eblk, *nblk = me.f.nblk;
-  double *ring = me.ring;
-  to_global(halt), to_global(eblk), to_global(nblk), to_global(ring);
-  if (!halted(halt))
-    diag_fold<false>(eblk, me.f.ne_blk, nblk, me.nwg, 0, ring + (long)(lt % RING) * D_COLS,
-                     lt > 1 ? ring + (long)((lt - 1) % RING) * D_COLS : nullptr, 0, 1);
+  const double *eblk = me.a.eblk, *nblk = me.f.nblk;
+  double *row = me.row;
+  to_global(halt), to_global(eblk), to_global(nblk), to_global(row);
+  if ((last || left == 1) && !halted(halt, lt))
+    diag_fold(eblk, me.a.nblk, nblk, me.nwg, 0, row, row + D_ROW, lt, 0, 1);
   __syncthreads();
   if (threadIdx.x == 0) {
     d->t = d->t + me.dt;
@@ -1646,36 +1643,11 @@ femx_status supg_union_upload(femx_supg_union *u) {
     const bool euler = h->p.use_euler != 0;  // the first step ran on the handle's own stream
     e.a = supg_args<float>(h, euler, 0.0);
     e.a.Unp = nullptr;
-    // the fix-up's arguments, as launch_fix builds them
     const Blocks &b = h->mesh->blk;
-    SupgFix &f = e.f;
-    f.n_sh = b.n_sh;
-    f.sh_node = b.d_sh_node.p;
-    f.sh_off = b.d_sh_off.p;
-    f.sh_slot = b.d_sh_slot.p;
-    f.sh_first4 = b.d_sh_first4.p;
-    f.partials = h->partials.p;
-    f.sh_m = h->sh_m.p;
-    f.sh_rec = h->sh_rec.p;
-    f.U = nullptr;
-    f.Un = nullptr;
-    f.Unp = nullptr;
-    f.Fprev = h->Fprev.p;
-    f.rec = h->bc.rec.p;
-    f.row_off = h->bc.row_off.p;
-    f.rows = h->bc.rows.p;
-    f.err = h->bc.err.p;
-    f.halt = h->halt.p;
-    f.nblk = h->nblk.p;
-    f.fold_row = nullptr;
-    f.fold_prev = nullptr;
-    f.eblk = h->eblk.p;
-    f.ne_blk = b.nb;
-    f.with_elem = 0;
-    f.fold_count = h->fold_count.p;
-    f.k = supg_const(h, 0.0, euler);
+    e.f = fix_args(h, euler, 0.0);
+    e.f.Unp = nullptr;
     for (int k = 0; k < 2; k++) e.Ub[k] = h->U[k].p;
-    e.ring = h->ring.p;
+    e.row = h->row.p;
     e.dyn = reinterpret_cast<SupgDyn *>(h->dyn.p);
     e.dt = h->p.dt;
     e.nwg = grid_for(b.n_sh, 256);
@@ -1783,9 +1755,10 @@ extern "C" femx_status femx_supg_union_step(femx_supg_union *u, int k) {
   if (nm == 0 || k == 0) return FEMX_OK;
   const int *blk_off = u->off.p, *fx_off = u->off.p + nm + 1;
   for (int i = 0; i < k; i++) {
-    supg_block_union<<<u->nblk, threads_for<8>(), 0, u->st>>>(u->tab.p, blk_off, nm, u->nblk);
-    supg_fixup_union<<<u->nfx, 256, 0, u->st>>>(u->tab.p, fx_off, nm);
-    supg_union_tick<<<nm, 256, 0, u->st>>>(u->tab.p);
+    const int last = i == k - 1;
+    supg_block_union<<<u->nblk, threads_for<8>(), 0, u->st>>>(u->tab.p, blk_off, nm, u->nblk, last);
+    supg_fixup_union<<<u->nfx, 256, 0, u->st>>>(u->tab.p, fx_off, nm, last);
+    supg_union_tick<<<nm, 256, 0, u->st>>>(u->tab.p, last);
   }
   FEMX_HIP(hipGetLastError());
   // the host's view of every member: the steps enqueued as on its own stream

@@ -205,6 +205,33 @@ def test_exit_condition(gpu):
     assert g.step(1) == 0
 
 
+@pytest.mark.parametrize("n,precision", [(5, 0), (9, 0), (9, 1)])
+def test_exit_inside_a_call(gpu, n, precision):
+    """The exit condition firing in the middle of one step(n) call stops the
+    solve where single-step calls do, with the same state, pressure, bulk
+    modulus and log row (the step had no log row of its own)."""
+    m, bc, params, ic = _case("hexa", n, 0.1, seed=8)
+    rows = bc.vel_rows.reshape(-1, 2, 4).copy()
+    rows[:, 1] = [300.0, 0.0, 0.0, 100.0]  # the lid speeds up linearly from 0, 3 t
+    rows[:, 0] = 0.0
+    bc.vel_rows = rows.reshape(-1, 4)
+    dm = gpu.DeviceMesh(m)
+    a, b = (gpu.SUPGSolver(dm, bc, exit_condition=0.4, precision=precision, **params) for _ in range(2))
+    a.set_state(ic)
+    b.set_state(ic)
+    done = 0
+    while a.step(1) == 1 and not a.get_log()[3] > 0.4:
+        done += 1
+    print("exit after step", done + 1, flush=True)
+    assert 2 <= done < 60
+    assert b.step(80) == done + 1
+    assert b.step(1) == 0
+    sa, sb = a.get_state(), b.get_state()
+    for k in ("sol", "pres", "lam", "regime", "time"):
+        assert np.array_equal(sa[k], sb[k]), k
+    assert np.array_equal(a.get_log(), b.get_log())
+
+
 def test_deterministic(gpu):
     m, bc, params, ic = _case("hexa", 6, 0.2, seed=9)
     dm = gpu.DeviceMesh(m)
