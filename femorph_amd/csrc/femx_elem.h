@@ -74,6 +74,9 @@ __device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x
 __device__ __forceinline__ double sqrt_e(double x) { return sqrt(x); }
 __device__ __forceinline__ float sqrt_e(float x) { return __builtin_amdgcn_sqrtf(x); }
 
+__device__ __forceinline__ double rsqrt_e(double x) { return 1.0 / sqrt(x); }
+__device__ __forceinline__ float rsqrt_e(float x) { return __builtin_amdgcn_rsqf(x); }
+
 // femUtils::invert3x3Matrix (src/femUtils.cpp:716-770), in T.
 template <typename T>
 __device__ __forceinline__ void inv3(const T m[3][3], T iv[3][3], T &det) {

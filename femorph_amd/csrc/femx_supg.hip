@@ -33,10 +33,12 @@
 namespace femx {
 namespace {
 
-// threads per workgroup = max elements per block of the mesh partition
-// (femx_mesh_upload cuts tet4 meshes into <= 256-element blocks, hexa8 into <= 128)
+// max elements per block of the mesh partition (femx_mesh_upload cuts tet4
+// meshes into <= 256-element blocks, hexa8 into <= 128); one thread per tet4,
+// two per hexa8
 template <int NPE>
-constexpr int threads_for() { return NPE == 4 ? 256 : 128; }
+constexpr int elems_for() { return NPE == 4 ? 256 : 128; }
+constexpr int SB = 256;
 
 // diagnostic row layout: 0..5 min/max u v w, 6,7 min/max tau, 8,9 min/max
 // lambda, 10 v-CFL max, 11 a-CFL max, 12 l-CFL max, 13,14 min/max E,
@@ -154,28 +156,6 @@ struct SupgArgs {
   SupgConst k;
 };
 
-template <int NPE>
-__device__ __forceinline__ void lconn_load(const uint8_t *lconn, int e, int id[NPE]) {
-  if (NPE == 4) {
-    const uchar4 c = reinterpret_cast<const uchar4 *>(lconn)[e];
-    id[0] = c.x; id[1] = c.y; id[2] = c.z; id[3] = c.w;
-  } else {
-    const uchar4 c0 = reinterpret_cast<const uchar4 *>(lconn)[2 * e], c1 = reinterpret_cast<const uchar4 *>(lconn)[2 * e + 1];
-    id[0] = c0.x; id[1] = c0.y; id[2] = c0.z; id[3] = c0.w;
-    id[4 % NPE] = c1.x; id[5 % NPE] = c1.y; id[6 % NPE] = c1.z; id[7 % NPE] = c1.w;
-  }
-}
-template <int NPE>
-__device__ __forceinline__ void lpos_load(const uint16_t *lpos, int e, int ps[NPE]) {
-  const ushort4 *p = reinterpret_cast<const ushort4 *>(lpos);
-  const ushort4 a = p[(NPE / 4) * e];
-  ps[0] = a.x; ps[1] = a.y; ps[2] = a.z; ps[3] = a.w;
-  if (NPE == 8) {
-    const ushort4 b = p[2 * e + 1];
-    ps[4 % NPE] = b.x; ps[5 % NPE] = b.y; ps[6 % NPE] = b.z; ps[7 % NPE] = b.w;
-  }
-}
-
 // The exit condition (:1635-1643): the workgroups that form the new states of
 // step `step` and see |u|^2 above the threshold put the step into *halt; the
 // rest of that step still runs, every later step's work is skipped.  It
@@ -211,45 +191,397 @@ __device__ __forceinline__ void supg_node(const double F[3], double4 fprev, doub
   fstore = make_double4(F[0], F[1], F[2], 0.0);
 }
 
-// Two waves per SIMD: the hexa8 variants then spill ~140-240 B per lane to
-// scratch, which costs less than running one wave per SIMD (0.58 vs 0.77 ms
-// per launch on the 2.1M-hexa cavity).
+// hexa8 element math.  It is bound by VALU issue (four cycles per wave
+// instruction in FP32 and FP64 alike), so it is arranged for few instructions
+// and no spills:
+//  - the map and the velocity are trilinear, so the sums over nodes at the
+//    Gauss points share most of their terms (Tri), and so do the node sums of
+//    the forces (TriSum); the averages of B-hat need no pass over the Gauss
+//    points (TriAvg);
+//  - two neighbouring lanes work on one element, each on the four Gauss points
+//    of one z = +-1/sqrt 3, and hold the element's fields and sums for that z
+//    only.  With one lane per element the same math needed 256 VGPRs, two
+//    waves per SIMD (316 us).
+// Per hexa8 element-step 2 x 2,000 wave-lane instructions against 6,650 node
+// by node; the block kernel at 2.1M hexa 356 -> 277 us mixed, at 85k hexa 47 ->
+// 31 us FP64.
+// The other lane's value: a DPP quad permute (1, 0, 3, 2).
+__device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
+__device__ __forceinline__ float pair_swap(float v) { return __int_as_float(pair_swap(__float_as_int(v))); }
+__device__ __forceinline__ double pair_swap(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)pair_swap((int)(unsigned)(b & 0xffffffffLL));
+  const unsigned hi = (unsigned)pair_swap((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <typename T>
+__device__ __forceinline__ T pair_sum(T v) { return v + pair_swap(v); }
+
+// A trilinear 3-vector field f = c1 + x cx + y cy + z cz + xy cxy + xz cxz + yz
+// cyz + xyz cxyz (femHexa8 node signs, src/femHexa8.cpp:15-17) on the lane's
+// plane of Gauss points.  z points towards the lane's own side, so both
+// lanes work at z = 1/sqrt 3; the element's map is then left-handed for one of
+// them.
+//   f     = (c00 + y A2) + x df/dx           c00 = c1 + z cz
+//   df/dx = A1 + y B                         A1 = cx + z cxz, B = cxy + z cxyz
+//   df/dy = A2 + x B                         A2 = cy + z cyz
+//   df/dz = (cz + y cyz) + x (cxz + y cxyz)
+// so most of the sums are shared between Gauss points.  Node values come in
+// as 1/8 of the field, the transforms' factor.
+template <typename T>
+struct Tri {
+  T c00[3], A1[3], A2[3], B[3], Cz[3], Cxz[3], Cyz[3], Cxyz[3];
+  T Dx[3], D[3], F[3];  // per y: df/dx, cz + y cyz, cxz + y cxyz
+  // component b from the values at the four nodes of the lane's side; the
+  // other lane holds the other side's
+  __device__ __forceinline__ void load(int b, const T own[4], T q) {
+    T g[4], d[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const T oth = pair_swap(own[k]);
+      d[k] = own[k] - oth;
+      g[k] = (own[k] + oth) + q * d[k];
+    }
+    xy(g, c00[b], A1[b], A2[b], B[b]);
+    xy(d, Cz[b], Cxz[b], Cyz[b], Cxyz[b]);
+  }
+  template <typename S>
+  __device__ __forceinline__ void from(const Tri<S> &f) {
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      c00[b] = (T)f.c00[b], A1[b] = (T)f.A1[b], A2[b] = (T)f.A2[b], B[b] = (T)f.B[b];
+      Cz[b] = (T)f.Cz[b], Cxz[b] = (T)f.Cxz[b], Cyz[b] = (T)f.Cyz[b], Cxyz[b] = (T)f.Cxyz[b];
+    }
+  }
+  static __device__ __forceinline__ void xy(const T g[4], T &s, T &x, T &y, T &c) {
+    const T p = g[0] + g[1], q = g[2] + g[3], r = g[1] - g[0], t = g[2] - g[3];
+    s = p + q;
+    y = q - p;
+    x = r + t;
+    c = t - r;
+  }
+  __device__ __forceinline__ void at_y(T y) {
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      Dx[b] = A1[b] + y * B[b];
+      D[b] = Cz[b] + y * Cyz[b];
+      F[b] = Cxz[b] + y * Cxyz[b];
+    }
+  }
+  __device__ __forceinline__ void at_x(T x, T L[3][3]) const {
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      L[0][b] = Dx[b];
+      L[1][b] = A2[b] + x * B[b];
+      L[2][b] = D[b] + x * F[b];
+    }
+  }
+};
+
+// The transpose: sums over the lane's Gauss points of v N + T0 dN/dx + T1
+// dN/dy + T2 dN/dz in the same coefficients of the trilinear test functions.
+template <typename T>
+struct TriSum {
+  T c00[3], A1[3], A2[3], B[3], Cz[3], Cxz[3], Cyz[3], Cxyz[3];
+  __device__ __forceinline__ void init() {
+#pragma unroll
+    for (int b = 0; b < 3; b++) c00[b] = A1[b] = A2[b] = B[b] = Cz[b] = Cxz[b] = Cyz[b] = Cxyz[b] = (T)0;
+  }
+  // Tl[i][l]: component i, local direction l
+  __device__ __forceinline__ void add(T x, T y, const T v[3], const T Tl[3][3]) {
+    const T xy = x * y;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const T t0 = Tl[i][0] + x * v[i];
+      c00[i] += v[i];
+      A1[i] += t0;
+      B[i] += y * t0;
+      A2[i] += Tl[i][1] + y * v[i];
+      B[i] += x * Tl[i][1];
+      Cz[i] += Tl[i][2];
+      Cxz[i] += x * Tl[i][2];
+      Cyz[i] += y * Tl[i][2];
+      Cxyz[i] += xy * Tl[i][2];
+    }
+  }
+  // The element's sums on the nodes of the lane's side, as the four (x, y)
+  // coefficients 1, x, y, xy of component b: with the test functions' z
+  // factors 1 + z, own p + (q p + c) and the other lane's p - (q p + c) for
+  // each pair p = c00, A1, A2, B and c = Cz, Cxz, Cyz, Cxyz.
+  static __device__ __forceinline__ T fold(T p, T c, T q) {
+    const T w = q * p + c;
+    return (p + w) + pair_swap(p - w);
+  }
+  __device__ __forceinline__ void nodes(int b, T q, T e[4]) const {
+    e[0] = fold(c00[b], Cz[b], q);
+    e[1] = fold(A1[b], Cxz[b], q);
+    e[2] = fold(A2[b], Cyz[b], q);
+    e[3] = fold(B[b], Cxyz[b], q);
+  }
+};
+// eval_avg_shapeDeriv (:660-707): the sums over the eight Gauss points of DN
+// dv, that is of the Jacobian's cofactors times the local derivatives.  In the
+// monomials of the trilinear map the two-point rule leaves (its points are
+// +-1/sqrt 3: odd powers vanish, a square gives 1/3)
+//   x: E2 x E3 + Exy x Exz / 3     xy: (E2 x Eyz + Exz x E1) / 3
+//   y: E3 x E1 + Eyz x Exy / 3     xz: (Eyz x E3 + E1 x Exy) / 3
+//   z: E1 x E2 + Exz x Eyz / 3     yz: (E3 x Exz + Exy x E2) / 3
+// (times 8) and nothing for 1 and xyz: 72 multiply-adds instead of a pass
+// over the Gauss points (about 400 instructions per lane).  Both lanes of an
+// element form them in their own local coordinates; the sign of the map's
+// handedness cancels in the average.  In FP64 on every path: the mean
+// divergence (the pressure) is a small sum of large terms, and FP64 issues as
+// fast as FP32 here.
+struct TriAvg {
+  using T = double;
+  T x[3], y[3], z[3], xy[3], xz[3], yz[3];
+  T vol;  // of the element
+  // r = a x b + f c x d
+  static __device__ __forceinline__ void cross2(const T a[3], const T b[3], T f, const T c[3], const T d[3], T r[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int j = (i + 1) % 3, k = (i + 2) % 3;
+      r[i] = (a[j] * b[k] - a[k] * b[j]) + f * (c[j] * d[k] - c[k] * d[j]);
+    }
+  }
+  // the monomials' coefficients 1, 2 and xy of a field (the field holds them at its z)
+  static __device__ __forceinline__ void base(const Tri<T> &f, T q, T f1[3], T f2[3], T fxy[3]) {
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      f1[b] = f.A1[b] - q * f.Cxz[b];
+      f2[b] = f.A2[b] - q * f.Cyz[b];
+      fxy[b] = f.B[b] - q * f.Cxyz[b];
+    }
+  }
+  __device__ __forceinline__ void form(const Tri<T> &X, T q, T sg) {
+    const T third = (T)(1.0 / 3.0);
+    T E1[3], E2[3], Exy[3];
+    base(X, q, E1, E2, Exy);
+    cross2(E2, X.Cz, third, Exy, X.Cxz, x);
+    cross2(X.Cz, E1, third, X.Cyz, Exy, y);
+    cross2(E1, E2, third, X.Cxz, X.Cyz, z);
+    cross2(E2, X.Cyz, (T)1, X.Cxz, E1, xy);
+    cross2(X.Cyz, X.Cz, (T)1, E1, Exy, xz);
+    cross2(X.Cz, X.Cxz, (T)1, Exy, E2, yz);
+    // the volume from the field x itself: sum_n DN_n x_n = 1
+    const T den = (x[0] * E1[0] + y[0] * E2[0] + z[0] * X.Cz[0]) +
+                  third * (xy[0] * Exy[0] + xz[0] * X.Cxz[0] + yz[0] * X.Cyz[0]);
+    vol = 8.0 * sg * den;
+    const T id = recip(den), id3 = id * third;
+#pragma unroll
+    for (int b = 0; b < 3; b++) x[b] *= id, y[b] *= id, z[b] *= id, xy[b] *= id3, xz[b] *= id3, yz[b] *= id3;
+  }
+  // P_b = sum_n avg_nb u_nb
+  __device__ __forceinline__ void dot(const Tri<T> &V, T q, T P[3]) const {
+    T u1[3], u2[3], uxy[3];
+    base(V, q, u1, u2, uxy);
+#pragma unroll
+    for (int b = 0; b < 3; b++)
+      P[b] = (x[b] * u1[b] + y[b] * u2[b] + z[b] * V.Cz[b]) + (xy[b] * uxy[b] + xz[b] * V.Cxz[b] + yz[b] * V.Cyz[b]);
+  }
+};
+
+// What eval_stabilization, eval_bulk_modulus and the diagnostics need of the
+// metric G = invJ^T invJ (src/femElement.cpp:222-231): |G|^2 and its trace.
+template <typename T>
+__device__ __forceinline__ void metric3(const T iJ[3][3], T &gg, T &tr) {
+  T d[3], o[3];
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    const int k = (i + 1) % 3;
+    d[i] = iJ[0][i] * iJ[0][i] + iJ[1][i] * iJ[1][i] + iJ[2][i] * iJ[2][i];
+    o[i] = iJ[0][i] * iJ[0][k] + iJ[1][i] * iJ[1][k] + iJ[2][i] * iJ[2][k];
+  }
+  tr = d[0] + d[1] + d[2];
+  gg = (d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) + (T)2 * (o[0] * o[0] + o[1] * o[1] + o[2] * o[2]);
+}
+// |J^T u|^2 = u^T G^-1 u and |invJ u|^2 = u^T G u (G^-1 = J J^T; the indices of
+// G are local directions, those of u physical ones, as in the reference)
+template <typename T>
+__device__ __forceinline__ T norm2_tmul(const T m[3][3], const T u[3]) {
+  T r = (T)0;
+#pragma unroll
+  for (int b = 0; b < 3; b++) {
+    const T x = m[0][b] * u[0] + m[1][b] * u[1] + m[2][b] * u[2];
+    r += x * x;
+  }
+  return r;
+}
+template <typename T>
+__device__ __forceinline__ T norm2_mul(const T m[3][3], const T u[3]) {
+  T r = (T)0;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const T x = m[a][0] * u[0] + m[a][1] * u[1] + m[a][2] * u[2];
+    r += x * x;
+  }
+  return r;
+}
+
+// The element math's constants in T.  An FP64 argument rounded to FP32 is a
+// vector conversion: its result goes back to an SGPR, so that the constants
+// take no VGPRs through the Gauss-point loop.
+__device__ __forceinline__ float uni(float v) { return __int_as_float(femx::uni(__float_as_int(v))); }
+template <typename T>
+struct ElemConst {
+  T mu, mu2, mu23, mu43, mu103, rho, alpha, cnu2, nu, f1;  // mu and its multiples by 2, 2/3, -4/3, 10/3
+  int k2, k3, k4;
+  __device__ __forceinline__ ElemConst(const SupgConst &k) {
+    mu = c(k.mu);
+    mu2 = c(2.0 * k.mu);
+    mu23 = c(k.mu * (2.0 / 3.0));
+    mu43 = c(k.mu * (-4.0 / 3.0));
+    mu103 = c(k.mu * (10.0 / 3.0));
+    rho = c(k.rho);
+    alpha = c(k.alpha);
+    nu = c((T)k.mu / (T)k.rho);
+    cnu2 = c(k.cI * (k.mu / k.rho) * (k.mu / k.rho));
+    f1 = k.k1 ? rho : (T)0;
+    k2 = k.k2;
+    k3 = k.k3;
+    k4 = k.k4;
+  }
+  static __device__ __forceinline__ T c(double v) {
+    if constexpr (sizeof(T) == 4) return uni((float)v);
+    else return v;
+  }
+};
+
+// Per-thread sums over the Gauss points and the diagnostic columns D_TAU ...
+template <typename T>
+struct ElemAcc {
+  T lam_int, reg;
+  T S0, S[3];  // B-hat: the average's factor is sum of f2 alpha_k = S0 - 4/3 mu S_k
+};
+
+// B-hat: the element's part of the strain, eps_k = 5/3 D_k - div / 3 + q_k and
+// tr eps = 2/3 div + r, with D_k = du_k/dx_k, from the averages P.
+template <typename T, bool BHAT>
+struct StrainConst {
+  T q[3], r;
+  __device__ __forceinline__ explicit StrainConst(const T P[3]) {
+    r = BHAT ? (P[0] + P[1] + P[2]) * (T)(1.0 / 3.0) : (T)0;
+#pragma unroll
+    for (int b = 0; b < 3; b++) q[b] = BHAT ? r - (T)(2.0 / 3.0) * P[b] : (T)0;
+  }
+};
+
+// One Gauss point (:1095-1507): from the velocity ug, its gradient gU[b][i] =
+// du_i/dx_b, |J^T u|^2 (l2sq), |invJ u|^2 (t2), |G|^2 (gg), tr G and dv, the
+// stabilization and the bulk modulus (lam, f3), c = (u.grad) u, and the
+// matrix A of the node forces A DN_n (f2 S + f4 I: stress and grad-div).
+template <typename T, bool BHAT, bool DIAG>
+__device__ __forceinline__ void gauss_point(const ElemConst<T> &k, double dt, const T ug[3], const T gU[3][3], T div,
+                                            T dv, T l2sq, T t2, T gg, T trG, const StrainConst<T, BHAT> &sc,
+                                            ElemAcc<T> &s, double *dg, T &f3, T c[3], T A[3][3]) {
+  // eval_stabilization (:336-377), tau without the (2/dt)^2 term
+  const T tau = rsqrt_e(t2 + gg * k.cnu2);
+  const T nuC = recip(trG * tau);
+  // eval_bulk_modulus (:382-441): lambda = alpha max(mu/rho, sqrt(u^T G^-1 u))
+  const T l2 = sqrt_e(l2sq);
+  const T lam = k.alpha * ((k.nu < l2) ? l2 : k.nu);
+  s.reg += (k.nu > l2) ? (T)1 : (T)2;
+  s.lam_int += lam * dv;
+  if (DIAG) {
+    // get_el_lengths_from_G (:756-790) and the CFL / tau / lambda extrema
+    // (:1187-1240), in FP64: 2 sqrt(o^T G^-1 o), o = u / |u|
+    const double u0 = ug[0], u1 = ug[1], u2 = ug[2];
+    const double un = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
+    const double el = 2.0 * (sqrt((double)l2sq) / un);
+    const double nk = k.nu, lm = lam, ta = tau;
+    dg[D_ACFL - D_TAU] = fmax(dg[D_ACFL - D_TAU], fabs(u0 * dt) / el);
+    dg[D_VCFL - D_TAU] = fmax(dg[D_VCFL - D_TAU], 2.0 * nk * (dt / (el * el)));
+    dg[D_LCFL - D_TAU] = fmax(dg[D_LCFL - D_TAU], 2.0 * lm * (dt / (el * el)));
+    dg[0] = fmin(dg[0], ta);
+    dg[1] = fmax(dg[1], ta);
+    dg[2] = fmin(dg[2], lm);
+    dg[3] = fmax(dg[3], lm);
+  }
+  // (u_g . grad) u
+#pragma unroll
+  for (int i = 0; i < 3; i++) c[i] = ug[0] * gU[0][i] + ug[1] * gU[1][i] + ug[2] * gU[2][i];
+  f3 = k.k3 ? k.rho * tau * dv : (T)0;
+  const T f4 = k.k4 ? k.rho * nuC * div * dv : (T)0, f2 = k.k2 ? dv : (T)0;
+  // strain B u (:222-296): sum_n DN_nb u_ni = gU[b][i], and stress s_k = 2 mu
+  // eps_k + lambda tr eps.  With B-hat the diagonal uses b_n = (avg_n -
+  // DN_n)/3, whose sums are B_k = (P_k - D_k)/3, so eps_k = D_k - 2 B_k + sum_j
+  // B_j, and the node forces are (f2 S + f4 I) DN_n + f2 avg_n o alpha with the
+  // diagonal (5 s_k - ssum)/3 = 10/3 mu eps_k + 2/3 (lambda - mu) tr eps and
+  // alpha_k = (ssum - 2 s_k)/3 = ((2 mu + lambda) tr eps - 4 mu eps_k)/3.
+  if (BHAT) {
+    const T w = div * (T)(1.0 / 3.0);
+    const T trE = (T)(2.0 / 3.0) * div + sc.r;
+    const T f2t = f2 * trE, f2s = f2 * k.mu103;
+    const T d = f4 + f2t * ((T)(2.0 / 3.0) * lam - k.mu23);
+    s.S0 += f2t * (lam * (T)(1.0 / 3.0) + k.mu23);
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const T eps = ((T)(5.0 / 3.0) * gU[i][i] + sc.q[i]) - w;
+      A[i][i] = f2s * eps + d;
+      s.S[i] += f2 * eps;
+    }
+  } else {
+    const T f2s = f2 * k.mu2, d = f4 + f2 * (lam * div);
+#pragma unroll
+    for (int i = 0; i < 3; i++) A[i][i] = f2s * gU[i][i] + d;
+  }
+  const T f2m = f2 * k.mu;
+  const T s3 = f2m * (gU[1][0] + gU[0][1]), s4 = f2m * (gU[2][1] + gU[1][2]), s5 = f2m * (gU[2][0] + gU[0][2]);
+  A[0][1] = A[1][0] = s3;
+  A[1][2] = A[2][1] = s4;
+  A[0][2] = A[2][0] = s5;
+}
+
 // Element block blk of one mesh; its diagnostic row is eblk[row].
 template <typename T, int NPE, bool BHAT, bool DYN, bool PRESS, bool PSEP, bool DIAG>
 __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int blk, const int row) {
   constexpr int NGP = Shape<NPE>::NGP;
-  constexpr int SB = threads_for<NPE>();
+  constexpr int EB = elems_for<NPE>();
+  // hexa8: coordinates and velocities are staged as 1/8 of their values, the
+  // factor of the element transforms (exact)
+  constexpr double SC = NPE == 8 ? 0.125 : 1.0;
   __shared__ double sx[256], sy[256], sz[256], sm[256];
   __shared__ double su[256], sv[256], sw[256];
   __shared__ double pu[PSEP ? 256 : 1], pv[PSEP ? 256 : 1], pw[PSEP ? 256 : 1];
-  __shared__ T sres[DYN ? 3 * NPE * SB : 1];
+  __shared__ T sres[DYN ? 3 * NPE * EB : 1];
   const int tid = threadIdx.x;
   if (halted(a.halt, a.step_id)) return;
   const int n0 = a.node_off[blk], nn = a.node_off[blk + 1] - n0;
   const int e0 = a.elem_off[blk], ne = a.elem_off[blk + 1] - e0;
-  const bool has_e = tid < ne;
-  const int e = e0 + tid;
-  constexpr bool LOWREG = sizeof(T) == 8 && NPE == 8;
-  T out[NPE][3];
-  int id[NPE], ps[NPE];
+  // hexa8: lanes 2 i and 2 i + 1 hold element i's z = -1 and z = 1 sides
+  constexpr int EN = NPE == 8 ? 4 : NPE;  // nodes whose contributions the thread writes
+  const int side = NPE == 8 ? tid & 1 : 0;
+  const int el = NPE == 8 ? tid >> 1 : tid;
+  const bool has_e = el < ne;
+  const int e = e0 + el;
+  T out[EN][3];
+  // the thread's nodes: its element's, or those of its side, and node 0
+  int own[EN], id0 = 0;
+  ushort4 ps4 = make_ushort4(0, 0, 0, 0);
   double dg[11];
 #pragma unroll
   for (int i = 0; i < 11; i++) dg[i] = d_identity(D_TAU + i);
   double lam_prev = 0.0;
   if (has_e) {
-    lconn_load<NPE>(a.lconn, e, id);
-    if (DYN) lpos_load<NPE>(a.lpos, e, ps);
+    const uchar4 c4 = reinterpret_cast<const uchar4 *>(a.lconn)[NPE == 8 ? 2 * e + side : e];
+    own[0] = c4.x; own[1] = c4.y; own[2] = c4.z; own[3] = c4.w;
+    const int oth0 = NPE == 8 ? pair_swap(own[0]) : own[0];  // (every lane of a pair takes part)
+    id0 = side ? oth0 : own[0];
+    if (DYN) {
+      // the thread's EN positions: its element's ushort4, or that of its side
+      ps4 = reinterpret_cast<const ushort4 *>(a.lpos)[NPE == 8 ? 2 * e + side : e];
+    }
     if (PRESS) lam_prev = a.lam[e];
   }
-  for (int j = tid; j < nn; j += SB) {
-    const int g = a.loc_node[n0 + j];
+  if (tid < nn) {
+    const int j = tid, g = a.loc_node[n0 + j];
     const double4 x = a.xyzm[g];
-    sx[j] = x.x; sy[j] = x.y; sz[j] = x.z; sm[j] = x.w;
+    sx[j] = SC * x.x; sy[j] = SC * x.y; sz[j] = SC * x.z; sm[j] = x.w;
     const double4 u = a.U[g];
-    su[j] = u.x; sv[j] = u.y; sw[j] = u.z;
+    su[j] = SC * u.x; sv[j] = SC * u.y; sw[j] = SC * u.z;
     if (PSEP) {
       const double4 q = a.Upress[g];
-      pu[j] = q.x; pv[j] = q.y; pw[j] = q.z;
+      pu[j] = SC * q.x; pv[j] = SC * q.y; pw[j] = SC * q.z;
     }
   }
   __syncthreads();
@@ -257,376 +589,224 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
     const SupgConst &k = a.k;
     using S = ShapeT<T, NPE>;
     // element math in T: differences of the staged FP64 values are formed
-    // in FP64 and rounded once, so FP32 gradients keep their digits
-    const T mu = (T)k.mu, rho = (T)k.rho;
-    // Element kinematics in local coordinates: the physical derivatives
-    // DN = invJ dN/dxi are never formed.  Every term the reference builds
-    // from DN (velocity gradient, divergence, B-hat strain, the K2/K4 node
-    // forces, u.grad N) is the same arithmetic regrouped through the local
-    // derivatives of the table and 3x3 products per Gauss point.
-    // FP64 hexa8 (LOWREG): the node velocities relative to node 0 are read
-    // from LDS where they are used, and each thread keeps its B-hat averages
-    // in its own slots of the contribution buffer sres, unused until after
-    // the Gauss-point loop, instead of in registers through it: with both
-    // live the kernel spilled 236 B per lane at two waves per SIMD.
-    T U0[3], dU[LOWREG ? 1 : NPE][3];  // node velocities relative to node 0 (dU[0] = 0)
-    U0[0] = (T)su[id[0]];
-    U0[1] = (T)sv[id[0]];
-    U0[2] = (T)sw[id[0]];
-    if constexpr (!LOWREG) {
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        dU[n][0] = (T)(su[id[n]] - su[id[0]]);
-        dU[n][1] = (T)(sv[id[n]] - sv[id[0]]);
-        dU[n][2] = (T)(sw[id[n]] - sw[id[0]]);
-      }
-    }
-    auto du = [&](int n, T d[3]) {
-      if constexpr (LOWREG) {
-        d[0] = (T)(su[id[n]] - su[id[0]]);
-        d[1] = (T)(sv[id[n]] - sv[id[0]]);
-        d[2] = (T)(sw[id[n]] - sw[id[0]]);
-      } else {
-        d[0] = dU[n][0];
-        d[1] = dU[n][1];
-        d[2] = dU[n][2];
-      }
-    };
-    // hexa8: the trilinear map's Jacobian rows are J_a = E_a + (xi terms),
-    // from 7 coefficient vectors (femHexa8 node signs, src/femHexa8.cpp:15-17);
-    // tet4 (femTetra4, N3 = 1 - sum xi): constant, J_a = x_a - x_3.
-    T E1[3], E2[3], E3[3], E12[3], E13[3], E23[3], E123[3], Jc[3][3];
-    {
-      T dx[NPE][3];
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        dx[n][0] = (T)(sx[id[n]] - sx[id[0]]);
-        dx[n][1] = (T)(sy[id[n]] - sy[id[0]]);
-        dx[n][2] = (T)(sz[id[n]] - sz[id[0]]);
-      }
-      if constexpr (NPE == 8) {
-        constexpr int s1[8] = {-1, 1, 1, -1, -1, 1, 1, -1}, s2[8] = {-1, -1, 1, 1, -1, -1, 1, 1},
-                      s3[8] = {-1, -1, -1, -1, 1, 1, 1, 1};
+    // in FP64 and rounded once, so FP32 gradients keep their digits.  The
+    // physical derivatives DN = invJ dN/dxi are never formed: every term the
+    // reference builds from DN (velocity gradient, divergence, B-hat strain,
+    // the K2/K4 node forces, u.grad N) is the same arithmetic regrouped
+    // through the local derivatives and 3x3 products per Gauss point.
+    const ElemConst<T> kc(k);
+    ElemAcc<T> acc = {};
+    double vol, mean_div = 0.0;  // the element's volume and mean divergence
+    if constexpr (NPE == 8) {
+      const T q = S::GP(1, 0);  // 1 / sqrt 3
+      // the lane's z direction: the map's handedness, and with it the sign of
+      // det J (the Gauss weights are 1)
+      const T sg = side ? (T)1 : (T)-1;
+      const double q64 = ShapeT<double, 8>::GP(1, 0);
+      auto field = [&](const double *v0, const double *v1, const double *v2, Tri<double> &f) {
+        const double *v[3] = {v0, v1, v2};
 #pragma unroll
         for (int b = 0; b < 3; b++) {
-          T e1 = (T)0, e2 = (T)0, e3 = (T)0, e12 = (T)0, e13 = (T)0, e23 = (T)0, e123 = (T)0;
+          double w[4];
 #pragma unroll
-          for (int n = 1; n < 8; n++) {
-            e1 += (T)s1[n] * dx[n][b];
-            e2 += (T)s2[n] * dx[n][b];
-            e3 += (T)s3[n] * dx[n][b];
-            e12 += (T)(s1[n] * s2[n]) * dx[n][b];
-            e13 += (T)(s1[n] * s3[n]) * dx[n][b];
-            e23 += (T)(s2[n] * s3[n]) * dx[n][b];
-            e123 += (T)(s1[n] * s2[n] * s3[n]) * dx[n][b];
+          for (int n = 0; n < 4; n++) w[n] = v[b][own[n]] - v[b][id0];
+          f.load(b, w, q64);
+        }
+      };
+      // the map and the velocity, rounded to T once; the volume averages of DN
+      // and P_k = sum_n avg_nk u_nk (B-hat), whose sum is the mean divergence
+      // (compute_pressure :446-501; PSEP: of the state before the fixed-DOF
+      // zeroing).  Each thread parks its nodes' averages (in the four (x, y)
+      // coefficients of its side) in its own slots of the contribution
+      // buffer, unused until the Gauss-point loop is over.
+      Tri<T> X, V;
+      T P[3] = {(T)0, (T)0, (T)0};
+      {
+        Tri<double> X64, V64;
+        double P64[3];
+        TriAvg av;
+        field(sx, sy, sz, X64);
+        av.form(X64, q64, (double)sg);
+        vol = av.vol;
+        X.from(X64);
+        field(su, sv, sw, V64);
+        av.dot(V64, q64, P64);
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          P[b] = (T)P64[b];
+          V64.c00[b] += 8.0 * (b == 0 ? su : b == 1 ? sv : sw)[id0];
+        }
+        V.from(V64);
+        if constexpr (PSEP) {
+          field(pu, pv, pw, V64);
+          av.dot(V64, q64, P64);
+        }
+        mean_div = P64[0] + P64[1] + P64[2];
+        if constexpr (BHAT && DYN) {
+#pragma unroll
+          for (int b = 0; b < 3; b++) {
+            sres[(0 * 3 + b) * SB + tid] = (T)av.z[b];
+            sres[(1 * 3 + b) * SB + tid] = (T)(av.x[b] + av.xz[b]);
+            sres[(2 * 3 + b) * SB + tid] = (T)(av.y[b] + av.yz[b]);
+            sres[(3 * 3 + b) * SB + tid] = (T)av.xy[b];
           }
-          E1[b] = (T)0.125 * e1;
-          E2[b] = (T)0.125 * e2;
-          E3[b] = (T)0.125 * e3;
-          E12[b] = (T)0.125 * e12;
-          E13[b] = (T)0.125 * e13;
-          E23[b] = (T)0.125 * e23;
-          E123[b] = (T)0.125 * e123;
         }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-          for (int b = 0; b < 3; b++) Jc[r][b] = dx[r][b] - dx[3][b];
       }
-    }
-    auto jacobian = [&](int g, T J[3][3]) {
-      if constexpr (NPE == 8) {
-        const T xi = S::GP(g, 0), et = S::GP(g, 1), ze = S::GP(g, 2);
+      if constexpr (DYN) {
+        const StrainConst<T, BHAT> sc(P);
+        TriSum<T> os;
+        os.init();
+#pragma unroll 1
+        for (int iy = 0; iy < 2; iy++) {
+          const T y = iy ? q : -q;
+          X.at_y(y);
+          V.at_y(y);
+#pragma unroll 1
+          for (int ix = 0; ix < 2; ix++) {
+            const T x = ix ? q : -q;
+            T J[3][3], iJ[3][3], L[3][3], ug[3], detJ;
+            X.at_x(x, J);
+            V.at_x(x, L);
+            inv3(J, iJ, detJ);
+            const T dv = detJ * sg;
+            // velocity and its gradient gU[b][i] = du_i/dx_b
+            T gU[3][3];
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+              ug[b] = (V.c00[b] + y * V.A2[b]) + x * L[0][b];
+#pragma unroll
+              for (int i = 0; i < 3; i++) gU[b][i] = iJ[b][0] * L[0][i] + iJ[b][1] * L[1][i] + iJ[b][2] * L[2][i];
+            }
+            const T div = gU[0][0] + gU[1][1] + gU[2][2];
+            T gg, trG, f3, c[3], A[3][3];
+            metric3(iJ, gg, trG);
+            // the metric's products with u pair the physical components with
+            // the local directions, as the reference does
+            const T ul[3] = {ug[0], ug[1], sg * ug[2]};
+            gauss_point<T, BHAT, DIAG>(kc, k.dt, ug, gU, div, dv, norm2_tmul(J, ul), norm2_mul(iJ, ul), gg, trG,
+                                       sc, acc, dg, f3, c, A);
+            const T f1 = kc.f1 * dv;
+            // A DN_n + f3 c (u.grad N_n) in the local derivatives:
+            // (A + f3 c (x) u) invJ dN_n
+            T v[3], Tl[3][3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+              v[i] = f1 * c[i];
+              const T fc = f3 * c[i];
+              const T a0 = A[i][0] + fc * ug[0], a1 = A[i][1] + fc * ug[1], a2 = A[i][2] + fc * ug[2];
+#pragma unroll
+              for (int l = 0; l < 3; l++) Tl[i][l] = a0 * iJ[0][l] + a1 * iJ[1][l] + a2 * iJ[2][l];
+            }
+            os.add(x, y, v, Tl);
+          }
+        }
+        acc.lam_int = pair_sum(acc.lam_int);
+        acc.reg = pair_sum(acc.reg);
 #pragma unroll
         for (int b = 0; b < 3; b++) {
-          J[0][b] = E1[b] + et * E12[b] + ze * E13[b] + (et * ze) * E123[b];
-          J[1][b] = E2[b] + xi * E12[b] + ze * E23[b] + (xi * ze) * E123[b];
-          J[2][b] = E3[b] + xi * E13[b] + et * E23[b] + (xi * et) * E123[b];
+          T m[4];
+          os.nodes(b, q, m);
+          if constexpr (BHAT) {
+            const T al = pair_sum(acc.S0 + kc.mu43 * acc.S[b]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) m[i] += sres[(i * 3 + b) * SB + tid] * al;
+          }
+          // nodes (x, y) = (-, -), (+, -), (+, +), (-, +) of the lane's side
+          const T p = m[0] - m[2], r = m[0] + m[2], t = m[1] - m[3], w = m[1] + m[3];
+          out[0][b] = p - t;
+          out[1 % EN][b] = p + t;
+          out[2 % EN][b] = r + w;
+          out[3 % EN][b] = r - w;
         }
-      } else {
+      }
+    } else {
+      // tet4 (femTetra4, N3 = 1 - sum xi): the Jacobian, its inverse, the
+      // velocity gradient and the metric are the same at every Gauss point,
+      // and so are the physical derivatives, DN_n = column n of invJ: the
+      // node forces are one matrix K = sum_g (A + f3 c (x) u) applied to
+      // them, plus the convection's values.
+      T J[3][3], iJ[3][3], L[3][3], gU[3][3], detJ, u[4][3];
+      {
+        const double *xs[3] = {sx, sy, sz}, *us[3] = {su, sv, sw};
 #pragma unroll
         for (int r = 0; r < 3; r++)
 #pragma unroll
-          for (int b = 0; b < 3; b++) J[r][b] = Jc[r][b];
+          for (int b = 0; b < 3; b++) {
+            J[r][b] = (T)(xs[b][own[r]] - xs[b][own[3]]);
+            L[r][b] = (T)(us[b][own[r]] - us[b][own[3]]);
+          }
+#pragma unroll
+        for (int n = 0; n < 4; n++)
+#pragma unroll
+          for (int b = 0; b < 3; b++) u[n][b] = (T)(us[b][own[n]] - us[b][id0]);
       }
-    };
-    // eval_avg_shapeDeriv (:660-707): volume average of DN (hexa only);
-    // with it the B-hat strain needs P_k = sum_n avg_nk u_nk per element.
-    auto avg_pass = [&](T avg[NPE][3]) {
-#pragma unroll
-      for (int n = 0; n < NPE; n++) avg[n][0] = avg[n][1] = avg[n][2] = (T)0;
-      T den = (T)0;
-      for (int g = 0; g < NGP; g++) {
-        T J[3][3], iJ[3][3], detJ;
-        jacobian(g, J);
-        inv3(J, iJ, detJ);
-        const T dv = detJ * S::W();
-        T Q[3][3];
-#pragma unroll
-        for (int b = 0; b < 3; b++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) Q[b][c] = iJ[b][c] * dv;
-#pragma unroll
-        for (int n = 0; n < NPE; n++)
-#pragma unroll
-          for (int b = 0; b < 3; b++)
-            avg[n][b] += Q[b][0] * S::dN(g, n, 0) + Q[b][1] * S::dN(g, n, 1) + Q[b][2] * S::dN(g, n, 2);
-        den += dv;
-      }
-      const T iden = recip(den);
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        avg[n][0] *= iden;
-        avg[n][1] *= iden;
-        avg[n][2] *= iden;
-      }
-    };
-    T avg[LOWREG ? 1 : NPE][3], P[3] = {(T)0, (T)0, (T)0};
-    if (BHAT && LOWREG) {
-      T av[NPE][3];
-      avg_pass(av);
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        T d[3];
-        du(n, d);
-        P[0] += av[n][0] * d[0];  // sum_n avg_n = 0: relative velocities suffice
-        P[1] += av[n][1] * d[1];
-        P[2] += av[n][2] * d[2];
-        if constexpr (DYN)
-#pragma unroll
-          for (int b = 0; b < 3; b++) sres[(n * 3 + b) * SB + tid] = av[n][b];
-      }
-    } else if (BHAT) {
-      // the same as avg_pass, written out (FP32 keeps its unrolled form)
-#pragma unroll
-      for (int n = 0; n < NPE; n++) avg[n][0] = avg[n][1] = avg[n][2] = (T)0;
-      T den = (T)0;
-      for (int g = 0; g < NGP; g++) {
-        T J[3][3], iJ[3][3], detJ;
-        jacobian(g, J);
-        inv3(J, iJ, detJ);
-        const T dv = detJ * S::W();
-        T Q[3][3];
-#pragma unroll
-        for (int b = 0; b < 3; b++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) Q[b][c] = iJ[b][c] * dv;
-#pragma unroll
-        for (int n = 0; n < NPE; n++)
-#pragma unroll
-          for (int b = 0; b < 3; b++)
-            avg[n][b] += Q[b][0] * S::dN(g, n, 0) + Q[b][1] * S::dN(g, n, 1) + Q[b][2] * S::dN(g, n, 2);
-        den += dv;
-      }
-      const T iden = recip(den);
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        avg[n][0] *= iden;
-        avg[n][1] *= iden;
-        avg[n][2] *= iden;
-        P[0] += avg[n][0] * dU[n][0];
-        P[1] += avg[n][1] * dU[n][1];
-        P[2] += avg[n][2] * dU[n][2];
-      }
-    }
-#pragma unroll
-    for (int n = 0; n < NPE; n++) out[n][0] = out[n][1] = out[n][2] = (T)0;
-    // per-thread diagnostic accumulators, columns D_TAU .. D_NU+1
-    T vol = (T)0, lam_int = (T)0, reg = (T)0, pnum = (T)0;
-    T Aacc[3] = {(T)0, (T)0, (T)0};  // sum over Gauss points of f2 alpha (the B-hat avg term)
-    const T nu_k = mu / rho;
-    // tet4: the Jacobian, its inverse and the metric are the same at every Gauss point
-    T iJc[3][3], detJc = (T)0;
-    if constexpr (NPE == 4) inv3(Jc, iJc, detJc);
-    for (int g = 0; g < NGP; g++) {
-      T iJ[3][3], detJ;
-      if constexpr (NPE == 8) {
-        T J[3][3];
-        jacobian(g, J);
-        inv3(J, iJ, detJ);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) iJ[r][c] = iJc[r][c];
-        detJ = detJc;
-      }
-      const T dv = detJ * S::W();
-      vol += dv;
-      // u at the Gauss point and the velocity gradient gU[b][i] = du_i/dx_b
-      T ug[3] = {U0[0], U0[1], U0[2]}, L[3][3];
-#pragma unroll
-      for (int c = 0; c < 3; c++) L[c][0] = L[c][1] = L[c][2] = (T)0;
-#pragma unroll
-      for (int n = 1; n < NPE; n++) {
-        const T Nn = S::N(g, n);
-        T dn[3];
-        du(n, dn);
-#pragma unroll
-        for (int i = 0; i < 3; i++) ug[i] += Nn * dn[i];
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          const T d = S::dN(g, n, c);
-          L[c][0] += d * dn[0];
-          L[c][1] += d * dn[1];
-          L[c][2] += d * dn[2];
-        }
-      }
-      T gU[3][3];
+      inv3(J, iJ, detJ);
 #pragma unroll
       for (int b = 0; b < 3; b++)
 #pragma unroll
         for (int i = 0; i < 3; i++) gU[b][i] = iJ[b][0] * L[0][i] + iJ[b][1] * L[1][i] + iJ[b][2] * L[2][i];
-      const T div = gU[0][0] + gU[1][1] + gU[2][2];
-      if (PRESS) {
-        if (PSEP) {
-          T Lp[3][3];
+      const T dv = detJ * S::W(), div = gU[0][0] + gU[1][1] + gU[2][2];
+      vol = (double)((T)NGP * dv);
+      const T U0[3] = {(T)su[id0], (T)sv[id0], (T)sw[id0]};
+      if constexpr (PRESS && PSEP) {
+        const double *qs[3] = {pu, pv, pw};
+        T dp = (T)0;
 #pragma unroll
-          for (int c = 0; c < 3; c++) Lp[c][0] = Lp[c][1] = Lp[c][2] = (T)0;
+        for (int b = 0; b < 3; b++)
 #pragma unroll
-          for (int n = 1; n < NPE; n++) {
-            const T q0 = (T)(pu[id[n]] - pu[id[0]]), q1 = (T)(pv[id[n]] - pv[id[0]]), q2 = (T)(pw[id[n]] - pw[id[0]]);
+          for (int r = 0; r < 3; r++) dp += iJ[b][r] * (T)(qs[b][own[r]] - qs[b][own[3]]);
+        mean_div = dp;
+      } else if constexpr (PRESS) {
+        mean_div = div;
+      }
+      if constexpr (DYN) {
+        T gg, trG, K[3][3], cN[4][3];
+        const T P[3] = {(T)0, (T)0, (T)0};
+        const StrainConst<T, false> sc(P);
+        metric3(iJ, gg, trG);
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-              const T d = S::dN(g, n, c);
-              Lp[c][0] += d * q0;
-              Lp[c][1] += d * q1;
-              Lp[c][2] += d * q2;
-            }
+        for (int i = 0; i < 3; i++) {
+          K[i][0] = K[i][1] = K[i][2] = (T)0;
+          cN[0][i] = cN[1][i] = cN[2][i] = cN[3][i] = (T)0;
+        }
+#pragma unroll 1
+        for (int g = 0; g < NGP; g++) {
+          T ug[3], f3, c[3], A[3][3];
+#pragma unroll
+          for (int b = 0; b < 3; b++)
+            ug[b] = U0[b] + (S::N(g, 1) * u[1][b] + S::N(g, 2 % NPE) * u[2][b] + S::N(g, 3 % NPE) * u[3][b]);
+          gauss_point<T, false, DIAG>(kc, k.dt, ug, gU, div, dv, norm2_tmul(J, ug), norm2_mul(iJ, ug), gg, trG, sc, acc,
+                                      dg, f3, c, A);
+          const T f1 = kc.f1 * dv;
+#pragma unroll
+          for (int i = 0; i < 3; i++) {
+            const T fc = f3 * c[i], vc = f1 * c[i];
+#pragma unroll
+            for (int b = 0; b < 3; b++) K[i][b] += A[i][b] + fc * ug[b];
+#pragma unroll
+            for (int n = 0; n < 4; n++) cN[n][i] += vc * S::N(g, n % NPE);
           }
-          T dp = (T)0;
+        }
 #pragma unroll
-          for (int b = 0; b < 3; b++) dp += iJ[b][0] * Lp[0][b] + iJ[b][1] * Lp[1][b] + iJ[b][2] * Lp[2][b];
-          pnum += dp * dv;
-        } else {
-          pnum += div * dv;
+        for (int i = 0; i < 3; i++) {
+          T f[3];
+#pragma unroll
+          for (int n = 0; n < 3; n++) {
+            f[n] = K[i][0] * iJ[0][n] + K[i][1] * iJ[1][n] + K[i][2] * iJ[2][n];
+            out[n % EN][i] = cN[n][i] + f[n];
+          }
+          out[3 % EN][i] = cN[3][i] - (f[0] + f[1] + f[2]);
         }
       }
-      if (!DYN) continue;
-      // metric G = invJ^T invJ in the reference's index order (src/femElement.cpp:222-231)
-      T G[3][3];
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) G[i][j] = iJ[0][i] * iJ[0][j] + iJ[1][i] * iJ[1][j] + iJ[2][i] * iJ[2][j];
-      // eval_stabilization (:336-377), tau without the (2/dt)^2 term
-      T t2 = (T)0, t3 = (T)0;
-#pragma unroll
-      for (int i = 0; i < 3; i++) {
-        t2 += ug[i] * (G[i][0] * ug[0] + G[i][1] * ug[1] + G[i][2] * ug[2]);
-        t3 += G[i][0] * G[i][0] + G[i][1] * G[i][1] + G[i][2] * G[i][2];
-      }
-      t3 = t3 * nu_k * nu_k * (T)k.cI;
-      const T tau = recip(sqrt_e(t2 + t3));
-      const T trG = G[0][0] + G[1][1] + G[2][2];
-      const T nuC = recip(trG * tau);
-      // eval_bulk_modulus (:382-441): lambda = alpha max(mu/rho, sqrt(u^T G^-1 u))
-      T iG[3][3], dG;
-      inv3(G, iG, dG);
-      T l2 = (T)0;
-#pragma unroll
-      for (int i = 0; i < 3; i++) l2 += (iG[i][0] * ug[0] + iG[i][1] * ug[1] + iG[i][2] * ug[2]) * ug[i];
-      l2 = sqrt_e(l2);
-      const T lam = (T)k.alpha * ((nu_k < l2) ? l2 : nu_k);
-      reg += (nu_k > l2) ? (T)1 : (T)2;
-      lam_int += lam * dv;
-      if (DIAG) {
-        // get_el_lengths_from_G (:756-790) and the CFL / tau / lambda extrema (:1187-1240), in FP64
-        const double u0 = ug[0], u1 = ug[1], u2 = ug[2];
-        const double un = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
-        const double o0 = u0 / un, o1 = u1 / un, o2 = u2 / un;
-        const double el = 2.0 * sqrt(((double)iG[0][0] * o0 + (double)iG[0][1] * o1 + (double)iG[0][2] * o2) * o0 +
-                                     ((double)iG[1][0] * o0 + (double)iG[1][1] * o1 + (double)iG[1][2] * o2) * o1 +
-                                     ((double)iG[2][0] * o0 + (double)iG[2][1] * o1 + (double)iG[2][2] * o2) * o2);
-        const double nk = nu_k, lm = lam, ta = tau;
-        dg[D_ACFL - D_TAU] = fmax(dg[D_ACFL - D_TAU], fabs(u0 * k.dt) / el);
-        dg[D_VCFL - D_TAU] = fmax(dg[D_VCFL - D_TAU], 2.0 * nk * (k.dt / (el * el)));
-        dg[D_LCFL - D_TAU] = fmax(dg[D_LCFL - D_TAU], 2.0 * lm * (k.dt / (el * el)));
-        dg[0] = fmin(dg[0], ta);
-        dg[1] = fmax(dg[1], ta);
-        dg[2] = fmin(dg[2], lm);
-        dg[3] = fmax(dg[3], lm);
-      }
-      // (u_g . grad) u
-      T c[3];
-#pragma unroll
-      for (int i = 0; i < 3; i++) c[i] = ug[0] * gU[0][i] + ug[1] * gU[1][i] + ug[2] * gU[2][i];
-      // strain B u (:222-296): sum_n DN_nb u_ni = gU[b][i]; with B-hat the
-      // diagonal uses b_n = (avg_n - DN_n)/3, whose sums are B_k = (P_k - D_k)/3
-      const T third = (T)(1.0 / 3.0);
-      T eps[6];
-      if (BHAT) {
-        const T B0 = (P[0] - gU[0][0]) * third, B1 = (P[1] - gU[1][1]) * third, B2 = (P[2] - gU[2][2]) * third;
-        const T Bs = B0 + B1 + B2;
-        eps[0] = gU[0][0] - (T)2 * B0 + Bs;
-        eps[1] = gU[1][1] - (T)2 * B1 + Bs;
-        eps[2] = gU[2][2] - (T)2 * B2 + Bs;
-      } else {
-        eps[0] = gU[0][0];
-        eps[1] = gU[1][1];
-        eps[2] = gU[2][2];
-      }
-      eps[3] = gU[1][0] + gU[0][1];
-      eps[4] = gU[2][1] + gU[1][2];
-      eps[5] = gU[2][0] + gU[0][2];
-      const T trE = eps[0] + eps[1] + eps[2];
-      const T s0 = (T)2 * mu * eps[0] + lam * trE, s1 = (T)2 * mu * eps[1] + lam * trE,
-              s2 = (T)2 * mu * eps[2] + lam * trE;
-      const T s3 = mu * eps[3], s4 = mu * eps[4], s5 = mu * eps[5];
-      const T ssum = s0 + s1 + s2;
-      const T f1 = k.k1 ? rho * dv : (T)0, f3 = k.k3 ? rho * tau * dv : (T)0;
-      const T f4 = k.k4 ? rho * nuC * div * dv : (T)0, f2 = k.k2 ? dv : (T)0;
-      // node forces (K2 u)_n + f4 DN_n = (f2 S + f4 I) DN_n (+ f2 avg_n o alpha
-      // with B-hat), with S the stress matrix (B-hat: diagonal (5 s_k - ssum)/3,
-      // alpha_k = (ssum - 2 s_k)/3); DN_n = invJ dN_n gives Mg = (f2 S + f4 I) invJ
-      const T sd0 = BHAT ? ((T)5 * s0 - ssum) * third : s0;
-      const T sd1 = BHAT ? ((T)5 * s1 - ssum) * third : s1;
-      const T sd2 = BHAT ? ((T)5 * s2 - ssum) * third : s2;
-      if (BHAT) {
-        Aacc[0] += f2 * ((ssum - (T)2 * s0) * third);
-        Aacc[1] += f2 * ((ssum - (T)2 * s1) * third);
-        Aacc[2] += f2 * ((ssum - (T)2 * s2) * third);
-      }
-      const T A[3][3] = {{f2 * sd0 + f4, f2 * s3, f2 * s5},
-                         {f2 * s3, f2 * sd1 + f4, f2 * s4},
-                         {f2 * s5, f2 * s4, f2 * sd2 + f4}};
-      T Mg[3][3], w3[3];
-#pragma unroll
-      for (int i = 0; i < 3; i++) {
-#pragma unroll
-        for (int cc = 0; cc < 3; cc++) Mg[i][cc] = A[i][0] * iJ[0][cc] + A[i][1] * iJ[1][cc] + A[i][2] * iJ[2][cc];
-        w3[i] = iJ[0][i] * ug[0] + iJ[1][i] * ug[1] + iJ[2][i] * ug[2];  // u.grad N_n = w3 . dN_n
-      }
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        const T d0 = S::dN(g, n, 0), d1 = S::dN(g, n, 1), d2 = S::dN(g, n, 2);
-        const T cv = f1 * S::N(g, n) + f3 * (w3[0] * d0 + w3[1] * d1 + w3[2] * d2);
-        out[n][0] += cv * c[0] + (Mg[0][0] * d0 + Mg[0][1] * d1 + Mg[0][2] * d2);
-        out[n][1] += cv * c[1] + (Mg[1][0] * d0 + Mg[1][1] * d1 + Mg[1][2] * d2);
-        out[n][2] += cv * c[2] + (Mg[2][0] * d0 + Mg[2][1] * d1 + Mg[2][2] * d2);
-      }
     }
-    if (BHAT && DYN && LOWREG) {
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        out[n][0] += sres[(n * 3 + 0) * SB + tid] * Aacc[0];
-        out[n][1] += sres[(n * 3 + 1) * SB + tid] * Aacc[1];
-        out[n][2] += sres[(n * 3 + 2) * SB + tid] * Aacc[2];
-      }
-    } else if (BHAT && DYN) {
-#pragma unroll
-      for (int n = 0; n < NPE; n++) {
-        out[n][0] += avg[n][0] * Aacc[0];
-        out[n][1] += avg[n][1] * Aacc[1];
-        out[n][2] += avg[n][2] * Aacc[2];
-      }
-    }
-    if (PRESS) a.pres[e] = -lam_prev * ((double)pnum / (double)vol);  // compute_pressure of the previous step (:498)
+    const bool writes = side == 0;  // the element's outputs
+    if (PRESS && writes) a.pres[e] = -lam_prev * mean_div;  // compute_pressure of the previous step (:498)
     if (DYN) {
-      const double lame = (double)lam_int / (double)vol;  // :1446
-      a.lam[e] = lame;
-      a.regime[e] = (double)reg / NGP;
+      const double lame = (double)acc.lam_int / vol;  // :1446
+      if (writes) {
+        a.lam[e] = lame;
+        a.regime[e] = (double)acc.reg / NGP;
+      }
       if (DIAG) {
         const double cE = (k.mu * (3 * lame + 2 * k.mu)) / (lame + k.mu), cnu = lame / (2 * (lame + k.mu));
         dg[D_E - D_TAU] = fmin(dg[D_E - D_TAU], cE);
@@ -634,25 +814,27 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         dg[D_NU - D_TAU] = fmin(dg[D_NU - D_TAU], cnu);
         dg[D_NU + 1 - D_TAU] = fmax(dg[D_NU + 1 - D_TAU], cnu);
       }
-      if constexpr (!(BHAT && LOWREG)) {
-        const T mdt = (T)(-k.dt);
+      if constexpr (!(BHAT && NPE == 8)) {
+        const T mdt = (T)(-k.dt * SC);
+        const int ps[4] = {ps4.x, ps4.y, ps4.z, ps4.w};
 #pragma unroll
-        for (int n = 0; n < NPE; n++)
+        for (int n = 0; n < EN; n++)
 #pragma unroll
-          for (int i = 0; i < 3; i++) sres[i * (NPE * SB) + ps[n]] = mdt * out[n][i];
+          for (int i = 0; i < 3; i++) sres[i * (NPE * EB) + ps[n]] = mdt * out[n][i];
       }
     }
   }
   if (!DYN) return;
-  if constexpr (BHAT && LOWREG) {
+  if constexpr (BHAT && NPE == 8) {
     // every thread has read its averages back from sres
     __syncthreads();
     if (has_e) {
-      const T mdt = (T)(-a.k.dt);
+      const T mdt = (T)(-a.k.dt * SC);
+      const int ps[4] = {ps4.x, ps4.y, ps4.z, ps4.w};
 #pragma unroll
-      for (int n = 0; n < NPE; n++)
+      for (int n = 0; n < EN; n++)
 #pragma unroll
-        for (int i = 0; i < 3; i++) sres[i * (NPE * SB) + ps[n]] = mdt * out[n][i];
+        for (int i = 0; i < 3; i++) sres[i * (NPE * EB) + ps[n]] = mdt * out[n][i];
     }
   }
   if (DIAG) block_diag_store<SB, 11>(dg, D_TAU, a.eblk + (long)row * D_COLS);
@@ -663,7 +845,8 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
 #pragma unroll
   for (int i = 0; i < 6; i++) nv[i] = d_identity(D_UMIN + i);
   const int base_s = e0 * NPE;
-  for (int j = tid; j < nn; j += SB) {
+  if (tid < nn) {
+    const int j = tid;
     // the node's contributions summed in FP64, or in FP32 with f32sum
     double F[3] = {0.0, 0.0, 0.0};
     const int s0 = a.lcsr_off[n0 + j] - base_s, s1 = a.lcsr_off[n0 + j + 1] - base_s;
@@ -671,9 +854,9 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
       float Ft[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll 4
       for (int s = s0; s < s1; s++) {
-        Ft[0] += (float)sres[0 * (NPE * SB) + s];
-        Ft[1] += (float)sres[1 * (NPE * SB) + s];
-        Ft[2] += (float)sres[2 * (NPE * SB) + s];
+        Ft[0] += (float)sres[0 * (NPE * EB) + s];
+        Ft[1] += (float)sres[1 * (NPE * EB) + s];
+        Ft[2] += (float)sres[2 * (NPE * EB) + s];
       }
       F[0] = Ft[0];
       F[1] = Ft[1];
@@ -681,9 +864,9 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
     } else {
 #pragma unroll 4
       for (int s = s0; s < s1; s++) {
-        F[0] += (double)sres[0 * (NPE * SB) + s];
-        F[1] += (double)sres[1 * (NPE * SB) + s];
-        F[2] += (double)sres[2 * (NPE * SB) + s];
+        F[0] += (double)sres[0 * (NPE * EB) + s];
+        F[1] += (double)sres[1 * (NPE * EB) + s];
+        F[2] += (double)sres[2 * (NPE * EB) + s];
       }
     }
     const int psl = a.loc_pslot[n0 + j];
@@ -691,7 +874,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
     if (psl < 0) {
       double4 next, pst, fst;
       const double4 fp = a.k.euler_step ? make_double4(0, 0, 0, 0) : a.Fprev[g];
-      supg_node(F, fp, sm[j], make_double4(su[j], sv[j], sw[j], 0.0), a.k, a.node_rec[g], a.rec, a.row_off, a.rows,
+      supg_node(F, fp, sm[j], make_double4(su[j] * (1.0 / SC), sv[j] * (1.0 / SC), sw[j] * (1.0 / SC), 0.0), a.k, a.node_rec[g], a.rec, a.row_off, a.rows,
                 a.err, next, pst, fst);
       a.Un[g] = next;
       if (a.Unp) a.Unp[g] = pst;
@@ -708,8 +891,13 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
   if (a.want_row) block_node_store<SB>(nv, nm2[0], a.eblk + (long)row * D_COLS);
 }
 
+// Waves per SIMD: FP32 hexa8 fits three (168 VGPRs) without spills as long as
+// its two Gauss points of one y are not unrolled; four spill 100 B per lane
+// (328 against 270 us at 2.1M hexa).  The others are bound to two (FP64 hexa8
+// spills 148 B).
+#define SUPG_BLOCK_WAVES(T, NPE) (sizeof(T) == 4 && NPE == 8 ? 3 : 2)
 template <typename T, int NPE, bool BHAT, bool DYN, bool PRESS, bool PSEP, bool DIAG>
-__global__ __launch_bounds__(threads_for<NPE>(), 2) void supg_block(SupgArgs<T> a) {
+__global__ __launch_bounds__(SB, SUPG_BLOCK_WAVES(T, NPE)) void supg_block(SupgArgs<T> a) {
   supg_block_run<T, NPE, BHAT, DYN, PRESS, PSEP, DIAG>(a, xcd_block(blockIdx.x, a.nblk), blockIdx.x);
 }
 
@@ -1062,7 +1250,6 @@ template <typename T, int NPE, bool BHAT>
 void launch_supg_t(femx_supg *s, SupgArgs<T> &a, bool dyn, bool press, bool diag) {
   const int grd = s->mesh->blk.nb;
   const bool psep = press && s->p.fixed_dofs != 0;
-  constexpr int SB = threads_for<NPE>();
 #define L(D, P, PS, G) supg_block<T, NPE, BHAT, D, P, PS, G><<<grd, SB, 0, s->st>>>(a)
   if (!dyn) {
     if (psep) L(false, true, true, false);
@@ -1201,8 +1388,8 @@ extern "C" femx_status femx_supg_create(femx_mesh *mh, const femx_bc_desc *bc, c
   if (p->fixed_dofs < 0 || p->fixed_dofs > 6) return set_error("ERROR: Invalid global fixed DOFs string."), FEMX_ERR_ARG;
   if (!valid_precision(p->precision)) return set_error("precision"), FEMX_ERR_ARG;
   if (!(p->dt > 0.0) || p->rho == 0.0) return set_error("parameters"), FEMX_ERR_ARG;
-  const int threads = m.npe == 4 ? 256 : 128;
-  if (m.blk.B > threads || m.blk.max_local > 256)
+  const int elems = m.npe == 4 ? elems_for<4>() : elems_for<8>();
+  if (m.blk.B > elems || m.blk.max_local > 256)
     return set_error("element blocks do not fit the SUPG workgroup"), FEMX_ERR_ARG;
   femx_status r;
   if ((r = upload_tables(m.device)) != FEMX_OK) return r;
@@ -1530,7 +1717,7 @@ __device__ __forceinline__ int supg_member_of(const int *off, int nm, int g) {
   return lo;
 }
 
-__global__ __launch_bounds__(threads_for<8>(), 2) void supg_block_union(const SupgMember *mem, const int *blk_off,
+__global__ __launch_bounds__(SB, SUPG_BLOCK_WAVES(float, 8)) void supg_block_union(const SupgMember *mem, const int *blk_off,
                                                                         int nm, int ntot, int last) {
   const int g = xcd_block(blockIdx.x, ntot);
   const int h = supg_member_of(blk_off, nm, g);
@@ -1756,7 +1943,7 @@ extern "C" femx_status femx_supg_union_step(femx_supg_union *u, int k) {
   const int *blk_off = u->off.p, *fx_off = u->off.p + nm + 1;
   for (int i = 0; i < k; i++) {
     const int last = i == k - 1;
-    supg_block_union<<<u->nblk, threads_for<8>(), 0, u->st>>>(u->tab.p, blk_off, nm, u->nblk, last);
+    supg_block_union<<<u->nblk, SB, 0, u->st>>>(u->tab.p, blk_off, nm, u->nblk, last);
     supg_fixup_union<<<u->nfx, 256, 0, u->st>>>(u->tab.p, fx_off, nm, last);
     supg_union_tick<<<nm, 256, 0, u->st>>>(u->tab.p, last);
   }
