@@ -174,6 +174,142 @@ void stream_put(hipStream_t st) {
   (void)hipStreamDestroy(st);
 }
 
+// ------------------------------------------------------------ read-back
+namespace {
+constexpr size_t PIN_CHUNK = size_t(2) << 20;
+constexpr size_t PIN_IDLE = 16;  // idle chunks kept per device (32 MiB)
+
+struct Pin {
+  unsigned char *p = nullptr;
+  hipEvent_t ev = nullptr;
+};
+
+struct PinPool {
+  std::mutex mu;
+  std::vector<Pin> idle[CACHE_DEVICES];
+};
+PinPool &pins() {
+  static PinPool *p = new PinPool();  // never destroyed, as the device cache
+  return *p;
+}
+
+void pin_free(Pin &c) {
+  if (c.ev) (void)hipEventDestroy(c.ev);
+  if (c.p) (void)hipHostFree(c.p);
+  c = Pin();
+}
+
+hipError_t pin_get(int d, Pin &c) {
+  {
+    std::lock_guard<std::mutex> lk(pins().mu);
+    auto &v = pins().idle[d];
+    if (!v.empty()) {
+      c = v.back();
+      v.pop_back();
+      return hipSuccess;
+    }
+  }
+  hipError_t e = hipHostMalloc((void **)&c.p, PIN_CHUNK, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&c.ev, hipEventDisableTiming);
+  if (e != hipSuccess) pin_free(c);
+  return e;
+}
+
+void pin_put(int d, Pin &c) {
+  if (!c.p) return;
+  {
+    std::lock_guard<std::mutex> lk(pins().mu);
+    if (pins().idle[d].size() < PIN_IDLE) {
+      pins().idle[d].push_back(c);
+      return;
+    }
+  }
+  pin_free(c);
+}
+
+// Pieces of at most one chunk, taken from a shared counter: the thread's two
+// chunks alternate, so that the next piece is in flight while one is copied out.
+hipError_t read_pieces(hipStream_t st, int d, const std::vector<ReadPiece> &q, std::atomic<size_t> &next) {
+  Pin c[2];
+  size_t in_c[2] = {0, 0};
+  bool busy[2] = {false, false};
+  hipError_t e = hipSetDevice(d);
+  for (int i = 0; i < 2 && e == hipSuccess; i++) e = pin_get(d, c[i]);
+  for (int i = 0; e == hipSuccess; i ^= 1) {
+    // queue the next piece into chunk i, then drain the other one
+    const size_t k = next.fetch_add(1);
+    if (k < q.size()) {
+      e = hipMemcpyAsync(c[i].p, q[k].src, q[k].bytes, hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipEventRecord(c[i].ev, st);
+      if (e != hipSuccess) break;
+      in_c[i] = k;
+      busy[i] = true;
+    }
+    const int o = i ^ 1;
+    if (busy[o]) {
+      e = hipEventSynchronize(c[o].ev);
+      if (e == hipSuccess) std::memcpy(q[in_c[o]].dst, c[o].p, q[in_c[o]].bytes);
+      busy[o] = false;
+    } else if (k >= q.size()) {
+      break;
+    }
+  }
+  // after an error no chunk goes back while a copy into it may still run
+  if (e != hipSuccess) (void)hipStreamSynchronize(st);
+  for (int i = 0; i < 2; i++) pin_put(d, c[i]);
+  return e;
+}
+}  // namespace
+
+femx_status read_back(hipStream_t st, const ReadPiece *p, int n) {
+  size_t total = 0;
+  for (int i = 0; i < n; i++) total += (p[i].bytes + 63) & ~size_t(63);
+  int d = 0;
+  FEMX_HIP(hipGetDevice(&d));
+  if (d < 0 || d >= CACHE_DEVICES) {
+    for (int i = 0; i < n; i++)
+      if (p[i].bytes) FEMX_HIP(hipMemcpyAsync(p[i].dst, p[i].src, p[i].bytes, hipMemcpyDeviceToHost, st));
+    FEMX_HIP(hipStreamSynchronize(st));
+    return FEMX_OK;
+  }
+  if (total <= PIN_CHUNK) {
+    Pin c;
+    FEMX_HIP(pin_get(d, c));
+    hipError_t e = hipSuccess;
+    size_t off = 0;
+    for (int i = 0; i < n && e == hipSuccess; i++) {
+      if (p[i].bytes) e = hipMemcpyAsync(c.p + off, p[i].src, p[i].bytes, hipMemcpyDeviceToHost, st);
+      off += (p[i].bytes + 63) & ~size_t(63);
+    }
+    const hipError_t w = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = w;
+    off = 0;
+    for (int i = 0; i < n && e == hipSuccess; i++) {
+      if (p[i].bytes) std::memcpy(p[i].dst, c.p + off, p[i].bytes);
+      off += (p[i].bytes + 63) & ~size_t(63);
+    }
+    pin_put(d, c);
+    FEMX_HIP(e);
+    return FEMX_OK;
+  }
+  std::vector<ReadPiece> q;
+  for (int i = 0; i < n; i++)
+    for (size_t o = 0; o < p[i].bytes; o += PIN_CHUNK)
+      q.push_back({(unsigned char *)p[i].dst + o, (const unsigned char *)p[i].src + o,
+                   std::min(PIN_CHUNK, p[i].bytes - o)});
+  const int h = q.size() < 4 ? 0 : take_helpers((int)std::min<size_t>(7, q.size() / 2 - 1));
+  std::atomic<size_t> next{0};
+  std::vector<hipError_t> err(h + 1, hipSuccess);
+  std::vector<std::thread> th;
+  for (int t = 1; t <= h; t++) th.emplace_back([&, t] { err[t] = read_pieces(st, d, q, next); });
+  err[0] = read_pieces(st, d, q, next);
+  for (auto &x : th) x.join();
+  if (h) give_helpers(h);
+  for (hipError_t e : err) FEMX_HIP(e);
+  FEMX_HIP(hipStreamSynchronize(st));
+  return FEMX_OK;
+}
+
 femx_status BCDev::build(const femx_bc_desc *bc, int N, bool with_pressure, hipStream_t st) {
   std::vector<int> node_rec(N, -1);
   std::vector<BCRecord> recs;
@@ -772,6 +908,17 @@ extern "C" femx_status femx_set_device_cache(size_t max_bytes_per_device) {
   }
   for (void *p : idle) (void)hipFree(p);
   for (hipStream_t st : streams) (void)hipStreamDestroy(st);
+  if (max_bytes_per_device == 0) {
+    std::vector<Pin> chunks;
+    {
+      std::lock_guard<std::mutex> lk(pins().mu);
+      for (auto &v : pins().idle) {
+        chunks.insert(chunks.end(), v.begin(), v.end());
+        v.clear();
+      }
+    }
+    for (Pin &c : chunks) pin_free(c);
+  }
   return FEMX_OK;
 }
 

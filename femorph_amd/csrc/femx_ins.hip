@@ -148,6 +148,19 @@ __global__ __launch_bounds__(256) void ins_pack(int N, const double *phi, const 
   vphi[a] = v;
 }
 
+// phi [N] and/or velocity [N][3] of the node records into the staging array.
+__global__ __launch_bounds__(256) void ins_unpack(int N, const double4 *vphi, double *phi, double *vel) {
+  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a >= N) return;
+  const double4 v = vphi[a];
+  if (phi) phi[a] = v.w;
+  if (vel) {
+    vel[3L * a] = v.x;
+    vel[3L * a + 1] = v.y;
+    vel[3L * a + 2] = v.z;
+  }
+}
+
 // ------------------------------------------------------------- element
 // Element t of the processing order (the mesh's Morton block order; every
 // per-element input is stored in that order).  Each XCD takes a contiguous
@@ -1003,19 +1016,18 @@ extern "C" femx_status femx_ins_get_state(femx_ins *s, double *phi, double *phi_
   }
   FEMX_HIP(hipSetDevice(s->mesh->device));
   const int N = s->mesh->N;
-  std::vector<double4> h(N);
-  FEMX_HIP(hipMemcpyAsync(h.data(), s->vphi.p, sizeof(double4) * N, hipMemcpyDeviceToHost, s->st));
-  if (phi_dot) FEMX_HIP(hipMemcpyAsync(phi_dot, s->phid.p, sizeof(double) * N, hipMemcpyDeviceToHost, s->st));
-  FEMX_HIP(hipStreamSynchronize(s->st));
-  for (int a = 0; a < N; a++) {
-    if (phi) phi[a] = h[a].w;
-    if (vel) {
-      vel[3L * a] = h[a].x;
-      vel[3L * a + 1] = h[a].y;
-      vel[3L * a + 2] = h[a].z;
-    }
+  // phi passes through the Krylov work vector w[0], free between solves
+  double *dphi = phi ? s->w[0].p : nullptr, *dvel = vel ? s->stage.p : nullptr;
+  ReadPiece rb[3];
+  int nrb = 0;
+  if (phi || vel) {
+    ins_unpack<<<grid_for(N, 256), 256, 0, s->st>>>(N, s->vphi.p, dphi, dvel);
+    FEMX_HIP(hipGetLastError());
   }
-  return FEMX_OK;
+  if (phi) rb[nrb++] = {phi, dphi, sizeof(double) * N};
+  if (vel) rb[nrb++] = {vel, dvel, sizeof(double) * 3 * N};
+  if (phi_dot) rb[nrb++] = {phi_dot, s->phid.p, sizeof(double) * N};
+  return read_back(s->st, rb, nrb);
 }
 
 extern "C" femx_status femx_ins_get_system(femx_ins *s, int *row_ptr, int *col, double *val, double *rhs,

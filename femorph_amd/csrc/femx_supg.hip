@@ -1151,6 +1151,12 @@ __global__ void block_to_orig(int E, const int *perm, const double *src, double 
   if (i < E) dst[perm[i]] = src[i];
 }
 
+// Node states (x, y, z, 0) as [N][3]: 3 N values, one per thread.
+__global__ __launch_bounds__(256) void pack3(int N, const double *U, double *dst) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < 3L * N) dst[i] = U[i / 3 * 4 + i % 3];
+}
+
 }  // namespace
 
 }  // namespace femx
@@ -1369,10 +1375,12 @@ femx_status flush_pressure(femx_supg *s) {
   return FEMX_OK;
 }
 
-femx_status check_bc_err(femx_supg *s) {
+// Reads the pieces back together with the BC error flag.
+femx_status read_checked(femx_supg *s, ReadPiece *p, int n) {
   int e = 0;
-  FEMX_HIP(hipMemcpyAsync(&e, s->bc.err.p, sizeof(int), hipMemcpyDeviceToHost, s->st));
-  FEMX_HIP(hipStreamSynchronize(s->st));
+  p[n] = {&e, s->bc.err.p, sizeof(int)};
+  const femx_status r = read_back(s->st, p, n + 1);
+  if (r != FEMX_OK) return r;
   if (e) return set_error("Could not find time in femUtils::interpTableData."), FEMX_ERR_BC;
   return FEMX_OK;
 }
@@ -1471,9 +1479,8 @@ extern "C" femx_status femx_supg_set_state(femx_supg *s, const double *sol) {
   FEMX_HIP(hipMemsetAsync(s->Fprev.p, 0, m.N * sizeof(double4), s->st));
   FEMX_HIP(hipMemsetAsync(s->row.p, 0, (D_ROW + 1) * sizeof(double), s->st));
   s->press_pending = true;
-  femx_status r = check_bc_err(s);
-  FEMX_HIP(hipStreamSynchronize(s->st));
-  return r;
+  ReadPiece none[1];
+  return read_checked(s, none, 0);
 }
 
 namespace {
@@ -1514,8 +1521,8 @@ femx_status supg_finish(femx_supg *s, int *steps_done) {
   s->pend_n = 0;
   if (steps_done) *steps_done = 0;
   int halt = INT_MAX;
-  FEMX_HIP(hipMemcpyAsync(&halt, s->halt.p, sizeof(int), hipMemcpyDeviceToHost, s->st));
-  femx_status r = check_bc_err(s);
+  ReadPiece rb[2] = {{&halt, s->halt.p, sizeof(int)}};
+  femx_status r = read_checked(s, rb, 1);
   if (r != FEMX_OK) return r;
   if (halt != INT_MAX) {
     const long stop = halt;
@@ -1584,28 +1591,32 @@ extern "C" femx_status femx_supg_get_state(femx_supg *s, double *sol, double *pr
   }
   femx_status r = flush_pressure(s);
   if (r != FEMX_OK) return r;
+  // what is asked for, in the caller's layouts, in one staging array kept by
+  // the handle: [N][3] then E values per element field
+  size_t len = 0, off = 0;
+  for (double *o : {pres, lam, regime}) len += o ? m.E : 0;
+  len += sol ? 3 * (size_t)m.N : 0;
+  if (s->scratch.n < len && (r = s->scratch.alloc(len)) != FEMX_OK) return r;
+  ReadPiece rb[5];
+  int nrb = 0;
   if (sol) {
-    std::vector<double4> h(m.N);
-    FEMX_HIP(hipMemcpyAsync(h.data(), s->U[s->cur].p, m.N * sizeof(double4), hipMemcpyDeviceToHost, s->st));
-    FEMX_HIP(hipStreamSynchronize(s->st));
-    for (int n = 0; n < m.N; n++) {
-      sol[3L * n] = h[n].x;
-      sol[3L * n + 1] = h[n].y;
-      sol[3L * n + 2] = h[n].z;
-    }
+    pack3<<<grid_for(3L * m.N, 256), 256, 0, s->st>>>(m.N, reinterpret_cast<const double *>(s->U[s->cur].p),
+                                                      s->scratch.p);
+    FEMX_HIP(hipGetLastError());
+    rb[nrb++] = {sol, s->scratch.p, 3 * (size_t)m.N * sizeof(double)};
+    off = 3 * (size_t)m.N;
   }
   double *outs[3] = {pres, lam, regime};
   DevBuf<double> *srcs[3] = {&s->pres, &s->lam, &s->regime};
   for (int k = 0; k < 3; k++) {
     if (!outs[k]) continue;
-    if ((r = s->scratch.alloc(m.E)) != FEMX_OK) return r;
-    block_to_orig<<<grid_for(m.E, 256), 256, 0, s->st>>>(m.E, m.blk.d_perm.p, srcs[k]->p, s->scratch.p);
+    block_to_orig<<<grid_for(m.E, 256), 256, 0, s->st>>>(m.E, m.blk.d_perm.p, srcs[k]->p, s->scratch.p + off);
     FEMX_HIP(hipGetLastError());
-    FEMX_HIP(hipMemcpyAsync(outs[k], s->scratch.p, m.E * sizeof(double), hipMemcpyDeviceToHost, s->st));
-    FEMX_HIP(hipStreamSynchronize(s->st));
+    rb[nrb++] = {outs[k], s->scratch.p + off, m.E * sizeof(double)};
+    off += m.E;
   }
   if (time) *time = s->time;
-  return check_bc_err(s);
+  return read_checked(s, rb, nrb);
 }
 
 extern "C" femx_status femx_supg_get_mass(femx_supg *s, double *l_M) {

@@ -1430,12 +1430,19 @@ femx_status flush_projection(femx_vms *s) {
   return FEMX_OK;
 }
 
-femx_status check_err(femx_vms *s) {
+// Reads the pieces (with room for one more) back together with the BC error flag.
+femx_status read_checked(femx_vms *s, ReadPiece *p, int n) {
   int e = 0;
-  FEMX_HIP(hipMemcpyAsync(&e, s->bc.err.p, sizeof(int), hipMemcpyDeviceToHost, s->st));
-  FEMX_HIP(hipStreamSynchronize(s->st));
+  p[n] = {&e, s->bc.err.p, sizeof(int)};
+  const femx_status r = read_back(s->st, p, n + 1);
+  if (r != FEMX_OK) return r;
   if (e) return set_error("Could not find time in femUtils::interpTableData."), FEMX_ERR_BC;
   return FEMX_OK;
+}
+
+femx_status check_err(femx_vms *s) {
+  ReadPiece none[1];
+  return read_checked(s, none, 0);
 }
 
 }  // namespace
@@ -1612,7 +1619,7 @@ extern "C" femx_status femx_vms_set_state(femx_vms *s, const double *sol, const 
   const bool mixed = f32_elem(s->p.precision);
   if (sdus) {
     femx_status r;
-    if ((r = s->scratch.alloc(ns)) != FEMX_OK) return r;
+    if ((long)s->scratch.n < ns && (r = s->scratch.alloc(ns)) != FEMX_OK) return r;
     FEMX_HIP(hipMemcpyAsync(s->scratch.p, sdus, ns * sizeof(double), hipMemcpyHostToDevice, s->st));
     if (mixed)
       sdus_to_blocks<float><<<grid_for(ns, 256), 256, 0, s->st>>>(m.E, m.blk.d_perm.p, s->scratch.p, s->sdus32.p);
@@ -1653,19 +1660,21 @@ extern "C" femx_status femx_vms_get_state(femx_vms *s, double *sol, double *sdus
   Mesh &m = *s->mesh;
   femx_status r = flush_projection(s);
   if (r != FEMX_OK) return r;
-  if (sol) FEMX_HIP(hipMemcpyAsync(sol, s->Q[s->cur].p, m.N * sizeof(double4), hipMemcpyDeviceToHost, s->st));
+  ReadPiece rb[3];
+  int nrb = 0;
+  if (sol) rb[nrb++] = {sol, s->Q[s->cur].p, m.N * sizeof(double4)};
   if (sdus) {
     const long ns = 12L * m.E;
-    if ((r = s->scratch.alloc(ns)) != FEMX_OK) return r;
+    if ((long)s->scratch.n < ns && (r = s->scratch.alloc(ns)) != FEMX_OK) return r;
     if (f32_elem(s->p.precision))
       sdus_from_blocks<float><<<grid_for(ns, 256), 256, 0, s->st>>>(m.E, m.blk.d_perm.p, s->sdus32.p, s->scratch.p);
     else
       sdus_from_blocks<double><<<grid_for(ns, 256), 256, 0, s->st>>>(m.E, m.blk.d_perm.p, s->sdus64.p, s->scratch.p);
     FEMX_HIP(hipGetLastError());
-    FEMX_HIP(hipMemcpyAsync(sdus, s->scratch.p, ns * sizeof(double), hipMemcpyDeviceToHost, s->st));
+    rb[nrb++] = {sdus, s->scratch.p, ns * sizeof(double)};
   }
   if (time) *time = s->time;
-  return check_err(s);
+  return read_checked(s, rb, nrb);
 }
 
 extern "C" femx_status femx_vms_get_mass(femx_vms *s, double *nd_mass) {
@@ -2079,12 +2088,11 @@ extern "C" femx_status femx_vms_batch_get_state(femx_vms_batch *b, int i, double
   femx_vms *s = b->s;
   femx_status r = flush_projection(s);
   if (r != FEMX_OK) return r;
-  if (sol)
-    FEMX_HIP(hipMemcpyAsync(sol, s->Q[s->cur].p + s->h_node0[i], s->h_nnodes[i] * sizeof(double4),
-                            hipMemcpyDeviceToHost, s->st));
-  FEMX_HIP(hipStreamSynchronize(s->st));
+  ReadPiece rb[2];
+  int nrb = 0;
+  if (sol) rb[nrb++] = {sol, s->Q[s->cur].p + s->h_node0[i], s->h_nnodes[i] * sizeof(double4)};
   if (time) *time = s->h_time[i];
-  return check_err(s);
+  return read_checked(s, rb, nrb);
 }
 
 extern "C" femx_status femx_vms_batch_info(femx_vms_batch *b, long long *info) {

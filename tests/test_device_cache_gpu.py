@@ -80,3 +80,28 @@ def test_cached_buffers_give_the_same_results(gpu):
         assert gpu.device_cache_bytes(0) == 0
     finally:
         gpu.set_device_cache(CAP)
+
+
+@pytest.mark.parametrize("n", [3, 43, 44, 90])
+def test_read_back_round_trips(gpu, n):
+    """States of one pinned chunk (2 MiB) or less, just above, and of many
+    chunks (several host threads) come back exactly as they were set."""
+    m = meshgen.hex_cube(n, 0.0)
+    rng = np.random.default_rng(n)
+    dm = gpu.DeviceMesh(m)
+    sol = rng.normal(size=(m.n_nodes, 3))
+    print("round trip of", m.n_nodes, "nodes", flush=True)
+    g = gpu.SUPGSolver(dm, meshgen.BoundaryConditions(), rho=1.0, mu=0.01, alpha=1.0, cI=4.0, dt=0.1 / n)
+    g.set_state(sol)
+    for _ in range(2):  # the second read takes its chunks from the pool
+        st = g.get_state()
+        np.testing.assert_array_equal(st["sol"], sol)
+        assert not st["pres"].any() and not st["lam"].any() and not st["regime"].any()
+    phi, phid, vel = rng.normal(size=m.n_nodes), rng.normal(size=m.n_nodes), rng.normal(size=(m.n_nodes, 3))
+    s = gpu.INSSolver(dm, dt=0.1, alpha_m=0.8, alpha_f=0.6, gamma=0.7)
+    s.set_state(phi, phid, vel)
+    for got, want in zip(s.get_state(), (phi, phid, vel)):
+        np.testing.assert_array_equal(got, want)
+    gpu.set_device_cache(0)  # gives the idle chunks back
+    gpu.set_device_cache(CAP)
+    np.testing.assert_array_equal(g.get_state()["sol"], sol)
