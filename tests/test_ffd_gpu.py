@@ -39,6 +39,24 @@ def test_morph_matches_oracle(gpu, box):
     assert c.shape == (tot, 3) and np.abs(d).sum() > 0
 
 
+@pytest.mark.parametrize("nx", range(2, 14))
+def test_morph_every_x_count(gpu, nx):
+    """Every number of control points along x (a kernel each), on odd point
+    counts, with the box's corners, faces and the points just outside them.
+    1e-13 of the largest displacement: the factored sum rounds per axis, at
+    most 3 x 13 roundings of terms no larger than it."""
+    n = (nx, 2 + nx % 5, 13 - nx % 4)
+    rng = np.random.default_rng(nx)
+    nodes = rng.choice(n[0] * n[1] * n[2], size=7, replace=False)
+    vals = rng.uniform(-0.2, 0.2, (len(nodes), 3))
+    edge = np.array(np.meshgrid(*[[-1e-9, 0.0, 0.5, 1.0, 1.0 + 1e-9]] * 3)).reshape(3, -1).T
+    pts = np.vstack([edge, rng.uniform(0.0, 1.0, (257, 3))])
+    box = ((0.0, 0.0, 0.0), n, (1.0, 0, 0), (0, 1.0, 0), (0, 0, 1.0))
+    got = gpu.ffd_morph(*box, nodes, vals, pts)
+    ref = oracle.ffd_morph(*box, nodes, vals, pts)
+    assert np.abs(got - ref).max() <= 1e-13
+
+
 def test_ffd_driver_end_to_end(gpu, tmp_path):
     """mesh.vtk (tet4) + command file -> morphed VTK whose DXYZ is the
     morph of every node, and one bernsteinGrid_<k>.vtk per box; the model
