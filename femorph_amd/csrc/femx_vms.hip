@@ -423,6 +423,7 @@ struct BlockArgs {
   const double4 *rows;
   int *err;
   double *bmax;  // [nblk] per-block max of the pre-BC |u|^2
+  int want_max;  // it is read: the last iteration of a call, every one with diagnostics
   // element diagnostics (eval_centroid_*, :699-724), NULL when off:
   const int *perm;   // block order -> original element id
   // [4E] T4: per block, each node's running sum of the block's contributions
@@ -840,7 +841,7 @@ __device__ __forceinline__ void vms_block_run(const BlockArgs<T> &a, const int b
     T4 *img = static_cast<T4 *>(a.diag_img) + 4L * e0;
     for (int q = tid; q < 4 * ne; q += VB) st_stream(img + q, sres[q]);
   }
-  block_max_store<VB>(m2, a.bmax, row);
+  if (a.want_max) block_max_store<VB>(m2, a.bmax, row);
 }
 
 // occupancy (waves per SIMD): FP32 element math 5 (4 with dual iterations), FP64 2
@@ -878,6 +879,7 @@ struct FixArgs {
   const double4 *rows;
   int *err;
   double *bmax;  // [grid] per-block max of the pre-BC |u|^2
+  int want_max;  // as BlockArgs
   const int *node_mesh;  // batches: mesh of every node (NULL for one mesh)
   const VmsConst *kt;
   VmsConst k;
@@ -957,7 +959,7 @@ __device__ __forceinline__ void vms_fixup_run(const FixArgs &a, const int s, con
     if (rec >= 0) a.Prn[rec] = pre;
     a.Qn[g] = post;
   }
-  block_max_store<256>(m2, bmax_row, 0);
+  if (a.want_max) block_max_store<256>(m2, bmax_row, 0);
 }
 
 template <typename T>
@@ -1206,6 +1208,10 @@ struct femx_vms {
   DevBuf<float> sdus32;
   DevBuf<double> bmax;  // per-block maxima of the last iteration: block kernel, then fix-up
   int n_bmax = 0;
+  // the iteration being launched writes its maxima (a call's last one, every
+  // one with diagnostics): the wave and block reductions end each workgroup,
+  // and nothing reads the other iterations' values
+  int want_max = 1;
   DevBuf<double> scratch;  // staging of reference-layout arrays
   DevBuf<int> rec_node;
   // block records of the block kernel (the BC flags depend on the handle)
@@ -1309,6 +1315,7 @@ BlockArgs<T> block_args(femx_vms *s, bool first_dual, double t, T *sdus) {
   a.rows = s->bc.rows.p;
   a.err = s->bc.err.p;
   a.bmax = s->bmax.p;
+  a.want_max = s->want_max;
   a.perm = b.d_perm.p;
   a.diag_img = s->diag ? s->diag_img.p : nullptr;
   a.diag_sdu = s->diag == 1 ? s->diag_sdu.p : nullptr;
@@ -1372,6 +1379,7 @@ FixArgs fix_args(femx_vms *s, bool first_dual, double t) {
   a.rows = s->bc.rows.p;
   a.err = s->bc.err.p;
   a.bmax = s->bmax.p + b.nb;
+  a.want_max = s->want_max;
   a.node_mesh = s->batch ? s->node_mesh.p : nullptr;
   a.kt = s->batch ? s->kt.p : nullptr;
   a.k = vms_const(s, t);
@@ -1641,6 +1649,7 @@ extern "C" femx_status femx_vms_step(femx_vms *s, int nsteps) {
   for (int k = 0; k < nsteps; k++) {
     s->time += s->p.dt;  // currentTime += timeStep (:1028)
     for (int d = 0; d <= s->p.tot_dual_steps; d++) {
+      s->want_max = s->diag || (k == nsteps - 1 && d == s->p.tot_dual_steps);
       femx_status r = launch_block(s, s->proj_pending, true, d > 0, d == 0, s->time);
       if (r != FEMX_OK) return r;
       if ((r = launch_fixup(s, d == 0, s->time)) != FEMX_OK) return r;
@@ -1870,6 +1879,7 @@ __global__ void vms_batch_tick(int n, VmsConst *kt, const double *dt) {
 femx_status batch_step_once(femx_vms *s) {
   vms_batch_tick<<<grid_for(s->n_mesh, 256), 256, 0, s->st>>>(s->n_mesh, s->kt.p, s->kdt.p);
   FEMX_HIP(hipGetLastError());
+  s->want_max = 0;  // batches have no reader of the maxima
   for (int d = 0; d <= s->p.tot_dual_steps; d++) {
     femx_status r = launch_block(s, s->proj_pending, true, d > 0, d == 0, 0.0);
     if (r != FEMX_OK) return r;
@@ -2207,7 +2217,7 @@ __device__ __forceinline__ int member_of(const int *off, int nm, int g) {
 
 __global__ __launch_bounds__(VB, VMS_BLOCK_WAVES(float, false)) void vms_block_union(const VmsMember *mem,
                                                                                       const int *blk_off, int nm,
-                                                                                      int ntot) {
+                                                                                      int ntot, int last) {
   const int g = xcd_block(blockIdx.x, ntot);
   const int h = member_of(blk_off, nm, g);
   const VmsMember &me = mem[h];
@@ -2222,12 +2232,13 @@ __global__ __launch_bounds__(VB, VMS_BLOCK_WAVES(float, false)) void vms_block_u
   a.Pr = me.Prb[par];
   a.Prn = me.Prb[par ^ 1];
   a.k.t = uni(dyn->t) + me.dt;  // currentTime += timeStep (:1028)
+  a.want_max = last || left == 1;
   args_to_global(a);
   const int blk = g - uni(blk_off[h]);
   vms_block_run<float, double, true, true, false, false>(a, blk, blk);
 }
 
-__global__ __launch_bounds__(256) void vms_fixup_union(const VmsMember *mem, const int *fx_off, int nm) {
+__global__ __launch_bounds__(256) void vms_fixup_union(const VmsMember *mem, const int *fx_off, int nm, int last) {
   const int g = blockIdx.x;
   const int h = member_of(fx_off, nm, g);
   const VmsMember &me = mem[h];
@@ -2242,6 +2253,7 @@ __global__ __launch_bounds__(256) void vms_fixup_union(const VmsMember *mem, con
   a.Pr = me.Prb[par];
   a.Prn = me.Prb[par ^ 1];
   a.k.t = uni(dyn->t) + me.dt;
+  a.want_max = last || left == 1;
   args_to_global(a);
   const int wg = g - uni(fx_off[h]);
   vms_fixup_run<double>(a, wg * 256 + (int)threadIdx.x, wg);
@@ -2403,8 +2415,9 @@ extern "C" femx_status femx_vms_union_step(femx_vms_union *u, int k) {
   if (nm == 0 || k == 0) return FEMX_OK;
   const int *blk_off = u->off.p, *fx_off = u->off.p + nm + 1;
   for (int i = 0; i < k; i++) {
-    if (u->nblk > 0) vms_block_union<<<u->nblk, VB, 0, u->st>>>(u->tab.p, blk_off, nm, u->nblk);
-    if (u->nfx > 0) vms_fixup_union<<<u->nfx, 256, 0, u->st>>>(u->tab.p, fx_off, nm);
+    const int last = i == k - 1;
+    if (u->nblk > 0) vms_block_union<<<u->nblk, VB, 0, u->st>>>(u->tab.p, blk_off, nm, u->nblk, last);
+    if (u->nfx > 0) vms_fixup_union<<<u->nfx, 256, 0, u->st>>>(u->tab.p, fx_off, nm, last);
     vms_union_tick<<<grid_for(nm, 64), 64, 0, u->st>>>(u->tab.p, nm);
   }
   FEMX_HIP(hipGetLastError());

@@ -294,6 +294,32 @@ def test_high_valence_node(gpu, precision, tol):
         assert rel_l2(sol, o.get("sol_n")) <= tol, (step, rel_l2(sol, o.get("sol_n")))
 
 
+@pytest.mark.parametrize("precision,tot_dual", [(0, 0), (1, 0), (1, 2), (2, 0)])
+def test_maxima_of_a_calls_last_iteration(gpu, precision, tot_dual):
+    """max |u| and the CFL number are those of the last dual iteration, also
+    when it is the last of many in one call (the others write no maxima), and
+    those of a union member's last step."""
+    m, bc, params, ic = _case("channel", 9, 0.15, seed=6)
+    dm = gpu.DeviceMesh(m)
+    a, b, c = (gpu.VMSSolver(dm, bc, precision=precision, tot_dual_steps=tot_dual, **params) for _ in range(3))
+    for g in (a, b, c):
+        g.set_state(ic)
+    got = []
+    for _ in range(4):
+        a.step(1)
+        got.append(a.get_cfl())
+    assert len(set(got)) == 4
+    b.step(4)
+    assert b.get_cfl() == got[3]
+    if precision == 1 and tot_dual == 0:
+        c.step(1)
+        u = gpu.VMSUnion()
+        u.add(c, 2)
+        u.step(5)  # its last step is not the call's
+        u.remove(c)
+        assert c.get_cfl() == got[2]
+
+
 @pytest.mark.parametrize("precision,tol", [(0, TOL64), (1, 1e-5), (2, 1e-5)])
 def test_node_of_no_element(gpu, precision, tol):
     """A node that no element uses: the update divides its zero residual by
