@@ -3,17 +3,26 @@
 // generalized-alpha update (:471-485), on gfx950.
 //
 // One stage per femx_ins_advdiff_solve call, all on the handle's stream:
-//   ins_element     one thread per element: the element matrix and vector of
-//                   formTransientAdvDiffLHS / formTransientAdvDiffRHS
-//                   (src/femElement.cpp:1471-1689) in FP64, scattered straight
-//                   into the order the gathers read (cpos / rpos maps)
+//   tet4, ins_rows_tet4: eight lanes per matrix row; each forms its share of
+//                   the row's elements' contributions (their row of the element
+//                   matrix and vector of formTransientAdvDiffLHS /
+//                   formTransientAdvDiffRHS, src/femElement.cpp:1471-1689, in
+//                   FP64), sums them in LDS, then the Dirichlet row
+//                   (applyDirichelet, src/femMatrix.cpp:183-205), the Jacobi
+//                   inverse and the start of the Krylov solve (x = 0, r = b,
+//                   z = D^-1 b, ||b||^2)
+//   hexa8           (an element has 8 rows and costs 20 times a tet: it is
+//                   formed once)
+//   ins_element     one thread per element: the element matrix and vector,
+//                   scattered straight into the order the gathers read (cpos /
+//                   rpos maps)
 //   ins_gather_mat  one thread per CSR entry: its contiguous run of element
 //                   values, ascending element (the order femSparseMatrix::
 //                   assemble adds them, src/femMatrix.cpp:129-160), then the
-//                   Dirichlet row (applyDirichelet :183-205), Jacobi inverse
+//                   Dirichlet row, Jacobi inverse
 //   ins_gather_rhs  one thread per node: the same for the element vectors
 //                   (femDenseVector::assemble), Dirichlet value, and the start
-//                   of the Krylov solve (x = 0, r = b, z = D^-1 b, ||b||^2)
+//                   of the Krylov solve
 //   GMRES           restarted, right Jacobi preconditioning, classical
 //                   Gram-Schmidt applied twice, zero initial guess; per
 //                   iteration a vector-CSR SpMV of z = D^-1 v, three
@@ -30,6 +39,7 @@
 //                                     + alphaF dt (1-gamma) u.grad phid  (:1641-1687)
 // which equals the reference's sums up to rounding.
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -264,6 +274,167 @@ __global__ __launch_bounds__(256) void ins_element(int E, const int *conn, const
   const int *rq = rpos + (long)e * NPE;
 #pragma unroll
   for (int b = 0; b < NPE; b++) erhs[rq[b]] = R[b];
+}
+
+// ---------------------------------------------------------- tet4 rows
+// A tet4's matrix row is cheap to form (constant Jacobian: about 400
+// instructions), and forming it again for each of its four rows costs less
+// than passing the element matrices through memory: the element kernel and
+// the two gathers moved 2.9 GB per assembly at 5.3M tets (106M scattered
+// 8-byte writes among them), 1.03 ms; this kernel gathers the node records
+// from the caches and writes the matrix, 0.60 ms (193k rows: 230 -> 112 us; half
+// the issue slots are used, the L1 lookups of the gathers two thirds of the
+// time).  Eight lanes per row: a row has about 24 elements, and the lanes of a
+// row read neighbouring records.
+constexpr int RLPR = 8;             // lanes per row
+constexpr int RROWS = 256 / RLPR;   // rows per workgroup pass
+constexpr int RCAP = 24;            // row entries summed in LDS per pass over the row's elements
+constexpr int RGRID = 3072;         // workgroups at most (each takes a contiguous range of rows)
+
+// The contributions of one element to the row of its corner a: v[b] += P_a Q_b,
+// R -= P_a R (the sums over the Gauss points of the header).
+__device__ __forceinline__ void tet4_row(const double4 X[4], const double4 V[4], int a, double iso2,
+                                         const InsConst &k, double v[4], double &R) {
+  double J[3][3], iJ[3][3], detJ;
+#pragma unroll
+  for (int r = 0; r < 3; r++) {
+    J[r][0] = X[r].x - X[3].x;
+    J[r][1] = X[r].y - X[3].y;
+    J[r][2] = X[r].z - X[3].z;
+  }
+  inv3(J, iJ, detJ);
+  // |G|^2 of evalGeometricMatrix: G[i][j] = sum_c invJ[c][i] invJ[c][j]
+  double t2 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    const int j = (i + 1) % 3;
+    const double d = iJ[0][i] * iJ[0][i] + iJ[1][i] * iJ[1][i] + iJ[2][i] * iJ[2][i];
+    const double o = iJ[0][i] * iJ[0][j] + iJ[1][i] * iJ[1][j] + iJ[2][i] * iJ[2][j];
+    t2 += d * d + 2.0 * (o * o);
+  }
+  const double tb = k.timeTau + t2 * iso2, wd = detJ * Shape<4>::W();
+  // the rule's values: N_b(g) = nb + nd (g == b)
+  const double nb = Shape<4>::N(0, 1), nd = Shape<4>::N(0, 0) - nb;
+  const double us[3] = {nb * ((V[0].x + V[1].x) + (V[2].x + V[3].x)), nb * ((V[0].y + V[1].y) + (V[2].y + V[3].y)),
+                        nb * ((V[0].z + V[1].z) + (V[2].z + V[3].z))};
+  const double ps = nb * ((X[0].w + X[1].w) + (X[2].w + X[3].w));
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    const double u[3] = {us[0] + nd * V[g].x, us[1] + nd * V[g].y, us[2] + nd * V[g].z};
+    // evalQuadraticTau (src/femElement.cpp:237-268), c = 1: u^T G u = |invJ u|^2
+    double t1 = 0.0, ad[4];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const double w = iJ[c][0] * u[0] + iJ[c][1] * u[1] + iJ[c][2] * u[2];
+      t1 += w * w;
+      ad[c] = iJ[0][c] * u[0] + iJ[1][c] * u[1] + iJ[2][c] * u[2];  // u.grad N_c
+    }
+    ad[3] = -(ad[0] + ad[1] + ad[2]);
+    const double tau = rsqrt(tb + t1);
+    double up = 0.0, ud = 0.0;  // u.grad phi, u.grad phid
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      up += ad[b] * V[b].w;
+      ud += ad[b] * X[b].w;
+    }
+    const double Rg = k.om * (ps + nd * X[g].w) + up + k.afdt1g * ud;
+    const double aa = a == 0 ? ad[0] : a == 1 ? ad[1] : a == 2 ? ad[2] : ad[3];
+    const double P = ((a == g ? nb + nd : nb) + tau * aa) * wd;
+    R -= P * Rg;
+#pragma unroll
+    for (int b = 0; b < 4; b++) v[b] += P * (k.am * (b == g ? nb + nd : nb) + k.afdtg * ad[b]);
+  }
+}
+
+// p[i] by a 32-bit byte offset (arrays below 4 GiB): one VGPR of address, not two.
+__device__ __forceinline__ double4 at32(const double4 *p, int i) {
+  return *reinterpret_cast<const double4 *>(reinterpret_cast<const char *>(p) + ((unsigned)i << 5));
+}
+
+// node: x y z and phid; vphi: velocity and phi.  Rows in the order rord
+// (along the mesh's Morton curve), row r's corners g_slot[g_off[r] ...) in
+// ascending element, cpos their element's columns' places in the row.
+__global__ __launch_bounds__(256, 3) void ins_rows_tet4(int N, const int *rord, const int *g_off, const int *g_slot,
+                                                     const ushort4 *cpos, const int4 *conn, const double4 *node,
+                                                     const double4 *vphi, const double *iso, InsConst k,
+                                                     const int *row_ptr, const int *col, const int *dir_flag,
+                                                     const double *dir_v, double *val, double *dinv, double *b,
+                                                     double *x, double *rvec, double *z, double *part) {
+  // the thread's sums of the row's entries: column tid of acc
+  __shared__ double acc[RCAP * 256];
+  const int tid = threadIdx.x, lane = tid & (RLPR - 1);
+  const int ngroups = (N + RROWS - 1) / RROWS, per = (ngroups + gridDim.x - 1) / gridDim.x;
+  const int first = xcd_block(blockIdx.x, gridDim.x) * per, last = min(ngroups, first + per);
+  double nrm[1] = {0.0};
+  for (int grp = first; grp < last; grp++) {
+    const int i = grp * RROWS + tid / RLPR;
+    if (i >= N) continue;
+    const int r = rord[i], q0 = row_ptr[r], len = row_ptr[r + 1] - q0, j1 = g_off[r + 1];
+    const bool fixed = dir_flag[r] != 0;
+    double R = 0.0, di = 0.0;
+    for (int c0 = 0; c0 < len; c0 += RCAP) {
+      const int n = min(RCAP, len - c0);
+      for (int q = 0; q < n; q++) acc[q * 256 + tid] = 0.0;
+      if (!fixed) {
+        // the next element's corner and connectivity are loaded while the
+        // current one is formed
+        int j = g_off[r] + lane, slot = 0;
+        int4 c = make_int4(0, 0, 0, 0);
+        if (j < j1) {
+          slot = g_slot[j];
+          c = conn[slot >> 2];
+        }
+        for (; j < j1; j += RLPR) {
+          const double4 X[4] = {at32(node, c.x), at32(node, c.y), at32(node, c.z), at32(node, c.w)};
+          const double4 V[4] = {at32(vphi, c.x), at32(vphi, c.y), at32(vphi, c.z), at32(vphi, c.w)};
+          const double d0 = iso[slot >> 2];
+          const ushort4 p0 = cpos[j];
+          const int a = slot & 3;
+          if (j + RLPR < j1) {
+            slot = g_slot[j + RLPR];
+            c = conn[slot >> 2];
+          }
+          double v[4] = {0.0, 0.0, 0.0, 0.0}, Rj = 0.0;
+          tet4_row(X, V, a, d0 * d0, k, v, Rj);
+          if (c0 == 0) R += Rj;
+          const int p[4] = {p0.x - c0, p0.y - c0, p0.z - c0, p0.w - c0};
+#pragma unroll
+          for (int s = 0; s < 4; s++)
+            if (p[s] >= 0 && p[s] < n) acc[p[s] * 256 + tid] += v[s];
+        }
+      }
+      // the row's lanes are one wave's: its LDS accesses stay in order
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int q = lane; q < n; q += RLPR) {
+        const double *t = acc + q * 256 + (tid & ~(RLPR - 1));
+        double s = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+        const bool dg = col[q0 + c0 + q] == r;
+        if (fixed) s = dg ? 1.0 : 0.0;
+        val[q0 + c0 + q] = s;
+        if (dg) di = s != 0.0 ? 1.0 / s : 1.0;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+#pragma unroll
+    for (int off = RLPR / 2; off > 0; off >>= 1) {
+      R += __shfl_xor(R, off);
+      di += __shfl_xor(di, off);  // one lane holds the diagonal's
+    }
+    if (lane == 0) {
+      const double s = fixed ? dir_v[r] : R;
+      dinv[r] = di;
+      b[r] = s;
+      x[r] = 0.0;
+      rvec[r] = s;
+      z[r] = di * s;
+      nrm[0] += s * s;
+    }
+  }
+  block_store<1>(nrm, 1, part, gridDim.x);
 }
 
 // ------------------------------------------------- reduction finishers
@@ -522,7 +693,7 @@ __global__ __launch_bounds__(64) void gm_givens(const double *part, int nb, Gmre
 // ------------------------------------------------------------- update
 // solve() :471-485 on node dof 4.
 __global__ __launch_bounds__(256) void ins_update(int N, double dt, double gm, double4 *vphi, double *phid,
-                                                  const double *x) {
+                                                  double *node, const double *x) {
   const int a = blockIdx.x * blockDim.x + threadIdx.x;
   if (a >= N) return;
   double4 v = vphi[a];
@@ -530,6 +701,13 @@ __global__ __launch_bounds__(256) void ins_update(int N, double dt, double gm, d
   v.w = v.w + dt * pd + gm * dt * (pn - pd);
   vphi[a] = v;
   phid[a] = pn;
+  if (node) node[4L * a + 3] = pn;
+}
+
+// phid of the node records (x y z phid).
+__global__ __launch_bounds__(256) void ins_node_phid(int N, const double *phid, double *node) {
+  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a < N) node[4L * a + 3] = phid[a];
 }
 
 }  // namespace
@@ -549,7 +727,12 @@ struct femx_ins {
   int lpr = 4;      // lanes per row of the CSR kernels
   DevBuf<double> phid, iso, emat, erhs, val, b, dinv, x, rvec, z, w[2], V, part, dir_v, stage;
   DevBuf<int> row_ptr, col, nz_row, c_ptr, cpos, rpos, dir_flag;
-  DevBuf<int> econn;  // connectivity in the element kernel's processing order
+  DevBuf<int> econn;  // connectivity in the element kernel's processing order (hexa8)
+  // tet4: node records (x y z phid), row order and the places of the
+  // elements' columns in the rows
+  DevBuf<double4> node;
+  DevBuf<int> rord;
+  DevBuf<ushort4> rcpos;
   DevBuf<GmresState> gst;
   GmresCtl *ctl = nullptr;  // pinned host copy of the control words
   bool have_solution = false;
@@ -659,6 +842,47 @@ void host_pattern(const Mesh &m, const std::vector<int> &n_off, const std::vecto
   });
 }
 
+// The same pattern for ins_rows_tet4, and per corner (in the order of n_slot:
+// by node, ascending element) the places of its element's four nodes in the
+// node's row.  False if a row is too long for 16-bit places.
+bool host_rows(const Mesh &m, const std::vector<int> &n_off, const std::vector<int> &n_slot,
+               std::vector<int> &row_ptr, std::vector<int> &col, std::vector<ushort4> &cpos) {
+  const int N = m.N;
+  const int *conn = m.h_conn.data();
+  constexpr int CH = 4096;  // nodes per work item
+  const long items = (N + CH - 1) / CH;
+  std::vector<std::vector<int>> cols(items);
+  std::atomic<bool> ok{true};
+  row_ptr.assign(N + 1, 0);
+  cpos.resize(n_slot.size());
+  parallel_items(items, [&](long c) {
+    std::vector<int> buf;
+    for (int r = (int)(c * CH); r < std::min<long>(N, (c + 1) * CH); r++) {
+      buf.assign(1, r);
+      for (int j = n_off[r]; j < n_off[r + 1]; j++) {
+        const int *q = conn + (n_slot[j] & ~3);
+        buf.insert(buf.end(), q, q + 4);
+      }
+      std::sort(buf.begin(), buf.end());
+      buf.erase(std::unique(buf.begin(), buf.end()), buf.end());
+      if (buf.size() > 65536) ok = false;
+      row_ptr[r + 1] = (int)buf.size();
+      cols[c].insert(cols[c].end(), buf.begin(), buf.end());
+      for (int j = n_off[r]; j < n_off[r + 1]; j++) {
+        unsigned short p[4];
+        for (int b = 0; b < 4; b++)
+          p[b] = (unsigned short)(std::lower_bound(buf.begin(), buf.end(), conn[(n_slot[j] & ~3) + b]) - buf.begin());
+        cpos[j] = make_ushort4(p[0], p[1], p[2], p[3]);
+      }
+    }
+  }, n_slot.size() >= (1u << 16));
+  for (int r = 0; r < N; r++) row_ptr[r + 1] += row_ptr[r];
+  col.resize(row_ptr[N]);
+  parallel_items(items, [&](long c) { std::copy(cols[c].begin(), cols[c].end(), col.begin() + row_ptr[c * CH]); },
+                 col.size() >= (1u << 16));
+  return ok;
+}
+
 InsConst ins_const(const femx_ins_params &p) {
   InsConst k;
   k.am = p.alpha_m;
@@ -724,28 +948,37 @@ femx_status ins_solve(femx_ins *s, femx_ins_stats *stats) {
   Mesh &m = *s->mesh;
   const int N = m.N, nb = s->nb, M = s->p.restart;
   const InsConst k = ins_const(s->p);
-  {
-    TimedLaunch tl(s->timer, s->timer.kind("ins_element", element_bytes(m)), s->st);
-    if (m.npe == 8)
-      ins_element<8><<<grid_for(m.E, 256), 256, 0, s->st>>>(m.E, s->econn.p, m.xyz.p, s->vphi.p, s->phid.p,
-                                                            s->iso.p, k, s->cpos.p, s->rpos.p, s->emat.p, s->erhs.p);
-    else
-      ins_element<4><<<grid_for(m.E, 256), 256, 0, s->st>>>(m.E, s->econn.p, m.xyz.p, s->vphi.p, s->phid.p,
-                                                            s->iso.p, k, s->cpos.p, s->rpos.p, s->emat.p, s->erhs.p);
-  }
-  {
+  int nb0;  // partial sums of ||b||^2
+  if (s->node.p) {
+    // the mesh and the node records once, the row places of every corner,
+    // the matrix and the solve's start written
+    const double bytes = m.E * (16.0 + 8.0 + 4.0 * 12.0) + s->nnz * 12.0 + N * (64.0 + 16.0 + 5.0 * 8.0);
+    TimedLaunch tl(s->timer, s->timer.kind("ins_rows", bytes), s->st);
+    nb0 = std::min(RGRID, grid_for(N, RROWS));
+    ins_rows_tet4<<<nb0, 256, 0, s->st>>>(N, s->rord.p, m.g_off.p, m.g_slot.p, s->rcpos.p,
+                                          reinterpret_cast<const int4 *>(m.conn.p), s->node.p, s->vphi.p, s->iso.p, k,
+                                          s->row_ptr.p, s->col.p, s->dir_flag.p, s->dir_v.p, s->val.p, s->dinv.p,
+                                          s->b.p, s->x.p, s->rvec.p, s->z.p, s->part.p);
+  } else {
+    {
+      TimedLaunch tl(s->timer, s->timer.kind("ins_element", element_bytes(m)), s->st);
+      const auto el = m.npe == 8 ? ins_element<8> : ins_element<4>;
+      el<<<grid_for(m.E, 256), 256, 0, s->st>>>(m.E, s->econn.p, m.xyz.p, s->vphi.p, s->phid.p, s->iso.p, k, s->cpos.p,
+                                                s->rpos.p, s->emat.p, s->erhs.p);
+    }
     const double bytes = s->nnz * (4.0 + 4.0 + 4.0 + 8.0) + (double)m.E * m.npe * m.npe * 8.0 + N * 12.0;
-    TimedLaunch tl(s->timer, s->timer.kind("ins_gather_mat", bytes), s->st);
-    ins_gather_mat<<<grid_for(s->nnz, RT), RT, 0, s->st>>>(s->nnz, s->c_ptr.p, s->emat.p, s->nz_row.p, s->col.p,
-                                                           s->dir_flag.p, s->val.p, s->dinv.p);
+    {
+      TimedLaunch tl(s->timer, s->timer.kind("ins_gather_mat", bytes), s->st);
+      ins_gather_mat<<<grid_for(s->nnz, RT), RT, 0, s->st>>>(s->nnz, s->c_ptr.p, s->emat.p, s->nz_row.p, s->col.p,
+                                                             s->dir_flag.p, s->val.p, s->dinv.p);
+    }
+    nb0 = grid_for(N, RT);
+    const double rbytes = (double)m.E * m.npe * 8.0 + N * (4.0 + 4.0 + 8.0 + 8.0 + 8.0 * 4);
+    TimedLaunch tl(s->timer, s->timer.kind("ins_gather_rhs", rbytes), s->st);
+    ins_gather_rhs<<<nb0, RT, 0, s->st>>>(N, m.g_off.p, s->erhs.p, s->dir_flag.p, s->dir_v.p, s->dinv.p, s->b.p,
+                                          s->x.p, s->rvec.p, s->z.p, s->part.p);
   }
-  {
-    const double bytes = (double)m.E * m.npe * 8.0 + N * (4.0 + 4.0 + 8.0 + 8.0 + 8.0 * 4);
-    TimedLaunch tl(s->timer, s->timer.kind("ins_gather_rhs", bytes), s->st);
-    ins_gather_rhs<<<grid_for(N, RT), RT, 0, s->st>>>(N, m.g_off.p, s->erhs.p, s->dir_flag.p, s->dir_v.p, s->dinv.p,
-                                                      s->b.p, s->x.p, s->rvec.p, s->z.p, s->part.p);
-  }
-  gm_start<<<1, 64, 0, s->st>>>(s->part.p, grid_for(N, RT), s->gst.p, 1);
+  gm_start<<<1, 64, 0, s->st>>>(s->part.p, nb0, s->gst.p, 1);
   femx_status r;
   const double spmv_bytes = s->nnz * 12.0 + N * (4.0 + 8.0 * 4);
   // host checks of the cycle flag: first where the previous solve stopped,
@@ -851,35 +1084,57 @@ extern "C" femx_status femx_ins_create(femx_mesh *mesh, const double *el_diff, i
     std::vector<int> at(n_off.begin(), n_off.end() - 1);
     for (long q = 0; q < (long)E * npe; q++) n_slot[at[m.h_conn[q]]++] = (int)q;
   }
-  std::vector<int> nz_row, c_ptr, c_idx;
-  host_pattern(m, n_off, n_slot, s->h_row_ptr, s->h_col, nz_row, c_ptr, c_idx);
-  s->nnz = s->h_row_ptr[N];
-  // where each element value goes: matrix entry contributions and node
-  // contributions in the gathers' (ascending element) order
-  std::vector<int> cpos(c_idx.size()), rpos((size_t)E * npe);
-  for (size_t q = 0; q < c_idx.size(); q++) cpos[c_idx[q]] = (int)q;
-  for (size_t j = 0; j < n_slot.size(); j++) rpos[n_slot[j]] = (int)j;
-  c_idx.clear();
-  c_idx.shrink_to_fit();
-  s->lpr = (double)s->nnz / N > 20.0 ? 8 : 4;
-  // the element kernel's inputs in processing order: the Morton block order
-  // of the mesh (element t is original element ord[t])
+  std::vector<int> nz_row, c_ptr, cpos_o, rpos_o, econn, rord;
+  std::vector<ushort4> rcpos;
+  std::vector<double> iso(E, 0.0);
   const std::vector<int> &ord = m.blk.perm;
   if ((long)ord.size() != E) return ins_fail(s, (set_error("femx_ins_create: mesh has no element order"), FEMX_ERR_ARG));
-  std::vector<double> iso(E, 0.0);
-  std::vector<int> econn((size_t)E * npe), cpos_o(cpos.size()), rpos_o(rpos.size());
-  for (int t = 0; t < E; t++) {
-    const int e = ord[t];
-    if (el_diff) {
-      const double *d = el_diff + 3L * e;
-      iso[t] = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+  // ins_rows_tet4 (node records below 4 GiB), else the element kernel and the gathers
+  const bool rows = npe == 4 && N < (1 << 27);
+  auto el_iso = [&](int e) {
+    if (!el_diff) return 0.0;
+    const double *d = el_diff + 3L * e;
+    return sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+  };
+  if (rows) {
+    if (!host_rows(m, n_off, n_slot, s->h_row_ptr, s->h_col, rcpos))
+      return ins_fail(s, (set_error("femx_ins_create: a matrix row has more than 65536 entries"), FEMX_ERR_ARG));
+    for (int e = 0; e < E; e++) iso[e] = el_iso(e);
+    // rows in the order their nodes first appear along the element blocks
+    rord.reserve(N);
+    std::vector<char> seen(N, 0);
+    for (int n : m.blk.loc_node)
+      if (!seen[n]) {
+        seen[n] = 1;
+        rord.push_back(n);
+      }
+    for (int n = 0; n < N; n++)
+      if (!seen[n]) rord.push_back(n);
+  } else {
+    std::vector<int> c_idx;
+    host_pattern(m, n_off, n_slot, s->h_row_ptr, s->h_col, nz_row, c_ptr, c_idx);
+    // where each element value goes: matrix entry contributions and node
+    // contributions in the gathers' (ascending element) order
+    std::vector<int> cpos(c_idx.size()), rpos((size_t)E * npe);
+    for (size_t q = 0; q < c_idx.size(); q++) cpos[c_idx[q]] = (int)q;
+    for (size_t j = 0; j < n_slot.size(); j++) rpos[n_slot[j]] = (int)j;
+    // the element kernel's inputs in processing order: the Morton block order
+    // of the mesh (element t is original element ord[t])
+    econn.resize((size_t)E * npe);
+    cpos_o.resize(cpos.size());
+    rpos_o.resize(rpos.size());
+    for (int t = 0; t < E; t++) {
+      const int e = ord[t];
+      iso[t] = el_iso(e);
+      for (int a = 0; a < npe; a++) {
+        econn[(size_t)t * npe + a] = m.h_conn[(size_t)e * npe + a];
+        rpos_o[(size_t)t * npe + a] = rpos[(size_t)e * npe + a];
+      }
+      for (int q = 0; q < npe * npe; q++) cpos_o[(size_t)t * npe * npe + q] = cpos[(size_t)e * npe * npe + q];
     }
-    for (int a = 0; a < npe; a++) {
-      econn[(size_t)t * npe + a] = m.h_conn[(size_t)e * npe + a];
-      rpos_o[(size_t)t * npe + a] = rpos[(size_t)e * npe + a];
-    }
-    for (int q = 0; q < npe * npe; q++) cpos_o[(size_t)t * npe * npe + q] = cpos[(size_t)e * npe * npe + q];
   }
+  s->nnz = s->h_row_ptr[N];
+  s->lpr = (double)s->nnz / N > 20.0 ? 8 : 4;
   std::vector<int> dflag(N, 0);
   std::vector<double> dv(N, 0.0);
   for (int i = 0; i < n_dir; i++) {
@@ -891,7 +1146,9 @@ extern "C" femx_status femx_ins_create(femx_mesh *mesh, const double *el_diff, i
   const int M = p->restart;
   if ((r = s->row_ptr.upload(s->h_row_ptr.data(), N + 1, s->st)) != FEMX_OK ||
       (r = s->col.upload(s->h_col.data(), s->nnz, s->st)) != FEMX_OK ||
-      (r = s->nz_row.upload(nz_row.data(), s->nnz, s->st)) != FEMX_OK ||
+      (r = s->nz_row.upload(nz_row.data(), nz_row.size(), s->st)) != FEMX_OK ||
+      (r = s->rord.upload(rord.data(), rord.size(), s->st)) != FEMX_OK ||
+      (r = s->rcpos.upload(rcpos.data(), rcpos.size(), s->st)) != FEMX_OK ||
       (r = s->c_ptr.upload(c_ptr.data(), c_ptr.size(), s->st)) != FEMX_OK ||
       (r = s->cpos.upload(cpos_o.data(), cpos_o.size(), s->st)) != FEMX_OK ||
       (r = s->rpos.upload(rpos_o.data(), rpos_o.size(), s->st)) != FEMX_OK ||
@@ -899,12 +1156,12 @@ extern "C" femx_status femx_ins_create(femx_mesh *mesh, const double *el_diff, i
       (r = s->iso.upload(iso.data(), E, s->st)) != FEMX_OK ||
       (r = s->dir_flag.upload(dflag.data(), N, s->st)) != FEMX_OK ||
       (r = s->dir_v.upload(dv.data(), N, s->st)) != FEMX_OK || (r = s->vphi.alloc(N)) != FEMX_OK ||
-      (r = s->phid.alloc(N)) != FEMX_OK || (r = s->emat.alloc((size_t)E * npe * npe)) != FEMX_OK ||
-      (r = s->erhs.alloc((size_t)E * npe)) != FEMX_OK || (r = s->val.alloc(s->nnz)) != FEMX_OK ||
+      (r = s->phid.alloc(N)) != FEMX_OK || (r = s->emat.alloc(rows ? 0 : (size_t)E * npe * npe)) != FEMX_OK ||
+      (r = s->erhs.alloc(rows ? 0 : (size_t)E * npe)) != FEMX_OK || (r = s->node.alloc(rows ? N : 0)) != FEMX_OK || (r = s->val.alloc(s->nnz)) != FEMX_OK ||
       (r = s->b.alloc(N)) != FEMX_OK || (r = s->dinv.alloc(N)) != FEMX_OK || (r = s->x.alloc(N)) != FEMX_OK ||
       (r = s->rvec.alloc(N)) != FEMX_OK || (r = s->w[0].alloc(N)) != FEMX_OK || (r = s->w[1].alloc(N)) != FEMX_OK ||
       (r = s->V.alloc((size_t)s->ldv * (M + 1))) != FEMX_OK ||
-      (r = s->part.alloc((size_t)MAXM * std::max(s->nb, grid_for(N, RT)))) != FEMX_OK || (r = s->stage.alloc((size_t)N * 3)) != FEMX_OK ||
+      (r = s->part.alloc((size_t)MAXM * std::max({s->nb, grid_for(N, RT), RGRID}))) != FEMX_OK || (r = s->stage.alloc((size_t)N * 3)) != FEMX_OK ||
       (r = s->gst.alloc(1)) != FEMX_OK)
     return ins_fail(s, r);
   GmresState h0;
@@ -913,6 +1170,9 @@ extern "C" femx_status femx_ins_create(femx_mesh *mesh, const double *el_diff, i
   h0.max_iter = p->max_iter;
   hipError_t he = hipMemsetAsync(s->vphi.p, 0, sizeof(double4) * N, s->st);
   if (he == hipSuccess) he = hipMemsetAsync(s->phid.p, 0, sizeof(double) * N, s->st);
+  // coordinates with a zero fourth component: phid = 0
+  if (he == hipSuccess && rows)
+    he = hipMemcpyAsync(s->node.p, m.xyz.p, sizeof(double4) * N, hipMemcpyDeviceToDevice, s->st);
   if (he == hipSuccess) he = hipMemsetAsync(s->x.p, 0, sizeof(double) * N, s->st);
   if (he == hipSuccess) he = hipMemsetAsync(s->V.p, 0, sizeof(double) * s->ldv * (M + 1), s->st);
   if (he == hipSuccess) he = hipMemcpyAsync(s->gst.p, &h0, sizeof(h0), hipMemcpyHostToDevice, s->st);
@@ -942,7 +1202,11 @@ extern "C" femx_status femx_ins_set_state(femx_ins *s, const double *phi, const 
   }
   FEMX_HIP(hipSetDevice(s->mesh->device));
   const int N = s->mesh->N;
-  if (phi_dot) FEMX_HIP(hipMemcpyAsync(s->phid.p, phi_dot, sizeof(double) * N, hipMemcpyHostToDevice, s->st));
+  if (phi_dot) {
+    FEMX_HIP(hipMemcpyAsync(s->phid.p, phi_dot, sizeof(double) * N, hipMemcpyHostToDevice, s->st));
+    if (s->node.p)
+      ins_node_phid<<<grid_for(N, 256), 256, 0, s->st>>>(N, s->phid.p, reinterpret_cast<double *>(s->node.p));
+  }
   if (phi) {
     FEMX_HIP(hipMemcpyAsync(s->stage.p, phi, sizeof(double) * N, hipMemcpyHostToDevice, s->st));
     ins_pack<<<grid_for(N, 256), 256, 0, s->st>>>(N, s->stage.p, nullptr, s->vphi.p);
@@ -1002,7 +1266,8 @@ extern "C" femx_status femx_ins_update(femx_ins *s) {
   const int N = s->mesh->N;
   {
     TimedLaunch tl(s->timer, s->timer.kind("ins_update", N * (32.0 * 2 + 8.0 * 3)), s->st);
-    ins_update<<<grid_for(N, 256), 256, 0, s->st>>>(N, s->p.dt, s->p.gamma, s->vphi.p, s->phid.p, s->x.p);
+    ins_update<<<grid_for(N, 256), 256, 0, s->st>>>(N, s->p.dt, s->p.gamma, s->vphi.p, s->phid.p,
+                                                      reinterpret_cast<double *>(s->node.p), s->x.p);
   }
   FEMX_HIP(hipGetLastError());
   s->have_solution = false;

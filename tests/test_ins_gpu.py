@@ -161,3 +161,28 @@ def test_iteration_cap_and_errors(gpu):
     st = z.advdiff_solve()
     assert st["converged"] and st["iterations"] == 0
     assert not z.get_system()[4].any()
+
+
+def test_system_with_long_rows(gpu):
+    """tet4 rows of more entries than one pass sums in LDS (a fan's centre
+    has 259), a node of no element and Dirichlet rows among them: the system
+    matches the oracle to 1e-12 of its largest entry."""
+    m0 = meshgen.tet_fan(3)
+    m = meshgen.Mesh(np.vstack([m0.coords, [[3.0, 3.0, 3.0]]]), m0.conn)
+    rng = np.random.default_rng(2)
+    diff = rng.uniform(0.0, 0.02, (m.n_elems, 3))
+    dn = np.arange(5, 40, 3, dtype=np.int32)
+    dv = rng.normal(size=(len(dn), 3))
+    vel = rng.normal(size=(m.n_nodes, 3))
+    phi, phid = rng.normal(size=m.n_nodes), rng.normal(size=m.n_nodes)
+    g = gpu.INSSolver(gpu.DeviceMesh(m), el_diff=diff, dir_node=dn, dir_val=dv, tol=1e-8, **PARAMS)
+    o = INSOracle(m, diff, dn, dv, PARAMS["dt"], PARAMS["alpha_m"], PARAMS["alpha_f"], PARAMS["gamma"], tol=1e-8)
+    g.set_state(phi=phi, phi_dot=phid, vel=vel)
+    o.phi, o.phid, o.vel = phi.copy(), phid.copy(), vel.copy()
+    g.advdiff_solve()
+    val, rhs = o.assemble()
+    rp, col, gval, grhs, _ = g.get_system()
+    assert np.array_equal(rp, o.rp) and np.array_equal(col, o.col)
+    assert np.diff(rp).max() > 200
+    assert np.abs(gval - val).max() <= 1e-12 * np.abs(val).max()
+    assert np.abs(grhs - rhs).max() <= 1e-12 * np.abs(rhs).max()
