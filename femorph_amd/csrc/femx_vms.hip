@@ -1038,16 +1038,32 @@ __global__ void vms_bc_only(int nrec, const int *rec_node, const BCRecord *rec, 
 // |res_u| and |res_p| (eval_residual_norms :774-793).  el_u / el_p NULL: the
 // maxima only.  (An element lists each node once: a corner's running sum
 // then includes exactly the elements up to its own.)
+struct DiagArgs {
+  int nb, nfix, head;  // element blocks, fix-up workgroups, workgroups in front of the blocks
+  const int *elem_off, *node_off;
+  const ushort4 *ecorn;
+  const int2 *lnode;
+  const int *perm;
+  const void *img;  // T4
+  const int *xoff, *xpos;
+  double *el_u, *el_p;
+  double *nmax;  // [nb][2]
+  // the maxima of the iteration before, reduced to prev_out by this launch
+  // (NULL: none, the first iteration of a call)
+  int n_bmax;
+  const double *prev_nmax, *prev_bmax;
+  double *prev_out;
+};
+
 template <typename T4>
-__global__ __launch_bounds__(256) void vms_diag_centroid(const int *elem_off, const int *node_off,
-                                                         const ushort4 *ecorn, const int2 *lnode, const int *perm,
-                                                         const T4 *img, const int *xoff, const int *xpos,
-                                                         double *el_u, double *el_p, double *nmax) {
+__device__ __forceinline__ void diag_centroid(const DiagArgs &a, const int blk) {
   // the running sums of the block's contributions, in the element math's
   // precision (FP32 with FEMX_MIXED: half the LDS, twice the waves)
   __shared__ T4 sp[4 * VB];
-  const int blk = blockIdx.x, tid = threadIdx.x;
-  const int e0 = elem_off[blk], ne = elem_off[blk + 1] - e0, n0 = node_off[blk];
+  const int tid = threadIdx.x;
+  const int e0 = a.elem_off[blk], ne = a.elem_off[blk + 1] - e0, n0 = a.node_off[blk];
+  const T4 *img = static_cast<const T4 *>(a.img);
+  const int *const xoff = a.xoff, *const xpos = a.xpos;
   // a thread's 4 contributions and up to XN cross terms each: every load of
   // one round is issued before the next round needs it
   constexpr int QN = 4, XN = 3;
@@ -1063,6 +1079,15 @@ __global__ __launch_bounds__(256) void vms_diag_centroid(const int *elem_off, co
       xa[u] = xoff[p];
       xb[u] = xoff[p + 1];
     }
+  }
+  // the element's corners: the entries of its four nodes' runs
+  int qc[4] = {0, 0, 0, 0};
+  if (tid < ne) {
+    const ushort4 ec = a.ecorn[e0 + tid];
+    const unsigned short cn[4] = {ec.x, ec.y, ec.z, ec.w};
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      qc[k] = (a.lnode[n0 + (cn[k] & EC_ID)].y & LN_BEGIN) + ((cn[k] >> EC_RANK_SHIFT) & EC_RANK);
   }
 #pragma unroll
   for (int u = 0; u < QN; u++)
@@ -1099,25 +1124,21 @@ __global__ __launch_bounds__(256) void vms_diag_centroid(const int *elem_off, co
   __syncthreads();
   double un = 0.0, pn = 0.0;
   if (tid < ne) {
-    const int i = e0 + tid;
-    const ushort4 ec = ecorn[i];
-    const unsigned short c[4] = {ec.x, ec.y, ec.z, ec.w};
     double u0 = 0.0, u1 = 0.0, u2 = 0.0, p = 0.0;
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-      const int j = c[a] & EC_ID, rank = (c[a] >> EC_RANK_SHIFT) & EC_RANK;
-      const T4 w = sp[(lnode[n0 + j].y & LN_BEGIN) + rank];
+    for (int k = 0; k < 4; k++) {
+      const T4 w = sp[qc[k]];
       u0 += (double)w.x * 0.25;
       u1 += (double)w.y * 0.25;
       u2 += (double)w.z * 0.25;
       p += (double)w.w * 0.25;
     }
-    if (el_u) {
-      const long eo = perm[i];
-      el_u[3 * eo] = u0;
-      el_u[3 * eo + 1] = u1;
-      el_u[3 * eo + 2] = u2;
-      el_p[eo] = p;
+    if (a.el_u) {
+      const long eo = a.perm[e0 + tid];
+      a.el_u[3 * eo] = u0;
+      a.el_u[3 * eo + 1] = u1;
+      a.el_u[3 * eo + 2] = u2;
+      a.el_p[eo] = p;
     }
     un = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
     pn = fabs(p);
@@ -1136,25 +1157,24 @@ __global__ __launch_bounds__(256) void vms_diag_centroid(const int *elem_off, co
   if (tid < 2) {
     double m = wm[tid][0];
     for (int w = 1; w < VB / 64; w++) m = wm[tid][w] > m ? wm[tid][w] : m;
-    nmax[2L * blk + tid] = m;
+    a.nmax[2L * blk + tid] = m;
   }
 }
 
-// One workgroup of RED_T threads: out[0..2] = max |res_u|, max |res_p|, max
-// pre-BC |u|^2.
-constexpr int RED_T = 1024;
-__global__ __launch_bounds__(RED_T) void vms_diag_reduce(int nb, const double *nmax, int n_bmax, const double *bmax,
-                                                         double *out) {
+// Maxima over workgroups: out[0..2] = max |res_u|, max |res_p|, max pre-BC
+// |u|^2 of one iteration; one workgroup of NT threads.
+template <int NT>
+__device__ __forceinline__ void diag_reduce(int nb, const double *nmax, int n_bmax, const double *bmax, double *out) {
   double v[3] = {0.0, 0.0, 0.0};
   // unrolled so that many independent loads are in flight per thread
 #pragma unroll 16
-  for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+  for (int i = threadIdx.x; i < nb; i += NT) {
     v[0] = nmax[2L * i] > v[0] ? nmax[2L * i] : v[0];
     v[1] = nmax[2L * i + 1] > v[1] ? nmax[2L * i + 1] : v[1];
   }
 #pragma unroll 16
-  for (int i = threadIdx.x; i < n_bmax; i += blockDim.x) v[2] = bmax[i] > v[2] ? bmax[i] : v[2];
-  __shared__ double wm[3][RED_T / 64];
+  for (int i = threadIdx.x; i < n_bmax; i += NT) v[2] = bmax[i] > v[2] ? bmax[i] : v[2];
+  __shared__ double wm[3][NT / 64];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     for (int off = 32; off > 0; off >>= 1) {
@@ -1166,9 +1186,40 @@ __global__ __launch_bounds__(RED_T) void vms_diag_reduce(int nb, const double *n
   __syncthreads();
   if (threadIdx.x < 3) {
     double m = wm[threadIdx.x][0];
-    for (int i = 1; i < RED_T / 64; i++) m = wm[threadIdx.x][i] > m ? wm[threadIdx.x][i] : m;
+    for (int i = 1; i < NT / 64; i++) m = wm[threadIdx.x][i] > m ? wm[threadIdx.x][i] : m;
     out[threadIdx.x] = m;
   }
+}
+
+// One launch after the block kernel of an iteration with diagnostics: the
+// fix-up of the shared nodes (T), the centroid residuals of every block (T4)
+// and the reduction of the iteration before, which nothing waits for, are
+// independent of each other.  The head is a multiple of 8 workgroups, so a
+// block's centroids run on the XCD that holds the image entries its
+// neighbours just wrote (xcd_block, as in the block kernel).
+// Bound by its chain of dependent loads on small meshes (offsets, positions,
+// other blocks' entries) and by those gathers on large ones.  Measured in one
+// launch against three (fix-up, centroids, reduction): 216k tets FP64 15.9
+// against 6.1 + 17.7 + 4.5 us, a whole iteration 42.6 against 55.2 us; 48k
+// tets FP32 19.2 against 30.4, 5.3M FP32 436 against 458, FP64 743 against
+// 789 us.
+template <typename T, typename T4>
+__global__ __launch_bounds__(256) void vms_fixup_diag(FixArgs f, DiagArgs a) {
+  const int w = blockIdx.x;
+  if (w >= a.head) {
+    diag_centroid<T4>(a, xcd_block(w - a.head, a.nb));
+  } else if (w < a.nfix) {
+    vms_fixup_run<T>(f, w * 256 + threadIdx.x, w);
+  } else if (w == a.nfix && a.prev_out) {
+    diag_reduce<256>(a.nb, a.prev_nmax, a.n_bmax, a.prev_bmax, a.prev_out);
+  }
+}
+
+// The reduction of a call's last iteration.
+constexpr int RED_T = 1024;
+__global__ __launch_bounds__(RED_T) void vms_diag_reduce(int nb, const double *nmax, int n_bmax, const double *bmax,
+                                                         double *out) {
+  diag_reduce<RED_T>(nb, nmax, n_bmax, bmax, out);
 }
 
 // reference layout sdus[(g*3+i)*E + original e]  <->  block order, tiled
@@ -1206,8 +1257,12 @@ struct femx_vms {
   DevBuf<int> sh_rec;    // per shared node: BC record or -1
   DevBuf<double> sdus64;
   DevBuf<float> sdus32;
-  DevBuf<double> bmax;  // per-block maxima of the last iteration: block kernel, then fix-up
+  // per-block maxima of an iteration: block kernel, then fix-up.  Two halves
+  // of n_bmax; iterations with diagnostics alternate (their maxima are reduced
+  // while the next iteration runs), half is the one of the last iteration
+  DevBuf<double> bmax;
   int n_bmax = 0;
+  int half = 0;
   // the iteration being launched writes its maxima (a call's last one, every
   // one with diagnostics): the wave and block reductions end each workgroup,
   // and nothing reads the other iterations' values
@@ -1233,7 +1288,7 @@ struct femx_vms {
   long diag_xn = 0;
   DevBuf<double> diag_sdu;   // [E][3]
   DevBuf<double> diag_el;    // [E][3] centroid residual u v w, then [E] p
-  DevBuf<double> diag_nmax;  // [blocks][2]
+  DevBuf<double> diag_nmax;  // [2][blocks][2], halves as bmax
   // per-iteration norms of the last DIAG_RING steps run with diagnostics:
   // [DIAG_RING][tot_dual_steps + 1][3], step k in row k mod DIAG_RING
   DevBuf<double> diag_ring;
@@ -1314,7 +1369,7 @@ BlockArgs<T> block_args(femx_vms *s, bool first_dual, double t, T *sdus) {
   a.row_off = s->bc.row_off.p;
   a.rows = s->bc.rows.p;
   a.err = s->bc.err.p;
-  a.bmax = s->bmax.p;
+  a.bmax = s->bmax.p + (long)s->n_bmax * s->half;
   a.want_max = s->want_max;
   a.perm = b.d_perm.p;
   a.diag_img = s->diag ? s->diag_img.p : nullptr;
@@ -1378,7 +1433,7 @@ FixArgs fix_args(femx_vms *s, bool first_dual, double t) {
   a.row_off = s->bc.row_off.p;
   a.rows = s->bc.rows.p;
   a.err = s->bc.err.p;
-  a.bmax = s->bmax.p + b.nb;
+  a.bmax = s->bmax.p + (long)s->n_bmax * s->half + b.nb;
   a.want_max = s->want_max;
   a.node_mesh = s->batch ? s->node_mesh.p : nullptr;
   a.kt = s->batch ? s->kt.p : nullptr;
@@ -1386,15 +1441,21 @@ FixArgs fix_args(femx_vms *s, bool first_dual, double t) {
   return a;
 }
 
+// Bytes of one fix-up: partials written and read; per shared node its index,
+// slot range, first slots, 1/m and BC record, the base state read and the
+// post-BC state written.
+double fixup_bytes(const femx_vms *s) {
+  const Blocks &b = s->mesh->blk;
+  if (b.n_sh == 0) return 0.0;
+  const double rec_bytes = f32_sum(s->p.precision) ? 16.0 : 32.0;  // one partial slot record
+  return b.sh_off[b.n_sh] * rec_bytes * 2 + b.n_sh * (4.0 + 4.0 + 16.0 + 8.0 + 4.0 + 32.0 + 32.0);
+}
+
 femx_status launch_fixup(femx_vms *s, bool first_dual, double t) {
   Blocks &b = s->mesh->blk;
   if (b.n_sh == 0) return FEMX_OK;
   const bool f32p = f32_sum(s->p.precision);
-  const double rec_bytes = f32p ? 16.0 : 32.0;  // one partial slot record
-  // partials written and read; per shared node its index, slot range, first
-  // slots, 1/m and BC record, the base state read and the post-BC state written
-  const double bytes = b.sh_off[b.n_sh] * rec_bytes * 2 + b.n_sh * (4.0 + 4.0 + 16.0 + 8.0 + 4.0 + 32.0 + 32.0);
-  TimedLaunch tl(s->timer, s->timer.kind("vms_fixup", bytes), s->st);
+  TimedLaunch tl(s->timer, s->timer.kind("vms_fixup", fixup_bytes(s)), s->st);
   const FixArgs a = fix_args(s, first_dual, t);
   if (f32p) vms_fixup<float><<<grid_for(b.n_sh, 256), 256, 0, s->st>>>(a);
   else vms_fixup<double><<<grid_for(b.n_sh, 256), 256, 0, s->st>>>(a);
@@ -1402,30 +1463,57 @@ femx_status launch_fixup(femx_vms *s, bool first_dual, double t) {
   return FEMX_OK;
 }
 
-// Diagnostics of dual iteration d from the running sums the block kernel
-// just left in the image: centroid residuals per block, then the maxima.
-template <typename T4>
-void launch_diag_t(femx_vms *s, int d) {
-  Mesh &m = *s->mesh;
-  const Blocks &b = m.blk;
-  double *el = s->diag == 1 ? s->diag_el.p : nullptr;
-  vms_diag_centroid<T4><<<b.nb, VB, 0, s->st>>>(b.d_elem_off.p, b.d_node_off.p, s->ecorn.p, s->lnode.p, b.d_perm.p,
-                                                reinterpret_cast<const T4 *>(s->diag_img.p), s->diag_xoff.p,
-                                                s->diag_xpos.p, el, el ? el + 3L * m.E : nullptr, s->diag_nmax.p);
-  const long row = (s->diag_steps % DIAG_RING) * (s->p.tot_dual_steps + 1) + d;
-  vms_diag_reduce<<<1, RED_T, 0, s->st>>>(b.nb, s->diag_nmax.p, s->n_bmax, s->bmax.p, s->diag_ring.p + 3L * row);
+// Ring row of dual iteration d of the current step.
+double *diag_row(femx_vms *s, int d) {
+  return s->diag_ring.p + 3L * ((s->diag_steps % DIAG_RING) * (s->p.tot_dual_steps + 1) + d);
 }
 
-femx_status launch_diag(femx_vms *s, int d) {
+// Fix-up and diagnostics of one iteration, from the partials and the running
+// sums the block kernel just left; the maxima of the iteration before go to
+// its ring row prev (NULL: none).
+femx_status launch_fixup_diag(femx_vms *s, bool first_dual, double t, double *prev) {
   Mesh &m = *s->mesh;
-  const bool f32 = f32_elem(s->p.precision);
-  // per corner its image entry and offset, per cross term a position and an
-  // entry (other blocks' runs), per element its corner record
+  const Blocks &b = m.blk;
+  const bool f32 = f32_elem(s->p.precision), f32p = f32_sum(s->p.precision);
+  // the fix-up's bytes; per corner its image entry and offset, per cross term
+  // a position and an entry (other blocks' runs), per element its corner record
   const double rec = f32 ? 16.0 : 32.0;
-  const double xn = s->diag_xn;
-  TimedLaunch tl(s->timer, s->timer.kind("vms_diag", m.E * 4.0 * (rec + 4.0) + xn * (rec + 4.0) + m.E * 8.0), s->st);
-  if (f32) launch_diag_t<float4>(s, d);
-  else launch_diag_t<double4>(s, d);
+  const double bytes = fixup_bytes(s) + m.E * 4.0 * (rec + 4.0) + s->diag_xn * (rec + 4.0) + m.E * 8.0;
+  TimedLaunch tl(s->timer, s->timer.kind("vms_fixup_diag", bytes), s->st);
+  const FixArgs f = fix_args(s, first_dual, t);
+  DiagArgs a;
+  a.nb = b.nb;
+  a.nfix = b.n_sh ? grid_for(b.n_sh, 256) : 0;
+  a.head = (a.nfix + 1 + 7) / 8 * 8;
+  a.elem_off = b.d_elem_off.p;
+  a.node_off = b.d_node_off.p;
+  a.ecorn = s->ecorn.p;
+  a.lnode = s->lnode.p;
+  a.perm = b.d_perm.p;
+  a.img = s->diag_img.p;
+  a.xoff = s->diag_xoff.p;
+  a.xpos = s->diag_xpos.p;
+  a.el_u = s->diag == 1 ? s->diag_el.p : nullptr;
+  a.el_p = a.el_u ? a.el_u + 3L * m.E : nullptr;
+  a.nmax = s->diag_nmax.p + 2L * b.nb * s->half;
+  a.n_bmax = s->n_bmax;
+  a.prev_nmax = s->diag_nmax.p + 2L * b.nb * (s->half ^ 1);
+  a.prev_bmax = s->bmax.p + (long)s->n_bmax * (s->half ^ 1);
+  a.prev_out = prev;
+  const int grd = a.head + b.nb;
+  if (f32p) vms_fixup_diag<float, float4><<<grd, 256, 0, s->st>>>(f, a);
+  else if (f32) vms_fixup_diag<double, float4><<<grd, 256, 0, s->st>>>(f, a);
+  else vms_fixup_diag<double, double4><<<grd, 256, 0, s->st>>>(f, a);
+  FEMX_HIP(hipGetLastError());
+  return FEMX_OK;
+}
+
+// The maxima of the iteration just run to its ring row.
+femx_status launch_diag_reduce(femx_vms *s, double *row) {
+  const Blocks &b = s->mesh->blk;
+  TimedLaunch tl(s->timer, s->timer.kind("vms_diag_reduce", 8.0 * (2.0 * b.nb + s->n_bmax)), s->st);
+  vms_diag_reduce<<<1, RED_T, 0, s->st>>>(b.nb, s->diag_nmax.p + 2L * b.nb * s->half, s->n_bmax,
+                                          s->bmax.p + (long)s->n_bmax * s->half, row);
   FEMX_HIP(hipGetLastError());
   return FEMX_OK;
 }
@@ -1545,8 +1633,8 @@ extern "C" femx_status femx_vms_create(femx_mesh *mh, const femx_bc_desc *bc, co
   const bool mixed = f32_elem(p->precision);
   if ((r = mixed ? s->sdus32.alloc(sdus_len(m.E)) : s->sdus64.alloc(sdus_len(m.E))) != FEMX_OK) return fail(r);
   s->n_bmax = m.blk.nb + grid_for(std::max(m.blk.n_sh, 1), 256);
-  if ((r = s->bmax.alloc(s->n_bmax)) != FEMX_OK) return fail(r);
-  if (hipMemsetAsync(s->bmax.p, 0, s->n_bmax * sizeof(double), s->st) != hipSuccess) return fail(FEMX_ERR_HIP);
+  if ((r = s->bmax.alloc(2L * s->n_bmax)) != FEMX_OK) return fail(r);
+  if (hipMemsetAsync(s->bmax.p, 0, 2L * s->n_bmax * sizeof(double), s->st) != hipSuccess) return fail(FEMX_ERR_HIP);
   for (int k = 0; k < 2; k++) {
     if (hipMemsetAsync(s->Pr[k].p, 0, std::max(s->bc.n_rec, 1) * sizeof(double4), s->st) != hipSuccess)
       return fail(FEMX_ERR_HIP);
@@ -1613,7 +1701,7 @@ extern "C" femx_status femx_vms_set_state(femx_vms *s, const double *sol, const 
   s->proj_pending = false;
   FEMX_HIP(hipMemcpyAsync(s->Q[0].p, sol, m.N * sizeof(double4), hipMemcpyHostToDevice, s->st));
   FEMX_HIP(hipMemsetAsync(s->bc.err.p, 0, sizeof(int), s->st));
-  FEMX_HIP(hipMemsetAsync(s->bmax.p, 0, s->n_bmax * sizeof(double), s->st));
+  FEMX_HIP(hipMemsetAsync(s->bmax.p, 0, 2L * s->n_bmax * sizeof(double), s->st));
   if (s->bc.n_rec > 0)
     vms_bc_only<<<grid_for(s->bc.n_rec, 256), 256, 0, s->st>>>(s->bc.n_rec, s->rec_node.p, s->bc.rec.p,
                                                                s->bc.row_off.p, s->bc.rows.p, 0.0, s->Q[0].p,
@@ -1646,21 +1734,24 @@ extern "C" femx_status femx_vms_set_state(femx_vms *s, const double *sol, const 
 extern "C" femx_status femx_vms_step(femx_vms *s, int nsteps) {
   if (!s || nsteps < 0) return set_error("bad argument"), FEMX_ERR_ARG;
   if (s->in_union) return set_error("the handle is in a union"), FEMX_ERR_ARG;
+  double *row = nullptr;  // ring row of the iteration before, its maxima not yet reduced
   for (int k = 0; k < nsteps; k++) {
     s->time += s->p.dt;  // currentTime += timeStep (:1028)
     for (int d = 0; d <= s->p.tot_dual_steps; d++) {
+      if (s->diag) s->half ^= 1;
       s->want_max = s->diag || (k == nsteps - 1 && d == s->p.tot_dual_steps);
       femx_status r = launch_block(s, s->proj_pending, true, d > 0, d == 0, s->time);
       if (r != FEMX_OK) return r;
-      if ((r = launch_fixup(s, d == 0, s->time)) != FEMX_OK) return r;
-      if (s->diag && (r = launch_diag(s, d)) != FEMX_OK) return r;
+      r = s->diag ? launch_fixup_diag(s, d == 0, s->time, row) : launch_fixup(s, d == 0, s->time);
+      if (r != FEMX_OK) return r;
+      if (s->diag) row = diag_row(s, d);
       s->cur ^= 1;
       s->proj_pending = true;
       s->iter++;
     }
     if (s->diag) s->diag_steps++;
   }
-  return FEMX_OK;
+  return row ? launch_diag_reduce(s, row) : FEMX_OK;
 }
 
 extern "C" femx_status femx_vms_get_state(femx_vms *s, double *sol, double *sdus, double *time) {
@@ -1696,7 +1787,8 @@ extern "C" femx_status femx_vms_get_mass(femx_vms *s, double *nd_mass) {
 extern "C" femx_status femx_vms_get_cfl(femx_vms *s, double *max_u, double *cfl) {
   if (!s) return set_error("null argument"), FEMX_ERR_ARG;
   std::vector<double> h(s->n_bmax);
-  FEMX_HIP(hipMemcpyAsync(h.data(), s->bmax.p, s->n_bmax * sizeof(double), hipMemcpyDeviceToHost, s->st));
+  FEMX_HIP(hipMemcpyAsync(h.data(), s->bmax.p + (long)s->n_bmax * s->half, s->n_bmax * sizeof(double),
+                          hipMemcpyDeviceToHost, s->st));
   FEMX_HIP(hipStreamSynchronize(s->st));
   double m2 = 0.0;
   const int used = s->mesh->blk.nb + (s->mesh->blk.n_sh ? grid_for(s->mesh->blk.n_sh, 256) : 0);
@@ -1766,7 +1858,7 @@ extern "C" femx_status femx_vms_set_diagnostics(femx_vms *s, int enable) {
     if ((r = s->diag_img.alloc(4 * E * rec)) != FEMX_OK ||
         (r = s->diag_xoff.upload(xoff.data(), xoff.size(), s->st)) != FEMX_OK ||
         (r = s->diag_xpos.upload(xpos.data(), xpos.size(), s->st)) != FEMX_OK ||
-        (r = s->diag_nmax.alloc(2L * std::max(b.nb, 1))) != FEMX_OK || (r = s->diag_ring.alloc(3L * nrow)) != FEMX_OK)
+        (r = s->diag_nmax.alloc(4L * std::max(b.nb, 1))) != FEMX_OK || (r = s->diag_ring.alloc(3L * nrow)) != FEMX_OK)
       return r;
     FEMX_HIP(hipMemsetAsync(s->diag_ring.p, 0, 3L * nrow * sizeof(double), s->st));
   }

@@ -271,6 +271,34 @@ def test_norms_ring_without_fields(gpu):
     np.testing.assert_allclose(g.get_norms(1)[0], d["iter_norms"], rtol=0, atol=0)
 
 
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("n,tot_dual", [(1, 1), (4, 0), (9, 1)])
+def test_norms_of_many_steps_a_call(gpu, precision, n, tot_dual):
+    """An iteration's maxima are reduced by the launch of the next one, the
+    last one's at the end of the call: five steps in one call leave the rows,
+    fields and state of five one-step calls, bit for bit (maxima have no
+    order), on one block (no shared nodes), a few and many; the CFL number
+    is the last row's."""
+    m, bc, params, ic = _case("channel", n, 0.1, seed=8)
+    got = []
+    for calls in ([5], [1] * 5):
+        _, g, _ = _pair(gpu, m, bc, params, ic, precision=precision, tot_dual_steps=tot_dual)
+        g.set_diagnostics(1)
+        for k in calls:
+            g.step(k)
+        cfl = g.get_cfl()[1]
+        norms = g.get_norms(5)
+        # (one cell: every node is on a wall, and all velocities stay zero)
+        assert np.isfinite(norms).all() and ((norms[:, :, 0] > 0).all() or n == 1)
+        assert norms[-1, -1, 2] == cfl
+        g.set_diagnostics(0)
+        g.step(1)
+        d = g.get_diagnostics()
+        got.append([norms, d["res_v"], d["res_p"], d["subgrid_u"], g.get_state()[0], np.array(g.get_cfl())])
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("precision,tol", [(0, TOL64), (1, 1e-5)])
 def test_high_valence_node(gpu, precision, tol):
     """A node with 512 incident tets: the block builder splits its corners
