@@ -7,6 +7,7 @@
 #include <cstring>
 #include <map>
 #include <numeric>
+#include <system_error>
 #include <thread>
 
 #include "femx_common.h"
@@ -228,14 +229,20 @@ void pin_put(int d, Pin &c) {
 }
 
 // Pieces of at most one chunk, taken from a shared counter: the thread's two
-// chunks alternate, so that the next piece is in flight while one is copied out.
+// chunks alternate, so that the next piece is in flight while one is copied
+// out.  Where no pinned memory is to be had the pieces are copied directly.
 hipError_t read_pieces(hipStream_t st, int d, const std::vector<ReadPiece> &q, std::atomic<size_t> &next) {
   Pin c[2];
   size_t in_c[2] = {0, 0};
   bool busy[2] = {false, false};
   hipError_t e = hipSetDevice(d);
-  for (int i = 0; i < 2 && e == hipSuccess; i++) e = pin_get(d, c[i]);
-  for (int i = 0; e == hipSuccess; i ^= 1) {
+  const bool pinned = e == hipSuccess && pin_get(d, c[0]) == hipSuccess && pin_get(d, c[1]) == hipSuccess;
+  if (e == hipSuccess && !pinned) {
+    (void)hipGetLastError();
+    for (size_t k; e == hipSuccess && (k = next.fetch_add(1)) < q.size();)
+      e = hipMemcpyAsync(q[k].dst, q[k].src, q[k].bytes, hipMemcpyDeviceToHost, st);
+  }
+  for (int i = 0; pinned && e == hipSuccess; i ^= 1) {
     // queue the next piece into chunk i, then drain the other one
     const size_t k = next.fetch_add(1);
     if (k < q.size()) {
@@ -266,15 +273,19 @@ femx_status read_back(hipStream_t st, const ReadPiece *p, int n) {
   for (int i = 0; i < n; i++) total += (p[i].bytes + 63) & ~size_t(63);
   int d = 0;
   FEMX_HIP(hipGetDevice(&d));
-  if (d < 0 || d >= CACHE_DEVICES) {
+  Pin c;
+  bool direct = d < 0 || d >= CACHE_DEVICES;
+  if (!direct && total <= PIN_CHUNK && pin_get(d, c) != hipSuccess) {
+    (void)hipGetLastError();
+    direct = true;
+  }
+  if (direct) {
     for (int i = 0; i < n; i++)
       if (p[i].bytes) FEMX_HIP(hipMemcpyAsync(p[i].dst, p[i].src, p[i].bytes, hipMemcpyDeviceToHost, st));
     FEMX_HIP(hipStreamSynchronize(st));
     return FEMX_OK;
   }
   if (total <= PIN_CHUNK) {
-    Pin c;
-    FEMX_HIP(pin_get(d, c));
     hipError_t e = hipSuccess;
     size_t off = 0;
     for (int i = 0; i < n && e == hipSuccess; i++) {
@@ -301,7 +312,11 @@ femx_status read_back(hipStream_t st, const ReadPiece *p, int n) {
   std::atomic<size_t> next{0};
   std::vector<hipError_t> err(h + 1, hipSuccess);
   std::vector<std::thread> th;
-  for (int t = 1; t <= h; t++) th.emplace_back([&, t] { err[t] = read_pieces(st, d, q, next); });
+  try {
+    th.reserve(h);
+    for (int t = 1; t <= h; t++) th.emplace_back([&, t] { err[t] = read_pieces(st, d, q, next); });
+  } catch (const std::system_error &) {  // fewer threads, the same pieces
+  }
   err[0] = read_pieces(st, d, q, next);
   for (auto &x : th) x.join();
   if (h) give_helpers(h);
