@@ -467,27 +467,38 @@ struct StrainConst {
 };
 
 // One Gauss point (:1095-1507): from the velocity ug, its gradient gU[b][i] =
-// du_i/dx_b, |J^T u|^2 (l2sq), |invJ u|^2 (t2), |G|^2 (gg), tr G and dv, the
-// stabilization and the bulk modulus (lam, f3), c = (u.grad) u, and the
-// matrix A of the node forces A DN_n (f2 S + f4 I: stress and grad-div).
+// du_i/dx_b, J and the velocity that G^-1 = J J^T is applied to (ul), |invJ
+// u|^2 (t2), |G|^2 (gg), tr G and dv, the stabilization and the bulk modulus
+// (lam, f3), c = (u.grad) u, and the matrix A of the node forces A DN_n (f2 S
+// + f4 I: stress and grad-div).
 template <typename T, bool BHAT, bool DIAG>
 __device__ __forceinline__ void gauss_point(const ElemConst<T> &k, double dt, const T ug[3], const T gU[3][3], T div,
-                                            T dv, T l2sq, T t2, T gg, T trG, const StrainConst<T, BHAT> &sc,
-                                            ElemAcc<T> &s, double *dg, T &f3, T c[3], T A[3][3]) {
+                                            T dv, const T J[3][3], const T ul[3], T t2, T gg, T trG,
+                                            const StrainConst<T, BHAT> &sc, ElemAcc<T> &s, double *dg, T &f3, T c[3],
+                                            T A[3][3]) {
   // eval_stabilization (:336-377), tau without the (2/dt)^2 term
   const T tau = rsqrt_e(t2 + gg * k.cnu2);
   const T nuC = recip(trG * tau);
   // eval_bulk_modulus (:382-441): lambda = alpha max(mu/rho, sqrt(u^T G^-1 u))
-  const T l2 = sqrt_e(l2sq);
+  const T l2 = sqrt_e(norm2_tmul(J, ul));
   const T lam = k.alpha * ((k.nu < l2) ? l2 : k.nu);
   s.reg += (k.nu > l2) ? (T)1 : (T)2;
   s.lam_int += lam * dv;
   if (DIAG) {
     // get_el_lengths_from_G (:756-790) and the CFL / tau / lambda extrema
-    // (:1187-1240), in FP64: 2 sqrt(o^T G^-1 o), o = u / |u|
+    // (:1187-1240), in FP64: 2 sqrt(o^T G^-1 o), o = u / |u|.  Of the
+    // direction, not |J^T u| / |u|: ahead of a front that spreads from rest u
+    // falls by orders of magnitude per element, and in T the square of |J^T u|
+    // would be 0 (an infinite CFL) where u is not
     const double u0 = ug[0], u1 = ug[1], u2 = ug[2];
     const double un = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
-    const double el = 2.0 * (sqrt((double)l2sq) / un);
+    const double o[3] = {(double)ul[0] / un, (double)ul[1] / un, (double)ul[2] / un};
+    double Jd[3][3];
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) Jd[r][b] = (double)J[r][b];
+    const double el = 2.0 * sqrt(norm2_tmul(Jd, o));
     const double nk = k.nu, lm = lam, ta = tau;
     dg[D_ACFL - D_TAU] = fmax(dg[D_ACFL - D_TAU], fabs(u0 * dt) / el);
     dg[D_VCFL - D_TAU] = fmax(dg[D_VCFL - D_TAU], 2.0 * nk * (dt / (el * el)));
@@ -696,8 +707,8 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
             // the metric's products with u pair the physical components with
             // the local directions, as the reference does
             const T ul[3] = {ug[0], ug[1], sg * ug[2]};
-            gauss_point<T, BHAT, DIAG>(kc, k.dt, ug, gU, div, dv, norm2_tmul(J, ul), norm2_mul(iJ, ul), gg, trG,
-                                       sc, acc, dg, f3, c, A);
+            gauss_point<T, BHAT, DIAG>(kc, k.dt, ug, gU, div, dv, J, ul, norm2_mul(iJ, ul), gg, trG, sc, acc, dg, f3,
+                                       c, A);
             const T f1 = kc.f1 * dv;
             // A DN_n + f3 c (u.grad N_n) in the local derivatives:
             // (A + f3 c (x) u) invJ dN_n
@@ -788,8 +799,8 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
 #pragma unroll
           for (int b = 0; b < 3; b++)
             ug[b] = U0[b] + (S::N(g, 1) * u[1][b] + S::N(g, 2 % NPE) * u[2][b] + S::N(g, 3 % NPE) * u[3][b]);
-          gauss_point<T, false, DIAG>(kc, k.dt, ug, gU, div, dv, norm2_tmul(J, ug), norm2_mul(iJ, ug), gg, trG, sc, acc,
-                                      dg, f3, c, A);
+          gauss_point<T, false, DIAG>(kc, k.dt, ug, gU, div, dv, J, ug, norm2_mul(iJ, ug), gg, trG, sc, acc, dg, f3, c,
+                                      A);
           const T f1 = kc.f1 * dv;
 #pragma unroll
           for (int i = 0; i < 3; i++) {

@@ -169,6 +169,45 @@ def test_log_columns_tet4(gpu):
         np.testing.assert_allclose(lg[2:], lo[2:], rtol=1e-12, atol=0, err_msg=f"step {step}")
 
 
+@pytest.mark.parametrize("kind,precision", [("hexa", 0), ("hexa", 1), ("hexa", 2), ("tet", 0), ("tet", 1)])
+def test_log_columns_from_rest(gpu, kind, precision):
+    """The log row of a cavity started from rest: ahead of the front |u| falls
+    by four orders of magnitude per layer, to 1e-36 (tet4) and below 1e-38
+    (hexa8), where squares of it are 0 in FP32.  The element lengths of the
+    CFL columns depend on its direction only.  Velocities within TOL64 (FP64)
+    or 1e-5 of the lid's, the other columns within the same relative
+    tolerances; on tet4 in FP32, where the direction of a velocity that is a
+    small difference moves the v-CFL, that column is bounded by the smallest
+    length of the mesh in any direction instead."""
+    if kind == "hexa":  # cubes: one length in every direction
+        m, n, exopts = meshgen.hex_cube(14, 0.0), 14, (0, 1, 1, 1, 1, 1)
+    else:
+        m, n, exopts = meshgen.tet_cube(10, 0.0), 10, (0, 0, 1, 1, 1, 1)
+    bc = meshgen.lid_cavity_bc(m)
+    params = dict(rho=1.0, mu=0.0025, alpha=1.0, cI=4.0, dt=0.002 / n)
+    tol = TOL64 if precision == 0 else 1e-5
+    o, g, _ = _pair(gpu, m, bc, params, np.zeros((m.n_nodes, 3)), exopts, precision=precision)
+    g.set_diagnostics(True)
+    small = False
+    for step in range(14):
+        o.step()
+        g.step()
+        u = np.linalg.norm(o.get("sol_n"), axis=1)
+        small |= bool(((u > 1e-36) & (u < 1e-20)).any())
+        lo, lg = o.get("log"), g.get_log()
+        assert np.isfinite(lg).all(), (step, lg)
+        assert lg[0] == lo[0] and lg[1] == lo[1]
+        np.testing.assert_allclose(lg[2:8], lo[2:8], rtol=0, atol=tol, err_msg=f"step {step}")
+        cols = list(range(8, 19))
+        if kind == "tet" and precision:
+            cols.remove(12)
+            x = m.coords[m.conn]
+            el_min = 2.0 * np.linalg.svd(x[:, :3] - x[:, 3:], compute_uv=False)[:, 2].min()
+            assert 0.0 < lg[12] <= 2.0 * params["mu"] * params["dt"] / el_min ** 2 * (1.0 + tol), step
+        np.testing.assert_allclose(lg[cols], lo[cols], rtol=tol, atol=0, err_msg=f"step {step}")
+    assert small
+
+
 def test_log_lcfl_running_max(gpu):
     """Column 14 (l-CFL) is a running maximum since step 1: the reference sets
     l_CFL_max once before the loop (femSUPGExplicitFluidSolver.cpp:996) and
