@@ -576,22 +576,29 @@ template <int LPR>
 __global__ __launch_bounds__(RT) void gm_spmv(int N, const int *rp, const int *col, const double *val,
                                               const double *z, const double *src, double *V, long ldv, double *w,
                                               int j, GmresState *st, const double *part, int nb, int givens) {
-  if (st->cyc_stop) return;
   double sc;
   if (givens) {
     // iteration j - 1 ends here: its norm, and in the first workgroup its
-    // rotation and stop test (after a stop this launch's output is not used)
+    // rotation and stop test (after a stop this launch's output is not used).
+    // That test may set the flag while other waves start, so one wave of each
+    // workgroup reads it for all, and the rotation waits for the barrier: no
+    // wave leaves before a barrier that another one of its workgroup reaches
     __shared__ double hn;
+    __shared__ int stopped;
     if (threadIdx.x < 64) {
-      const double s = wave_total(part, 0, nb);
+      const int stop = uni(st->cyc_stop);
+      const double s = stop ? 0.0 : wave_total(part, 0, nb);
       if (threadIdx.x == 0) {
         hn = sqrt(s);
-        if (blockIdx.x == 0) fin_givens(st, hn, j - 1);
+        stopped = stop;
       }
     }
     __syncthreads();
+    if (stopped) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) fin_givens(st, hn, j - 1);
     sc = hn != 0.0 ? 1.0 / hn : 0.0;
   } else {
+    if (st->cyc_stop) return;
     sc = st->vscale;
   }
   const int lane = threadIdx.x & (LPR - 1);

@@ -186,3 +186,24 @@ def test_system_with_long_rows(gpu):
     assert np.diff(rp).max() > 200
     assert np.abs(gval - val).max() <= 1e-12 * np.abs(val).max()
     assert np.abs(grhs - rhs).max() <= 1e-12 * np.abs(rhs).max()
+
+
+@pytest.mark.parametrize("restart", [30, 4])
+@pytest.mark.parametrize("cap", range(1, 11))
+def test_stop_at_every_iteration(gpu, cap, restart):
+    """A solve stopped by its iteration cap, at each place where the stop can
+    be found: by the next iteration's product (between the host's looks), by
+    the launch before a look, at the end of a cycle; the second and third
+    solves look where the first one stopped.  The iterate is the oracle's
+    (n = 12: 69 workgroups of the product)."""
+    m, g, o = _pair(gpu, "tet", 12, 6, tol=1e-15, restart=restart, max_iter=cap)
+    g.prescribe_velocity(0, 0.4)
+    o.prescribe(0, 0.4)
+    _, it, rr = o.advdiff_solve()
+    assert it == cap
+    for _ in range(3):
+        st = g.advdiff_solve()
+        assert not st["converged"] and st["iterations"] == cap
+        assert abs(st["rel_residual"] - rr) <= 1e-6 * rr + 1e-12, (st, rr)  # (of ||b||: the systems' rounding)
+        x = g.get_system()[4]
+        assert rel_l2(x, o.phid_new) <= 1e-9, rel_l2(x, o.phid_new)
