@@ -126,6 +126,20 @@ struct DevBuf {
   DevBuf &operator=(const DevBuf &) = delete;
 };
 
+// Makes a device the calling thread's current one for a scope.
+struct DeviceGuard {
+  int before = -1;
+  explicit DeviceGuard(int device) {
+    if (hipGetDevice(&before) != hipSuccess || before == device) before = -1;
+    else (void)hipSetDevice(device);
+  }
+  ~DeviceGuard() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+  DeviceGuard(const DeviceGuard &) = delete;
+  DeviceGuard &operator=(const DeviceGuard &) = delete;
+};
+
 // ------------------------------------------------------------ read-back
 // Copies device arrays to the caller's (pageable) host arrays after the work
 // queued on st, and waits for them.  A plain hipMemcpy to pageable memory

@@ -271,8 +271,11 @@ hipError_t read_pieces(hipStream_t st, int d, const std::vector<ReadPiece> &q, s
 femx_status read_back(hipStream_t st, const ReadPiece *p, int n) {
   size_t total = 0;
   for (int i = 0; i < n; i++) total += (p[i].bytes + 63) & ~size_t(63);
+  // chunks and events of the stream's device, whatever the caller's current
+  // one is: an event is recorded on streams of its own device only
   int d = 0;
-  FEMX_HIP(hipGetDevice(&d));
+  FEMX_HIP(hipStreamGetDevice(st, &d));
+  const DeviceGuard guard(d);
   Pin c;
   bool direct = d < 0 || d >= CACHE_DEVICES;
   if (!direct && total <= PIN_CHUNK && pin_get(d, c) != hipSuccess) {

@@ -1621,6 +1621,7 @@ extern "C" femx_status femx_supg_get_state(femx_supg *s, double *sol, double *pr
   if (!s) return set_error("null argument"), FEMX_ERR_ARG;
   if (s->in_union) return set_error("the handle is in a union"), FEMX_ERR_ARG;
   Mesh &m = *s->mesh;
+  const DeviceGuard guard(m.device);
   if (s->pend_n > 0) {
     const femx_status f = supg_finish(s, nullptr);
     if (f != FEMX_OK && f != FEMX_EXIT_CONDITION) return f;

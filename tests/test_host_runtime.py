@@ -1,0 +1,101 @@
+"""The library's host code over a HIP runtime on the host (tests/host/hip_stub.cpp:
+two devices, memory is host memory, kernels do nothing), each case in a process
+of its own: what a caller's current device, missing pinned memory or missing
+threads may not change.  No GPU needed."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+STUB = os.path.join(ROOT, "tests", "host", "hip_stub.cpp")
+
+PRELUDE = """
+import ctypes as C, sys, threading
+import numpy as np
+stub = C.CDLL({stub!r}, mode=C.RTLD_GLOBAL)
+stub.stub_limits.argtypes = [C.c_int, C.c_int, C.c_long]
+sys.path.insert(0, {root!r})
+from femorph_amd import femx, meshgen
+from femorph_amd.mesh import BoundaryConditions, Mesh
+assert femx.device_count() == 2
+
+def log():
+    b = C.create_string_buffer(1 << 20)
+    stub.stub_log(b, len(b))
+    return [l.split() for l in b.value.decode().splitlines()]
+
+def vms(n_nodes):
+    # 6 tets and nodes that no element uses: a state of any size
+    m = meshgen.tet_cube(1)
+    m = Mesh(np.vstack([m.coords, np.full((n_nodes - 8, 3), 2.0)]), m.conn)
+    dm = femx.DeviceMesh(m)
+    g = femx.VMSSolver(dm, BoundaryConditions(), rho=1.0, mu=0.01, inv_eps=1.0, c1=4.0, c2=2.0, dt=0.01)
+    sol = np.random.default_rng(n_nodes).normal(size=(n_nodes, 4))
+    g.set_state(sol)
+    return g, sol
+
+def check(g, sol):
+    np.testing.assert_array_equal(g.get_state()[0], sol)
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    if not shutil.which("g++") or not os.path.exists("/opt/rocm/include/hip/hip_runtime.h"):
+        pytest.skip("no host compiler or HIP headers")
+    out = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-pthread", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", STUB, "-o", out], check=True)
+    return out
+
+
+def _run(stub, code):
+    script = PRELUDE.format(stub=stub, root=ROOT) + textwrap.dedent(code) + "\nprint('ok')\n"
+    r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), (r.returncode, r.stdout + r.stderr)
+
+
+# one chunk of 2 MiB holds 65,516 nodes' states, 6 tets' subgrid velocities
+# and the error flag, each rounded up to 64 bytes
+@pytest.mark.parametrize("n_nodes", [100, 65516, 65517, 400000])
+def test_read_back_with_another_current_device(stub, n_nodes):
+    """A state is read by a thread whose current device is not the handle's;
+    that device stays the thread's."""
+    _run(stub, f"""
+    g, sol = vms({n_nodes})
+    assert stub.hipSetDevice(1) == 0
+    check(g, sol)
+    assert stub.stub_device() == 1
+    assert stub.hipSetDevice(1) == 0
+    h, hsol = vms({n_nodes})
+    err = []
+    def reader():  # a new thread's current device is 0
+        try:
+            check(h, hsol)
+            assert stub.stub_device() == 0
+        except BaseException as e:
+            err.append(e)
+    t = threading.Thread(target=reader)
+    t.start()
+    t.join()
+    assert not err, err
+    """)
+
+
+# no pinned memory at all, one chunk only, an odd number; no threads, one; pool given back
+@pytest.mark.parametrize("pinned,threads", [(0, 99), (1, 99), (3, 99), (99, 0), (99, 1), (0, 0)])
+@pytest.mark.parametrize("n_nodes", [100, 65516, 65517, 400000])
+def test_read_back_without_pinned_memory_or_threads(stub, n_nodes, pinned, threads):
+    _run(stub, f"""
+    g, sol = vms({n_nodes})
+    stub.stub_limits({pinned}, {threads}, -1)
+    for _ in range(3):
+        check(g, sol)
+    stub.stub_limits(99, 99, -1)
+    femx.set_device_cache(0)
+    check(g, sol)
+    """)
