@@ -1547,6 +1547,9 @@ femx_status supg_enqueue(femx_supg *s, int nsteps) {
   return FEMX_OK;
 }
 
+// The handle's stream waits for its union's work queued so far.
+femx_status union_wait(femx_supg *h);
+
 // Waits for the enqueued steps and applies the exit condition (:1633-1643):
 // when a step's max |u| exceeded it, the later steps did not run and the
 // host counters are rewound to that step.
@@ -1668,6 +1671,13 @@ extern "C" femx_status femx_supg_get_mass(femx_supg *s, double *l_M) {
 
 extern "C" femx_status femx_supg_get_log(femx_supg *s, double *cols19) {
   if (!s || !cols19) return set_error("null argument"), FEMX_ERR_ARG;
+  // a union member's log row comes from the union's stream, and after an exit
+  // this call may write it (supg_finish): the union's work on it comes first
+  // (a member that the exit condition stopped is left alone by later steps)
+  if (s->in_union) {
+    const femx_status w = union_wait(s);
+    if (w != FEMX_OK) return w;
+  }
   if (s->pend_n > 0) {
     const femx_status f = supg_finish(s, nullptr);
     if (f != FEMX_OK && f != FEMX_EXIT_CONDITION) return f;
@@ -1868,6 +1878,15 @@ struct femx_supg_union {
 
 namespace {
 
+femx_status union_wait(femx_supg *h) {
+  hipEvent_t ev = nullptr;
+  FEMX_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  const bool ok = hipEventRecord(ev, h->in_union->st) == hipSuccess && hipStreamWaitEvent(h->st, ev, 0) == hipSuccess;
+  (void)hipEventDestroy(ev);
+  if (!ok) return set_error("hipStreamWaitEvent failed"), FEMX_ERR_HIP;
+  return FEMX_OK;
+}
+
 femx_status supg_union_upload(femx_supg_union *u) {
   const int nm = (int)u->mem.size();
   std::vector<SupgMember> t(nm);
@@ -2021,12 +2040,8 @@ extern "C" int femx_supg_union_left(femx_supg_union *u, femx_supg *h) {
 
 extern "C" femx_status femx_supg_union_remove(femx_supg_union *u, femx_supg *h) {
   if (!u || !h || h->in_union != u) return set_error("handle not in this union"), FEMX_ERR_ARG;
-  // the handle's stream waits for the union's work on it
-  hipEvent_t ev = nullptr;
-  FEMX_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  const bool ok = hipEventRecord(ev, u->st) == hipSuccess && hipStreamWaitEvent(h->st, ev, 0) == hipSuccess;
-  (void)hipEventDestroy(ev);
-  if (!ok) return set_error("hipStreamWaitEvent failed"), FEMX_ERR_HIP;
+  const femx_status w = union_wait(h);
+  if (w != FEMX_OK) return w;
   u->mem.erase(std::find(u->mem.begin(), u->mem.end(), h));
   h->in_union = nullptr;
   h->u_left = 0;

@@ -315,7 +315,8 @@ femx_status femx_supg_finish(femx_supg *s, int *steps_done);
  * femx_supg_finish checks them for the exit condition (a step past one
  * whose max |u| exceeded EXITCOND does not run) and femx_supg_get_state
  * reads the state.  While in a union a handle is not stepped, set, read or
- * switched to diagnostics on its own. */
+ * switched to diagnostics on its own, but for femx_supg_get_log, which waits
+ * for the union's enqueued steps. */
 /* 1 if h can join a union (its options and sizes allow it), else 0. */
 int femx_supg_union_accepts(femx_supg *h);
 femx_status femx_supg_union_create(femx_supg_union **out);

@@ -99,3 +99,31 @@ def test_read_back_without_pinned_memory_or_threads(stub, n_nodes, pinned, threa
     femx.set_device_cache(0)
     check(g, sol)
     """)
+
+
+def test_log_of_a_union_member_waits_for_the_union(stub):
+    """The log row of a handle in a union is written on the union's stream:
+    the read (and what the exit condition adds) on the handle's own stream
+    comes after it."""
+    _run(stub, """
+    m = meshgen.hex_cube(7, 0.0)
+    g = femx.SUPGSolver(femx.DeviceMesh(m), BoundaryConditions(), rho=1.0, mu=0.01, alpha=1.0, cI=4.0, dt=0.01,
+                        precision=femx.FEMX_MIXED)
+    g.set_state(np.zeros((m.n_nodes, 3)))
+    g.step(1)
+    log()
+    g.get_log()
+    own = {l[1] for l in log() if l[0] == "read"}
+    assert len(own) == 1
+    own = own.pop()
+    u = femx.SUPGUnion()
+    u.add(g, 3)
+    u.step(2)
+    union = {l[1] for l in log() if l[0] == "launch"}
+    assert len(union) == 1 and own not in union
+    g.get_log()
+    calls = [l for l in log() if l[1] == own]
+    assert calls[0] == ["wait", own, union.pop()], calls
+    assert calls[1][0] == "read", calls
+    u.remove(g)
+    """)

@@ -199,3 +199,40 @@ def test_supg_union_rejects_non_members(gpu):
         assert not gpu.load().femx_supg_union_accepts(h._h)
         with pytest.raises(gpu.FemxError, match="union members"):
             u.add(h, 2)
+
+
+@pytest.mark.parametrize("exit_step", [None, 4])
+def test_supg_union_member_log(gpu, exit_step):
+    """femx_supg_get_log of a handle in a union: the row of its last enqueued
+    step, or of the one that the exit condition made the last (here the fourth
+    of nine), as of the handle stepped on its own."""
+    m, bc, p = _supg_member(gpu, 6, 1, 100.0)
+    dm = gpu.DeviceMesh(m)
+    if exit_step:
+        # a lid that speeds up linearly, 1 at step 10, so that max |u| passes
+        # the threshold between two steps
+        rows = bc.vel_rows.reshape(-1, 2, 4).copy()
+        rows[:, 0] = 0.0
+        rows[:, 1] = [1.0, 0.0, 0.0, 10.0 * p["dt"]]
+        bc.vel_rows = rows.reshape(-1, 4)
+        p = dict(p, exit_condition=0.1 * (exit_step - 0.5))
+    a, b, c = (gpu.SUPGSolver(dm, bc, precision=gpu.FEMX_MIXED, **p) for _ in range(3))
+    for g in (a, b, c):
+        g.set_state(np.zeros((m.n_nodes, 3)))
+        g.step(1)
+    u = gpu.SUPGUnion()
+    u.add(b, 8)
+    u.add(c, 3)
+    u.step(2)
+    a.step(2)
+    np.testing.assert_array_equal(b.get_log(), a.get_log())
+    u.step(6)
+    a.step(6)
+    ref = a.get_log()
+    assert ref[0] == (exit_step or 9)
+    for _ in range(2):
+        np.testing.assert_array_equal(b.get_log(), ref)
+    u.remove(b)
+    u.remove(c)
+    np.testing.assert_array_equal(b.get_log(), ref)
+    np.testing.assert_array_equal(b.get_state()["sol"], a.get_state()["sol"])
