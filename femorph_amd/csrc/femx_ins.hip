@@ -12,7 +12,8 @@
 //                   inverse and the start of the Krylov solve (x = 0, r = b,
 //                   z = D^-1 b, ||b||^2)
 //   hexa8           (an element has 8 rows and costs 20 times a tet: it is
-//                   formed once)
+//                   formed once), and tet4 meshes with a row too long for one
+//                   wave (row_work)
 //   ins_element     one thread per element: the element matrix and vector,
 //                   scattered straight into the order the gathers read (cpos /
 //                   rpos maps)
@@ -294,6 +295,16 @@ constexpr int RLPR = 8;             // lanes per row
 constexpr int RROWS = 256 / RLPR;   // rows per workgroup pass
 constexpr int RCAP = 24;            // row entries summed in LDS per pass over the row's elements
 constexpr int RGRID = 3072;         // workgroups at most (each takes a contiguous range of rows)
+
+// The most element formations that one lane may have for a row: passes over
+// the row's elements (one per RCAP entries) times the lane's share of them.
+// They are a chain that the launch waits for, 1.28 us each; the element kernel
+// and the gathers take 30 us + 0.19 ns per element, so the limit is where the
+// chain alone takes that long.  Assembly with one node of 128 / 512 elements
+// (48 / 704 formations) among 1.11M tets: 123 / 895 us by rows, 239 / 279 us
+// with the gathers; among 48k tets 70 / 852 us and 44 / 87 us.  Ordinary
+// meshes have 3 to 16.
+inline long row_work(long E) { return 24 + E / 6700; }
 
 // The contributions of one element to the row of its corner a: v[b] += P_a Q_b,
 // R -= P_a R (the sums over the Gauss points of the header).
@@ -878,20 +889,26 @@ void host_pattern(const Mesh &m, const std::vector<int> &n_off, const std::vecto
 
 // The same pattern for ins_rows_tet4, and per corner (in the order of n_slot:
 // by node, ascending element) the places of its element's four nodes in the
-// node's row.  False if a row is too long for 16-bit places.
+// node's row.  False if a row has more than row_work(E) element formations for
+// one of its lanes, all rows together 1.5 times as many as there are corners
+// (the other path's time against 4 E formations by rows is 1.6), or a row is
+// too long for 16-bit places: the mesh then takes the element kernel and the
+// gathers.
 bool host_rows(const Mesh &m, const std::vector<int> &n_off, const std::vector<int> &n_slot,
                std::vector<int> &row_ptr, std::vector<int> &col, std::vector<ushort4> &cpos) {
   const int N = m.N;
   const int *conn = m.h_conn.data();
   constexpr int CH = 4096;  // nodes per work item
-  const long items = (N + CH - 1) / CH;
+  const long items = (N + CH - 1) / CH, most = row_work(m.E);
   std::vector<std::vector<int>> cols(items);
   std::atomic<bool> ok{true};
+  std::atomic<long> formed{0};
   row_ptr.assign(N + 1, 0);
   cpos.resize(n_slot.size());
   parallel_items(items, [&](long c) {
     std::vector<int> buf;
-    for (int r = (int)(c * CH); r < std::min<long>(N, (c + 1) * CH); r++) {
+    long work = 0;
+    for (int r = (int)(c * CH); r < std::min<long>(N, (c + 1) * CH) && ok; r++) {
       buf.assign(1, r);
       for (int j = n_off[r]; j < n_off[r + 1]; j++) {
         const int *q = conn + (n_slot[j] & ~3);
@@ -899,7 +916,9 @@ bool host_rows(const Mesh &m, const std::vector<int> &n_off, const std::vector<i
       }
       std::sort(buf.begin(), buf.end());
       buf.erase(std::unique(buf.begin(), buf.end()), buf.end());
-      if (buf.size() > 65536) ok = false;
+      const long passes = ((long)buf.size() + RCAP - 1) / RCAP, elems = n_off[r + 1] - n_off[r];
+      work += passes * elems;
+      if (buf.size() > 65536 || passes * ((elems + RLPR - 1) / RLPR) > most) ok = false;
       row_ptr[r + 1] = (int)buf.size();
       cols[c].insert(cols[c].end(), buf.begin(), buf.end());
       for (int j = n_off[r]; j < n_off[r + 1]; j++) {
@@ -909,12 +928,14 @@ bool host_rows(const Mesh &m, const std::vector<int> &n_off, const std::vector<i
         cpos[j] = make_ushort4(p[0], p[1], p[2], p[3]);
       }
     }
+    formed += work;
   }, n_slot.size() >= (1u << 16));
+  if (!ok || formed > 6L * m.E) return false;
   for (int r = 0; r < N; r++) row_ptr[r + 1] += row_ptr[r];
   col.resize(row_ptr[N]);
   parallel_items(items, [&](long c) { std::copy(cols[c].begin(), cols[c].end(), col.begin() + row_ptr[c * CH]); },
                  col.size() >= (1u << 16));
-  return ok;
+  return true;
 }
 
 InsConst ins_const(const femx_ins_params &p) {
@@ -1134,16 +1155,15 @@ extern "C" femx_status femx_ins_create(femx_mesh *mesh, const double *el_diff, i
   std::vector<double> iso(E, 0.0);
   const std::vector<int> &ord = m.blk.perm;
   if ((long)ord.size() != E) return ins_fail(s, (set_error("femx_ins_create: mesh has no element order"), FEMX_ERR_ARG));
-  // ins_rows_tet4 (node records below 4 GiB), else the element kernel and the gathers
-  const bool rows = npe == 4 && N < (1 << 27);
+  // ins_rows_tet4 (node records below 4 GiB, no row too long for it), else
+  // the element kernel and the gathers
+  const bool rows = npe == 4 && N < (1 << 27) && host_rows(m, n_off, n_slot, s->h_row_ptr, s->h_col, rcpos);
   auto el_iso = [&](int e) {
     if (!el_diff) return 0.0;
     const double *d = el_diff + 3L * e;
     return sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
   };
   if (rows) {
-    if (!host_rows(m, n_off, n_slot, s->h_row_ptr, s->h_col, rcpos))
-      return ins_fail(s, (set_error("femx_ins_create: a matrix row has more than 65536 entries"), FEMX_ERR_ARG));
     for (int e = 0; e < E; e++) iso[e] = el_iso(e);
     // rows in the order their nodes first appear along the element blocks
     rord.reserve(N);
@@ -1156,6 +1176,7 @@ extern "C" femx_status femx_ins_create(femx_mesh *mesh, const double *el_diff, i
     for (int n = 0; n < N; n++)
       if (!seen[n]) rord.push_back(n);
   } else {
+    std::vector<ushort4>().swap(rcpos);
     std::vector<int> c_idx;
     host_pattern(m, n_off, n_slot, s->h_row_ptr, s->h_col, nz_row, c_ptr, c_idx);
     // where each element value goes: matrix entry contributions and node

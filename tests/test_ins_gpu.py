@@ -207,3 +207,49 @@ def test_stop_at_every_iteration(gpu, cap, restart):
         assert abs(st["rel_residual"] - rr) <= 1e-6 * rr + 1e-12, (st, rr)  # (of ||b||: the systems' rounding)
         x = g.get_system()[4]
         assert rel_l2(x, o.phid_new) <= 1e-9, rel_l2(x, o.phid_new)
+
+
+def _fan(points, seed=0):
+    """Tets (centre, face) over the convex hull of points on a sphere: the
+    centre's row has points + 1 entries."""
+    from scipy.spatial import ConvexHull
+    v = np.random.default_rng(seed).normal(size=(points, 3))
+    v /= np.linalg.norm(v, axis=1)[:, None]
+    x = np.vstack([np.zeros(3), v])
+    conn = np.hstack([np.zeros((2 * points - 4, 1), int), ConvexHull(v).simplices + 1]).astype(np.int32)
+    neg = meshgen._tet_det(meshgen.Mesh(x, conn)) < 0
+    conn[neg, 2], conn[neg, 3] = conn[neg, 3].copy(), conn[neg, 2].copy()
+    return meshgen.Mesh(x, conn)
+
+
+@pytest.mark.parametrize("points,by_rows", [(23, True), (24, True), (30, True), (47, True), (48, False), (258, False),
+                                            (65538, False)])
+def test_assembly_by_row_length(gpu, points, by_rows):
+    """tet4 systems on both sides of the choice between the row kernel (which
+    forms a row's elements once per 24 entries) and the element kernel with
+    the gathers: rows of one pass, of two, too much work for one lane, and
+    more entries than 16-bit places hold.  Both match the oracle to 1e-12 of
+    the largest entry (the sums of the centre's row in the oracle's element
+    order, or in eight lanes' partial sums)."""
+    m = meshgen.tet_fan(7) if points == 65538 else _fan(points)
+    assert m.n_nodes == points + 1
+    rng = np.random.default_rng(points)
+    diff = rng.uniform(0.0, 0.02, (m.n_elems, 3))
+    dn = np.arange(2, min(points, 40), 7, dtype=np.int32)
+    dv = rng.normal(size=(len(dn), 3))
+    vel = rng.normal(size=(m.n_nodes, 3))
+    phi, phid = rng.normal(size=m.n_nodes), rng.normal(size=m.n_nodes)
+    g = gpu.INSSolver(gpu.DeviceMesh(m), el_diff=diff, dir_node=dn, dir_val=dv, tol=1e-8, max_iter=20, **PARAMS)
+    o = INSOracle(m, diff, dn, dv, PARAMS["dt"], PARAMS["alpha_m"], PARAMS["alpha_f"], PARAMS["gamma"], tol=1e-8)
+    g.set_state(phi=phi, phi_dot=phid, vel=vel)
+    o.phi, o.phid, o.vel = phi.copy(), phid.copy(), vel.copy()
+    print("rows of", points + 1, "entries", flush=True)
+    g.kernel_timing(True)
+    g.advdiff_solve()
+    assert ("ins_rows" in g.kernel_times()) == by_rows
+    val, rhs = o.assemble()
+    rp, col, gval, grhs, _ = g.get_system()
+    assert np.array_equal(rp, o.rp) and np.array_equal(col, o.col)
+    assert np.diff(rp).max() == points + 1
+    assert np.abs(gval - val).max() <= 1e-12 * np.abs(val).max()
+    assert np.abs(grhs - rhs).max() <= 1e-12 * np.abs(rhs).max()
