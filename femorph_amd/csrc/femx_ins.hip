@@ -84,6 +84,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Lane i's value (i uniform), in SGPRs.
+__device__ __forceinline__ double read_lane(double v, int i) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffLL), i);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), i);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // Block sums of acc[0..cnt) -> part[i * nb + blockIdx.x] (RT threads).
 template <int J>
 __device__ __forceinline__ void block_store(const double (&acc)[J], int cnt, double *part, int nb) {
@@ -629,40 +637,48 @@ __global__ __launch_bounds__(RT) void gm_spmv(int N, const int *rp, const int *c
 //   mode 0: dots w . v_i
 //   mode 1: h = the dots (H[:, j] = h),  w -= sum_i h_i v_i, dots w . v_i
 //   mode 2: h = the dots (H[:, j] += h), w -= sum_i h_i v_i, ||w||^2, z = D^-1 w
-// The dots of the pass before are summed from pin.
-template <int J>
+//           (LAST)
+// The dots of the pass before are summed from pin.  Bound by the stream of the
+// basis: a row's values are all loaded before the first is used, and the
+// registers are kept to the J sums and J values.  The dots go to SGPRs (read
+// from LDS by every lane they took 2 J VGPRs), and the last pass, which needs
+// one sum, is a kernel of its own (both kinds in one copied the sums): J = 4 /
+// 8 / 16 / 32 39 / 42 / 75 / 140 VGPRs and 8 / 8 / 6 / 3 waves per SIMD against
+// 42 / 74 / 139 / 256 and 8 / 6 / 3 / 1; a pass of a 30-iteration solve, 195k
+// rows 32.8 -> 16.1 us, 913k rows 83.9 -> 30.3 us (16 iterations 26.5 -> 19.9).
+template <int J, bool LAST>
 __global__ __launch_bounds__(RT) void gm_orth(int N, double *w, const double *V, long ldv, int j, GmresState *st,
                                               const double *pin, double *part, int nb, int mode,
                                               const double *dinv, double *z) {
   if (st->cyc_stop) return;
   __shared__ double hs[J];
   if (mode != 0) fin_h(st, pin, nb, j + 1, j, mode - 1, hs);
-  double h[J], acc[J];
+  const int lane = threadIdx.x & 63;
+  const double hl = mode != 0 && lane <= j ? hs[lane] : 0.0;
+  constexpr int NA = LAST ? 1 : J;
+  double h[J], acc[NA];
 #pragma unroll
-  for (int i = 0; i < J; i++) {
-    h[i] = (mode != 0 && i <= j) ? hs[i] : 0.0;
-    acc[i] = 0.0;
-  }
+  for (int i = 0; i < J; i++) h[i] = read_lane(hl, i);
+#pragma unroll
+  for (int i = 0; i < NA; i++) acc[i] = 0.0;
   for (int r = blockIdx.x * RT + threadIdx.x; r < N; r += nb * RT) {
     double v[J];
     double s = w[r];
 #pragma unroll
-    for (int i = 0; i < J; i++)
-      if (i <= j) {
-        v[i] = V[(long)i * ldv + r];
-        s -= h[i] * v[i];
-      }
-    if (mode != 0) w[r] = s;
-    if (mode != 2) {
+    for (int i = 0; i < J; i++) v[i] = i <= j ? V[(long)i * ldv + r] : 0.0;
 #pragma unroll
-      for (int i = 0; i < J; i++)
-        if (i <= j) acc[i] += s * v[i];
-    } else {
+    for (int i = 0; i < J; i++) s -= h[i] * v[i];
+    if (LAST) {
+      w[r] = s;
       acc[0] += s * s;
       z[r] = dinv[r] * s;
+    } else {
+      if (mode != 0) w[r] = s;
+#pragma unroll
+      for (int i = 0; i < NA; i++) acc[i] += s * v[i];
     }
   }
-  block_store<J>(acc, mode == 2 ? 1 : j + 1, part, nb);
+  block_store<NA>(acc, LAST ? 1 : j + 1, part, nb);
 }
 
 // y = H^-1 g on the cycle's upper triangle.
@@ -982,8 +998,9 @@ void launch_resid(femx_ins *s, int force) {
 // Krylov kernels sized for the basis in use: j < J.
 template <int J>
 void orth_j(femx_ins *s, double *w, int j, int mode) {
-  gm_orth<J><<<s->nb, RT, 0, s->st>>>(s->mesh->N, w, s->V.p, s->ldv, j, s->gst.p, orth_part(s, mode > 0 ? mode - 1 : 0),
-                                       orth_part(s, mode), s->nb, mode, s->dinv.p, s->z.p);
+  const auto k = mode == 2 ? gm_orth<J, true> : gm_orth<J, false>;
+  k<<<s->nb, RT, 0, s->st>>>(s->mesh->N, w, s->V.p, s->ldv, j, s->gst.p, orth_part(s, mode > 0 ? mode - 1 : 0),
+                             orth_part(s, mode), s->nb, mode, s->dinv.p, s->z.p);
 }
 void launch_orth(femx_ins *s, double *w, int j, int mode) {
   if (j < 4) orth_j<4>(s, w, j, mode);
