@@ -57,6 +57,23 @@ def test_morph_every_x_count(gpu, nx):
     assert np.abs(got - ref).max() <= 1e-13
 
 
+@pytest.mark.parametrize("n_in", [0, 1, 63, 64, 65, 200, 457])
+def test_morph_waves_outside_the_box(gpu, n_in):
+    """Waves with no point in the box, some and all, and a last wave that is
+    not full (457 = 7 x 64 + 9 points, the first n_in in the box)."""
+    rng = np.random.default_rng(n_in)
+    pts = np.vstack([rng.uniform(0.05, 0.95, (n_in, 3)), rng.uniform(1.05, 3.0, (457 - n_in, 3))])
+    box = ((0.0, 0.0, 0.0), (13, 5, 4), (1.0, 0, 0), (0, 1.0, 0), (0, 0, 1.0))
+    nodes = rng.choice(13 * 5 * 4, size=9, replace=False)
+    vals = rng.uniform(-0.2, 0.2, (9, 3))
+    for q in (pts, pts[::-1]):
+        got = gpu.ffd_morph(*box, nodes, vals, q)
+        ref = oracle.ffd_morph(*box, nodes, vals, q)
+        assert np.abs(got - ref).max() <= 1e-13
+        out = (q > 1.0).all(axis=1)
+        np.testing.assert_array_equal(got[out], ref[out])
+
+
 def test_ffd_driver_end_to_end(gpu, tmp_path):
     """mesh.vtk (tet4) + command file -> morphed VTK whose DXYZ is the
     morph of every node, and one bernsteinGrid_<k>.vtk per box; the model
