@@ -36,10 +36,12 @@ struct FfdDev {
 // component took 13 operations per control point, kept the tables in scratch
 // memory and called pow for every entry: 553 us for 500k points and a 7 x 6
 // x 5 lattice, now 25 (25 TFLOP/s of the 77 the VALU reaches and 1 TB/s: the
-// scalar loads between the rows are what is left).
+// scalar loads between the rows are what is left).  out may be coords: a point
+// is read and written by its own thread (so neither is restrict; the times
+// are the same).
 template <int NX>
-__global__ __launch_bounds__(256) void ffd_morph(int N, const double *__restrict__ coords, FfdDev b,
-                                                 const double *__restrict__ disps, double *__restrict__ out) {
+__global__ __launch_bounds__(256) void ffd_morph(int N, const double *coords, FfdDev b,
+                                                 const double *__restrict__ disps, double *out) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= N) return;
   const double a0 = coords[3L * p] - b.minp[0], a1 = coords[3L * p + 1] - b.minp[1], a2 = coords[3L * p + 2] - b.minp[2];

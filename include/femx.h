@@ -394,8 +394,9 @@ femx_status femx_ffd_morph(const femx_ffd_box *box, int n_points, const double *
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops): femx_ffd_morph of
  * `n_points` DEVICE-resident points, `coords` [n][3] in and `disp` [n][3]
- * out (device pointers), enqueued on `stream` (a hipStream_t; NULL = the
- * null stream) without allocating, copying or synchronising.  The box and
+ * out (device pointers; they may be the same), enqueued on `stream` (a
+ * hipStream_t; NULL = the null stream) without allocating, copying or
+ * synchronising.  The box and
  * its displacement list are host data, at most 64 displaced control points
  * (13 control points per axis, as femx_ffd_morph).  The control-point
  * lattice goes to a fixed device array of 52,728 bytes per GPU, held until

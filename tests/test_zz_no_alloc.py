@@ -75,6 +75,20 @@ def test_noalloc_equals_morph_on_two_calls(gpu):
         hip.free()
 
 
+def test_noalloc_in_place(gpu):
+    """coords and disp may be the same array."""
+    hip = _Hip()
+    try:
+        case = _case(BOX_A, 20001, 64, 3)
+        pts = case[-1]
+        dc = hip.upload(pts)
+        gpu.ffd_morph_noalloc(*case[:-1], len(pts), dc.value, dc.value, None)
+        assert hip.L.hipDeviceSynchronize() == 0
+        assert np.array_equal(hip.download(dc, pts.shape), gpu.ffd_morph(*case))
+    finally:
+        hip.free()
+
+
 def test_noalloc_rejects_sizes_beyond_its_limit(gpu):
     X0, n, S, T, U = BOX_B
     with pytest.raises(gpu.FemxError, match="at most 64"):
