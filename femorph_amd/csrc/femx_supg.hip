@@ -424,7 +424,7 @@ __device__ __forceinline__ T norm2_mul(const T m[3][3], const T u[3]) {
 __device__ __forceinline__ float uni(float v) { return __int_as_float(femx::uni(__float_as_int(v))); }
 template <typename T>
 struct ElemConst {
-  T mu, mu2, mu23, mu43, mu103, rho, alpha, cnu2, nu, f1;  // mu and its multiples by 2, 2/3, -4/3, 10/3
+  T mu, mu2, mu23, mu43, mu103, rho, alpha, cnu, nu, f1;  // mu and its multiples by 2, 2/3, -4/3, 10/3
   int k2, k3, k4;
   __device__ __forceinline__ ElemConst(const SupgConst &k) {
     mu = c(k.mu);
@@ -435,7 +435,7 @@ struct ElemConst {
     rho = c(k.rho);
     alpha = c(k.alpha);
     nu = c((T)k.mu / (T)k.rho);
-    cnu2 = c(k.cI * (k.mu / k.rho) * (k.mu / k.rho));
+    cnu = c(k.cI * (k.mu / k.rho));
     f1 = k.k1 ? rho : (T)0;
     k2 = k.k2;
     k3 = k.k3;
@@ -477,7 +477,8 @@ __device__ __forceinline__ void gauss_point(const ElemConst<T> &k, double dt, co
                                             const StrainConst<T, BHAT> &sc, ElemAcc<T> &s, double *dg, T &f3, T c[3],
                                             T A[3][3]) {
   // eval_stabilization (:336-377), tau without the (2/dt)^2 term
-  const T tau = rsqrt_e(t2 + gg * k.cnu2);
+  // (nu and cI nu apart: cI nu^2 alone leaves FP32's range before the term does)
+  const T tau = rsqrt_e(t2 + (gg * k.nu) * k.cnu);
   const T nuC = recip(trG * tau);
   // eval_bulk_modulus (:382-441): lambda = alpha max(mu/rho, sqrt(u^T G^-1 u))
   const T l2 = sqrt_e(norm2_tmul(J, ul));

@@ -208,6 +208,29 @@ def test_log_columns_from_rest(gpu, kind, precision):
     assert small
 
 
+@pytest.mark.parametrize("kind", ["hexa", "tet"])
+@pytest.mark.parametrize("mu,size", [(1e-21, 1.0), (1e19, 1e5)])
+def test_log_columns_viscosity_range(gpu, kind, mu, size):
+    """FP32 element math where cI nu^2 alone is below (4e-42) or above (4e38)
+    the range of FP32 while cI nu^2 |G|^2, the term of tau it belongs to, is
+    in it: velocities, tau and lambda of the log row from rest within 1e-5 of
+    the oracle's, as test_log_columns_mixed."""
+    m = meshgen.hex_cube(5, 0.0) if kind == "hexa" else meshgen.tet_cube(5, 0.0)
+    bc = meshgen.lid_cavity_bc(m)
+    m = meshgen.Mesh(m.coords * size, m.conn)
+    # the time scale of the faster of convection and diffusion
+    dt = 0.02 * min(size, size * size / mu)
+    params = dict(rho=1.0, mu=mu, alpha=1.0, cI=4.0, dt=0.02 * dt)
+    o, g, _ = _pair(gpu, m, bc, params, np.zeros((m.n_nodes, 3)), (0, int(kind == "hexa"), 1, 1, 1, 1), precision=1)
+    g.set_diagnostics(True)
+    for step in range(3):
+        o.step()
+        g.step()
+        lo, lg = o.get("log"), g.get_log()
+        np.testing.assert_allclose(lg[2:8], lo[2:8], rtol=0, atol=1e-5, err_msg=f"step {step}")
+        np.testing.assert_allclose(lg[8:12], lo[8:12], rtol=1e-5, atol=0, err_msg=f"step {step}")
+
+
 def test_log_lcfl_running_max(gpu):
     """Column 14 (l-CFL) is a running maximum since step 1: the reference sets
     l_CFL_max once before the loop (femSUPGExplicitFluidSolver.cpp:996) and
