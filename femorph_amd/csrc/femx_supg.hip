@@ -621,7 +621,15 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
     // through the local derivatives and 3x3 products per Gauss point.
     const ElemConst<T> kc(k);
     ElemAcc<T> acc = {};
-    double vol, mean_div = 0.0;  // the element's volume and mean divergence
+    double vol;                     // the element's volume
+    const bool writes = side == 0;  // of the element's outputs
+    // compute_pressure of the previous step (:498) from the mean divergence,
+    // stored as soon as it is known: held through the Gauss-point loop, with
+    // the fixed-DOF variants' second field formed behind the velocity's, it
+    // spilled 332 B a lane in FP32 and 400 in FP64
+    auto pressure = [&](double mean_div) {
+      if (PRESS && writes) a.pres[e] = -lam_prev * mean_div;
+    };
     if constexpr (NPE == 8) {
       const T q = S::GP(1, 0);  // 1 / sqrt 3
       // the lane's z direction: the map's handedness, and with it the sign of
@@ -654,19 +662,20 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         av.form(X64, q64, (double)sg);
         vol = av.vol;
         X.from(X64);
+        if constexpr (PSEP) {
+          field(pu, pv, pw, V64);
+          av.dot(V64, q64, P64);
+          pressure(P64[0] + P64[1] + P64[2]);
+        }
         field(su, sv, sw, V64);
         av.dot(V64, q64, P64);
+        if constexpr (!PSEP) pressure(P64[0] + P64[1] + P64[2]);
 #pragma unroll
         for (int b = 0; b < 3; b++) {
           P[b] = (T)P64[b];
           V64.c00[b] += 8.0 * (b == 0 ? su : b == 1 ? sv : sw)[id0];
         }
         V.from(V64);
-        if constexpr (PSEP) {
-          field(pu, pv, pw, V64);
-          av.dot(V64, q64, P64);
-        }
-        mean_div = P64[0] + P64[1] + P64[2];
         if constexpr (BHAT && DYN) {
 #pragma unroll
           for (int b = 0; b < 3; b++) {
@@ -780,9 +789,9 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         for (int b = 0; b < 3; b++)
 #pragma unroll
           for (int r = 0; r < 3; r++) dp += iJ[b][r] * (T)(qs[b][own[r]] - qs[b][own[3]]);
-        mean_div = dp;
+        pressure(dp);
       } else if constexpr (PRESS) {
-        mean_div = div;
+        pressure(div);
       }
       if constexpr (DYN) {
         T gg, trG, K[3][3], cN[4][3];
@@ -824,8 +833,6 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         }
       }
     }
-    const bool writes = side == 0;  // the element's outputs
-    if (PRESS && writes) a.pres[e] = -lam_prev * mean_div;  // compute_pressure of the previous step (:498)
     if (DYN) {
       const double lame = (double)acc.lam_int / vol;  // :1446
       if (writes) {
@@ -922,10 +929,13 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
   if (a.want_row) block_node_store<SB>(nv, nm2[0], a.eblk + (long)row * D_COLS);
 }
 
-// Waves per SIMD: FP32 hexa8 fits three (168 VGPRs) without spills as long as
-// its two Gauss points of one y are not unrolled; four spill 100 B per lane
-// (328 against 270 us at 2.1M hexa).  The others are bound to two (FP64 hexa8
-// spills 148 B).
+// Waves per SIMD: every FP32 hexa8 variant fits three (168 VGPRs) without
+// spills (with diagnostics 0 to 84 B a lane, 116 in the first step without
+// B-hat) as long as its two Gauss points of one y are not unrolled; four spill
+// 100 B per lane (328 against 270 us at 2.1M hexa).  The others are bound to
+// two (FP64 hexa8 spills 84 B with B-hat, 244 with diagnostics, none without
+// either).  A step of 2.1M hexa, FP32 / FP64: plain 281 / 480, fixed DOFs 304 /
+// 530, without B-hat 266 / 390 us.
 #define SUPG_BLOCK_WAVES(T, NPE) (sizeof(T) == 4 && NPE == 8 ? 3 : 2)
 template <typename T, int NPE, bool BHAT, bool DYN, bool PRESS, bool PSEP, bool DIAG>
 __global__ __launch_bounds__(SB, SUPG_BLOCK_WAVES(T, NPE)) void supg_block(SupgArgs<T> a) {
