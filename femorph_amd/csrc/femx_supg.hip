@@ -447,7 +447,25 @@ struct ElemConst {
   }
 };
 
-// Per-thread sums over the Gauss points and the diagnostic columns D_TAU ...
+// A thread's extrema over its Gauss points, from which the columns D_TAU ..
+// D_LCFL are made once: tau, lambda, 1 / el^2 and its products with lambda and
+// u_0^2 (the squared a-CFL); NaN never wins.
+template <typename T>
+struct DiagAcc {
+  T tau[2] = {(T)INFINITY, (T)-INFINITY}, lam[2] = {(T)INFINITY, (T)-INFINITY};
+  double acfl2 = 0.0, el_2 = 0.0, lel_2 = 0.0;
+  __device__ __forceinline__ void columns(double dt, double nu, double *dg) const {
+    dg[0] = fmin(dg[0], (double)tau[0]);
+    dg[1] = fmax(dg[1], (double)tau[1]);
+    dg[D_LAM - D_TAU] = fmin(dg[D_LAM - D_TAU], (double)lam[0]);
+    dg[D_LAM + 1 - D_TAU] = fmax(dg[D_LAM + 1 - D_TAU], (double)lam[1]);
+    dg[D_VCFL - D_TAU] = fmax(dg[D_VCFL - D_TAU], 2.0 * nu * dt * el_2);
+    dg[D_ACFL - D_TAU] = fmax(dg[D_ACFL - D_TAU], dt * sqrt(acfl2));
+    dg[D_LCFL - D_TAU] = fmax(dg[D_LCFL - D_TAU], 2.0 * dt * lel_2);
+  }
+};
+
+// Per-thread sums over the Gauss points.
 template <typename T>
 struct ElemAcc {
   T lam_int, reg;
@@ -472,10 +490,10 @@ struct StrainConst {
 // (lam, f3), c = (u.grad) u, and the matrix A of the node forces A DN_n (f2 S
 // + f4 I: stress and grad-div).
 template <typename T, bool BHAT, bool DIAG>
-__device__ __forceinline__ void gauss_point(const ElemConst<T> &k, double dt, const T ug[3], const T gU[3][3], T div,
-                                            T dv, const T J[3][3], const T ul[3], T t2, T gg, T trG,
-                                            const StrainConst<T, BHAT> &sc, ElemAcc<T> &s, double *dg, T &f3, T c[3],
-                                            T A[3][3]) {
+__device__ __forceinline__ void gauss_point(const ElemConst<T> &k, const T ug[3], const T gU[3][3], T div, T dv,
+                                            const T J[3][3], const T ul[3], T t2, T gg, T trG,
+                                            const StrainConst<T, BHAT> &sc, ElemAcc<T> &s, DiagAcc<T> &dg, T &f3,
+                                            T c[3], T A[3][3]) {
   // eval_stabilization (:336-377), tau without the (2/dt)^2 term
   // (nu and cI nu apart: cI nu^2 alone leaves FP32's range before the term does)
   const T tau = rsqrt_e(t2 + (gg * k.nu) * k.cnu);
@@ -486,28 +504,29 @@ __device__ __forceinline__ void gauss_point(const ElemConst<T> &k, double dt, co
   s.reg += (k.nu > l2) ? (T)1 : (T)2;
   s.lam_int += lam * dv;
   if (DIAG) {
-    // get_el_lengths_from_G (:756-790) and the CFL / tau / lambda extrema
-    // (:1187-1240), in FP64: 2 sqrt(o^T G^-1 o), o = u / |u|.  Of the
-    // direction, not |J^T u| / |u|: ahead of a front that spreads from rest u
-    // falls by orders of magnitude per element, and in T the square of |J^T u|
-    // would be 0 (an infinite CFL) where u is not
-    const double u0 = ug[0], u1 = ug[1], u2 = ug[2];
-    const double un = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
-    const double o[3] = {(double)ul[0] / un, (double)ul[1] / un, (double)ul[2] / un};
-    double Jd[3][3];
+    // get_el_lengths_from_G (:756-790), el = 2 sqrt(o^T G^-1 o), o = u / |u|, and
+    // the CFL extrema (:1187-1240), in FP64.  Ahead of a front that spreads from
+    // rest u falls by orders of magnitude per element: the squares of FP32
+    // values are all in FP64's range, FP64 values are scaled into it
+    double w[3] = {(double)ul[0], (double)ul[1], (double)ul[2]}, Jd[3][3];
+    if constexpr (sizeof(T) == 8) {
+      const double f = fmax(fmax(fabs(w[0]), fabs(w[1])), fabs(w[2])) < 0x1p-400 ? 0x1p+700 : 1.0;
+#pragma unroll
+      for (int b = 0; b < 3; b++) w[b] *= f;
+    }
 #pragma unroll
     for (int r = 0; r < 3; r++)
 #pragma unroll
       for (int b = 0; b < 3; b++) Jd[r][b] = (double)J[r][b];
-    const double el = 2.0 * sqrt(norm2_tmul(Jd, o));
-    const double nk = k.nu, lm = lam, ta = tau;
-    dg[D_ACFL - D_TAU] = fmax(dg[D_ACFL - D_TAU], fabs(u0 * dt) / el);
-    dg[D_VCFL - D_TAU] = fmax(dg[D_VCFL - D_TAU], 2.0 * nk * (dt / (el * el)));
-    dg[D_LCFL - D_TAU] = fmax(dg[D_LCFL - D_TAU], 2.0 * lm * (dt / (el * el)));
-    dg[0] = fmin(dg[0], ta);
-    dg[1] = fmax(dg[1], ta);
-    dg[2] = fmin(dg[2], lm);
-    dg[3] = fmax(dg[3], lm);
+    const double el_2 = (w[0] * w[0] + w[1] * w[1] + w[2] * w[2]) / (4.0 * norm2_tmul(Jd, w));  // 1 / el^2
+    const double u0 = (double)ul[0];
+    dg.acfl2 = fmax(dg.acfl2, u0 * u0 * el_2);
+    dg.el_2 = fmax(dg.el_2, el_2);
+    dg.lel_2 = fmax(dg.lel_2, (double)lam * el_2);
+    dg.tau[0] = fmin(dg.tau[0], tau);
+    dg.tau[1] = fmax(dg.tau[1], tau);
+    dg.lam[0] = fmin(dg.lam[0], lam);
+    dg.lam[1] = fmax(dg.lam[1], lam);
   }
   // (u_g . grad) u
 #pragma unroll
@@ -577,9 +596,6 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
   // the thread's nodes: its element's, or those of its side, and node 0
   int own[EN], id0 = 0;
   ushort4 ps4 = make_ushort4(0, 0, 0, 0);
-  double dg[11];
-#pragma unroll
-  for (int i = 0; i < 11; i++) dg[i] = d_identity(D_TAU + i);
   double lam_prev = 0.0;
   if (has_e) {
     const uchar4 c4 = reinterpret_cast<const uchar4 *>(a.lconn)[NPE == 8 ? 2 * e + side : e];
@@ -610,6 +626,9 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
   }
   if (halt_step < a.step_id) return;
   __syncthreads();
+  double dg[11];
+#pragma unroll
+  for (int i = 0; i < 11; i++) dg[i] = d_identity(D_TAU + i);
   if (has_e) {
     const SupgConst &k = a.k;
     using S = ShapeT<T, NPE>;
@@ -621,12 +640,16 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
     // through the local derivatives and 3x3 products per Gauss point.
     const ElemConst<T> kc(k);
     ElemAcc<T> acc = {};
+    DiagAcc<T> da;
     double vol;                     // the element's volume
     const bool writes = side == 0;  // of the element's outputs
     // compute_pressure of the previous step (:498) from the mean divergence,
     // stored as soon as it is known: held through the Gauss-point loop, with
     // the fixed-DOF variants' second field formed behind the velocity's, it
-    // spilled 332 B a lane in FP32 and 400 in FP64
+    // spilled 332 B a lane in FP32 and 400 in FP64.  (FP64 without B-hat or
+    // fixed DOFs fits with it: 386 against 391 us at 2.1M hexa)
+    constexpr bool PHOLD = sizeof(T) == 8 && NPE == 8 && !BHAT && !PSEP;
+    double div_held = 0.0;
     auto pressure = [&](double mean_div) {
       if (PRESS && writes) a.pres[e] = -lam_prev * mean_div;
     };
@@ -669,7 +692,8 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         }
         field(su, sv, sw, V64);
         av.dot(V64, q64, P64);
-        if constexpr (!PSEP) pressure(P64[0] + P64[1] + P64[2]);
+        if constexpr (PHOLD) div_held = P64[0] + P64[1] + P64[2];
+        else if constexpr (!PSEP) pressure(P64[0] + P64[1] + P64[2]);
 #pragma unroll
         for (int b = 0; b < 3; b++) {
           P[b] = (T)P64[b];
@@ -717,8 +741,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
             // the metric's products with u pair the physical components with
             // the local directions, as the reference does
             const T ul[3] = {ug[0], ug[1], sg * ug[2]};
-            gauss_point<T, BHAT, DIAG>(kc, k.dt, ug, gU, div, dv, J, ul, norm2_mul(iJ, ul), gg, trG, sc, acc, dg, f3,
-                                       c, A);
+            gauss_point<T, BHAT, DIAG>(kc, ug, gU, div, dv, J, ul, norm2_mul(iJ, ul), gg, trG, sc, acc, da, f3, c, A);
             const T f1 = kc.f1 * dv;
             // A DN_n + f3 c (u.grad N_n) in the local derivatives:
             // (A + f3 c (x) u) invJ dN_n
@@ -809,8 +832,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
 #pragma unroll
           for (int b = 0; b < 3; b++)
             ug[b] = U0[b] + (S::N(g, 1) * u[1][b] + S::N(g, 2 % NPE) * u[2][b] + S::N(g, 3 % NPE) * u[3][b]);
-          gauss_point<T, false, DIAG>(kc, k.dt, ug, gU, div, dv, J, ug, norm2_mul(iJ, ug), gg, trG, sc, acc, dg, f3, c,
-                                      A);
+          gauss_point<T, false, DIAG>(kc, ug, gU, div, dv, J, ug, norm2_mul(iJ, ug), gg, trG, sc, acc, da, f3, c, A);
           const T f1 = kc.f1 * dv;
 #pragma unroll
           for (int i = 0; i < 3; i++) {
@@ -833,6 +855,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         }
       }
     }
+    if constexpr (PHOLD) pressure(div_held);
     if (DYN) {
       const double lame = (double)acc.lam_int / vol;  // :1446
       if (writes) {
@@ -840,6 +863,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
         a.regime[e] = (double)acc.reg / NGP;
       }
       if (DIAG) {
+        da.columns(k.dt, (double)kc.nu, dg);
         const double cE = (k.mu * (3 * lame + 2 * k.mu)) / (lame + k.mu), cnu = lame / (2 * (lame + k.mu));
         dg[D_E - D_TAU] = fmin(dg[D_E - D_TAU], cE);
         dg[D_E + 1 - D_TAU] = fmax(dg[D_E + 1 - D_TAU], cE);
@@ -930,12 +954,12 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
 }
 
 // Waves per SIMD: every FP32 hexa8 variant fits three (168 VGPRs) without
-// spills (with diagnostics 0 to 84 B a lane, 116 in the first step without
+// spills (with diagnostics 0 to 20 B a lane, 68 in the first step without
 // B-hat) as long as its two Gauss points of one y are not unrolled; four spill
 // 100 B per lane (328 against 270 us at 2.1M hexa).  The others are bound to
-// two (FP64 hexa8 spills 84 B with B-hat, 244 with diagnostics, none without
-// either).  A step of 2.1M hexa, FP32 / FP64: plain 281 / 480, fixed DOFs 304 /
-// 530, without B-hat 266 / 390 us.
+// two (FP64 hexa8 spills 84 B with B-hat, 156 with diagnostics, none without
+// either).  A step of 2.1M hexa, FP32 / FP64: plain 278 / 478, fixed DOFs 302 /
+// 527, without B-hat 265 / 386, plain with diagnostics 388 / 741 us.
 #define SUPG_BLOCK_WAVES(T, NPE) (sizeof(T) == 4 && NPE == 8 ? 3 : 2)
 template <typename T, int NPE, bool BHAT, bool DYN, bool PRESS, bool PSEP, bool DIAG>
 __global__ __launch_bounds__(SB, SUPG_BLOCK_WAVES(T, NPE)) void supg_block(SupgArgs<T> a) {
