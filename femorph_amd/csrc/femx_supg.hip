@@ -505,20 +505,25 @@ __device__ __forceinline__ void gauss_point(const ElemConst<T> &k, const T ug[3]
   s.lam_int += lam * dv;
   if (DIAG) {
     // get_el_lengths_from_G (:756-790), el = 2 sqrt(o^T G^-1 o), o = u / |u|, and
-    // the CFL extrema (:1187-1240), in FP64.  Ahead of a front that spreads from
-    // rest u falls by orders of magnitude per element: the squares of FP32
-    // values are all in FP64's range, FP64 values are scaled into it
+    // the CFL extrema (:1187-1240), in FP64, as 1 / el^2 = |u|^2 / (4 |J^T u|^2).
+    // Ahead of a front that spreads from rest u falls by orders of magnitude
+    // per element: the squares of FP32 values are all in FP64's range, FP64
+    // values are scaled into it for |J^T u|^2 (but not for |u|^2: below 1e-154
+    // the reference's lengths are off by its rounding, and so are these)
     double w[3] = {(double)ul[0], (double)ul[1], (double)ul[2]}, Jd[3][3];
-    if constexpr (sizeof(T) == 8) {
-      const double f = fmax(fmax(fabs(w[0]), fabs(w[1])), fabs(w[2])) < 0x1p-400 ? 0x1p+700 : 1.0;
-#pragma unroll
-      for (int b = 0; b < 3; b++) w[b] *= f;
-    }
 #pragma unroll
     for (int r = 0; r < 3; r++)
 #pragma unroll
       for (int b = 0; b < 3; b++) Jd[r][b] = (double)J[r][b];
-    const double el_2 = (w[0] * w[0] + w[1] * w[1] + w[2] * w[2]) / (4.0 * norm2_tmul(Jd, w));  // 1 / el^2
+    double un2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2], q = norm2_tmul(Jd, w);
+    if (sizeof(T) == 8 && un2 < 0x1p-800) {
+      constexpr double f = 0x1p+700;
+#pragma unroll
+      for (int b = 0; b < 3; b++) w[b] *= f;
+      un2 = un2 * f * f;
+      q = norm2_tmul(Jd, w);
+    }
+    const double el_2 = un2 / (4.0 * q);
     const double u0 = (double)ul[0];
     dg.acfl2 = fmax(dg.acfl2, u0 * u0 * el_2);
     dg.el_2 = fmax(dg.el_2, el_2);
@@ -959,7 +964,7 @@ __device__ __forceinline__ void supg_block_run(const SupgArgs<T> &a, const int b
 // 100 B per lane (328 against 270 us at 2.1M hexa).  The others are bound to
 // two (FP64 hexa8 spills 84 B with B-hat, 156 with diagnostics, none without
 // either).  A step of 2.1M hexa, FP32 / FP64: plain 278 / 478, fixed DOFs 302 /
-// 527, without B-hat 265 / 386, plain with diagnostics 388 / 741 us.
+// 527, without B-hat 265 / 386, plain with diagnostics 388 / 755 us.
 #define SUPG_BLOCK_WAVES(T, NPE) (sizeof(T) == 4 && NPE == 8 ? 3 : 2)
 template <typename T, int NPE, bool BHAT, bool DYN, bool PRESS, bool PSEP, bool DIAG>
 __global__ __launch_bounds__(SB, SUPG_BLOCK_WAVES(T, NPE)) void supg_block(SupgArgs<T> a) {

@@ -209,6 +209,30 @@ def test_log_columns_from_rest(gpu, kind, precision):
 
 
 @pytest.mark.parametrize("kind", ["hexa", "tet"])
+def test_log_columns_below_the_range_of_squares(gpu, kind):
+    """FP64 from rest with so small a time step that the front falls by ten
+    orders of magnitude per layer, to 1e-160: |J^T u|^2 is 0 there, |u|^2 a few
+    thousand units of the smallest number.  All columns within 1e-12 of the
+    oracle's but the v-CFL, 1e-3 (four of those units)."""
+    n = 16
+    m = meshgen.hex_cube(n, 0.0) if kind == "hexa" else meshgen.tet_cube(n, 0.0)
+    params = dict(rho=1.0, mu=0.0025, alpha=1.0, cI=4.0, dt=2e-10 / n)
+    o, g, _ = _pair(gpu, m, meshgen.lid_cavity_bc(m), params, np.zeros((m.n_nodes, 3)),
+                    (0, int(kind == "hexa"), 1, 1, 1, 1))
+    g.set_diagnostics(True)
+    for step in range(17):
+        o.step()
+        g.step()
+        lo, lg = o.get("log"), g.get_log()
+        np.testing.assert_allclose(lg[2:8], lo[2:8], rtol=0, atol=TOL64, err_msg=f"step {step}")
+        np.testing.assert_allclose(lg[12], lo[12], rtol=1e-3, atol=0, err_msg=f"step {step}")
+        cols = [c for c in range(8, 19) if c != 12]
+        np.testing.assert_allclose(lg[cols], lo[cols], rtol=TOL64, atol=0, err_msg=f"step {step}")
+    u = np.abs(o.get("sol_n")).max(axis=1)
+    assert ((u > 1e-162) & (u < 1e-154)).any()
+
+
+@pytest.mark.parametrize("kind", ["hexa", "tet"])
 @pytest.mark.parametrize("mu,size", [(1e-21, 1.0), (1e19, 1e5)])
 def test_log_columns_viscosity_range(gpu, kind, mu, size):
     """FP32 element math where cI nu^2 alone is below (4e-42) or above (4e38)
