@@ -7,7 +7,6 @@
 #include <cstring>
 #include <map>
 #include <numeric>
-#include <system_error>
 #include <thread>
 
 #include "femx_common.h"
@@ -187,10 +186,13 @@ struct Pin {
 
 struct PinPool {
   std::mutex mu;
-  std::vector<Pin> idle[CACHE_DEVICES];
+  Pin idle[CACHE_DEVICES][PIN_IDLE];
+  size_t n_idle[CACHE_DEVICES] = {};
 };
 PinPool &pins() {
-  static PinPool *p = new PinPool();  // never destroyed, as the device cache
+  // never destroyed, as the device cache; no allocation, which could fail
+  alignas(PinPool) static unsigned char room[sizeof(PinPool)];
+  static PinPool *p = new (room) PinPool();
   return *p;
 }
 
@@ -203,10 +205,8 @@ void pin_free(Pin &c) {
 hipError_t pin_get(int d, Pin &c) {
   {
     std::lock_guard<std::mutex> lk(pins().mu);
-    auto &v = pins().idle[d];
-    if (!v.empty()) {
-      c = v.back();
-      v.pop_back();
+    if (pins().n_idle[d] > 0) {
+      c = pins().idle[d][--pins().n_idle[d]];
       return hipSuccess;
     }
   }
@@ -220,44 +220,57 @@ void pin_put(int d, Pin &c) {
   if (!c.p) return;
   {
     std::lock_guard<std::mutex> lk(pins().mu);
-    if (pins().idle[d].size() < PIN_IDLE) {
-      pins().idle[d].push_back(c);
+    if (pins().n_idle[d] < PIN_IDLE) {
+      pins().idle[d][pins().n_idle[d]++] = c;
       return;
     }
   }
   pin_free(c);
 }
 
-// Pieces of at most one chunk, taken from a shared counter: the thread's two
-// chunks alternate, so that the next piece is in flight while one is copied
+// The k-th piece of at most one chunk of p[0 .. n); false past the last.
+bool piece(const ReadPiece *p, int n, size_t k, ReadPiece &q) {
+  for (int i = 0; i < n; i++) {
+    const size_t m = (p[i].bytes + PIN_CHUNK - 1) / PIN_CHUNK;
+    if (k < m) {
+      const size_t o = k * PIN_CHUNK;
+      q = {(unsigned char *)p[i].dst + o, (const unsigned char *)p[i].src + o, std::min(PIN_CHUNK, p[i].bytes - o)};
+      return true;
+    }
+    k -= m;
+  }
+  return false;
+}
+
+// Pieces taken from a shared counter: the thread's two chunks alternate, so that the next piece is in flight while one is copied
 // out.  Where no pinned memory is to be had the pieces are copied directly.
-hipError_t read_pieces(hipStream_t st, int d, const std::vector<ReadPiece> &q, std::atomic<size_t> &next) {
+hipError_t read_pieces(hipStream_t st, int d, const ReadPiece *p, int n, std::atomic<size_t> &next) {
   Pin c[2];
-  size_t in_c[2] = {0, 0};
+  ReadPiece in_c[2], q;
   bool busy[2] = {false, false};
   hipError_t e = hipSetDevice(d);
   const bool pinned = e == hipSuccess && pin_get(d, c[0]) == hipSuccess && pin_get(d, c[1]) == hipSuccess;
   if (e == hipSuccess && !pinned) {
     (void)hipGetLastError();
-    for (size_t k; e == hipSuccess && (k = next.fetch_add(1)) < q.size();)
-      e = hipMemcpyAsync(q[k].dst, q[k].src, q[k].bytes, hipMemcpyDeviceToHost, st);
+    while (e == hipSuccess && piece(p, n, next.fetch_add(1), q))
+      e = hipMemcpyAsync(q.dst, q.src, q.bytes, hipMemcpyDeviceToHost, st);
   }
   for (int i = 0; pinned && e == hipSuccess; i ^= 1) {
     // queue the next piece into chunk i, then drain the other one
-    const size_t k = next.fetch_add(1);
-    if (k < q.size()) {
-      e = hipMemcpyAsync(c[i].p, q[k].src, q[k].bytes, hipMemcpyDeviceToHost, st);
+    const bool more = piece(p, n, next.fetch_add(1), q);
+    if (more) {
+      e = hipMemcpyAsync(c[i].p, q.src, q.bytes, hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipEventRecord(c[i].ev, st);
       if (e != hipSuccess) break;
-      in_c[i] = k;
+      in_c[i] = q;
       busy[i] = true;
     }
     const int o = i ^ 1;
     if (busy[o]) {
       e = hipEventSynchronize(c[o].ev);
-      if (e == hipSuccess) std::memcpy(q[in_c[o]].dst, c[o].p, q[in_c[o]].bytes);
+      if (e == hipSuccess) std::memcpy(in_c[o].dst, c[o].p, in_c[o].bytes);
       busy[o] = false;
-    } else if (k >= q.size()) {
+    } else if (!more) {
       break;
     }
   }
@@ -306,22 +319,22 @@ femx_status read_back(hipStream_t st, const ReadPiece *p, int n) {
     FEMX_HIP(e);
     return FEMX_OK;
   }
-  std::vector<ReadPiece> q;
-  for (int i = 0; i < n; i++)
-    for (size_t o = 0; o < p[i].bytes; o += PIN_CHUNK)
-      q.push_back({(unsigned char *)p[i].dst + o, (const unsigned char *)p[i].src + o,
-                   std::min(PIN_CHUNK, p[i].bytes - o)});
-  const int h = q.size() < 4 ? 0 : take_helpers((int)std::min<size_t>(7, q.size() / 2 - 1));
+  // (no exception leaves this function, and none a helper thread: a piece's
+  // place is found from its number, nothing is allocated but the threads)
+  size_t pieces = 0;
+  for (int i = 0; i < n; i++) pieces += (p[i].bytes + PIN_CHUNK - 1) / PIN_CHUNK;
+  constexpr int HELPERS = 7;
+  const int h = pieces < 4 ? 0 : take_helpers((int)std::min<size_t>(HELPERS, pieces / 2 - 1));
   std::atomic<size_t> next{0};
-  std::vector<hipError_t> err(h + 1, hipSuccess);
-  std::vector<std::thread> th;
+  hipError_t err[HELPERS + 1] = {};
+  std::thread th[HELPERS];
   try {
-    th.reserve(h);
-    for (int t = 1; t <= h; t++) th.emplace_back([&, t] { err[t] = read_pieces(st, d, q, next); });
-  } catch (const std::system_error &) {  // fewer threads, the same pieces
+    for (int t = 0; t < h; t++) th[t] = std::thread([&, t] { err[t + 1] = read_pieces(st, d, p, n, next); });
+  } catch (const std::exception &) {  // no thread or no memory for it: fewer threads, the same pieces
   }
-  err[0] = read_pieces(st, d, q, next);
-  for (auto &x : th) x.join();
+  err[0] = read_pieces(st, d, p, n, next);
+  for (auto &x : th)
+    if (x.joinable()) x.join();
   if (h) give_helpers(h);
   for (hipError_t e : err) FEMX_HIP(e);
   FEMX_HIP(hipStreamSynchronize(st));
@@ -926,17 +939,17 @@ extern "C" femx_status femx_set_device_cache(size_t max_bytes_per_device) {
   }
   for (void *p : idle) (void)hipFree(p);
   for (hipStream_t st : streams) (void)hipStreamDestroy(st);
-  if (max_bytes_per_device == 0) {
-    std::vector<Pin> chunks;
-    {
-      std::lock_guard<std::mutex> lk(pins().mu);
-      for (auto &v : pins().idle) {
-        chunks.insert(chunks.end(), v.begin(), v.end());
-        v.clear();
+  if (max_bytes_per_device == 0)
+    for (int d = 0; d < CACHE_DEVICES; d++)
+      for (;;) {
+        Pin c;
+        {
+          std::lock_guard<std::mutex> lk(pins().mu);
+          if (pins().n_idle[d] == 0) break;
+          c = pins().idle[d][--pins().n_idle[d]];
+        }
+        pin_free(c);
       }
-    }
-    for (Pin &c : chunks) pin_free(c);
-  }
   return FEMX_OK;
 }
 

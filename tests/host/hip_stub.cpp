@@ -11,7 +11,6 @@
 #include <memory>
 #include <mutex>
 #include <new>
-#include <string>
 #include <system_error>
 #include <thread>
 
@@ -27,7 +26,13 @@ thread_local int g_device = 0;
 std::atomic<int> g_streams{0}, g_pinned{1 << 30}, g_threads{1 << 30};
 std::atomic<long> g_new_max{-1};
 std::mutex g_mu;
-std::string g_log;
+char g_log[1 << 20];
+int g_log_len = 0;
+// (the runtime's own objects come from malloc: its memory does not run out)
+template <typename T>
+T *make(T v) {
+  return static_cast<T *>(memcpy(malloc(sizeof(T)), &v, sizeof(T)));
+}
 Stream *S(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
 Event *E(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
 void note(const char *what, hipStream_t s, int other = -1) {
@@ -35,7 +40,8 @@ void note(const char *what, hipStream_t s, int other = -1) {
   if (other >= 0) snprintf(b, sizeof(b), "%s %d %d\n", what, s ? S(s)->id : 0, other);
   else snprintf(b, sizeof(b), "%s %d\n", what, s ? S(s)->id : 0);
   std::lock_guard<std::mutex> lk(g_mu);
-  g_log += b;
+  const int n = (int)strlen(b);
+  if (g_log_len + n < (int)sizeof(g_log)) memcpy(g_log + g_log_len, b, n + 1), g_log_len += n;
 }
 bool take(std::atomic<int> &left) {
   if (left.load() <= 0) return false;
@@ -54,9 +60,10 @@ void stub_limits(int pinned, int threads, long new_max) {
 }
 int stub_log(char *out, int n) {
   std::lock_guard<std::mutex> lk(g_mu);
-  const int len = (int)g_log.size();
-  snprintf(out, n, "%s", g_log.c_str());
-  g_log.clear();
+  const int len = g_log_len;
+  snprintf(out, n, "%s", g_log);
+  g_log_len = 0;
+  g_log[0] = 0;
   return len;
 }
 int stub_device() { return g_device; }
@@ -84,9 +91,9 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { return memset(d, v, n), hipSuccess; }
 hipError_t hipMemcpyToSymbol(const void *, const void *, size_t, size_t, hipMemcpyKind) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
-  return *s = reinterpret_cast<hipStream_t>(new Stream{g_device, ++g_streams}), hipSuccess;
+  return *s = reinterpret_cast<hipStream_t>(make(Stream{g_device, ++g_streams})), hipSuccess;
 }
-hipError_t hipStreamDestroy(hipStream_t s) { return delete S(s), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { return free(S(s)), hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d) { return *d = s ? S(s)->device : g_device, hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
@@ -94,10 +101,10 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
-  return *e = reinterpret_cast<hipEvent_t>(new Event{g_device, nullptr}), hipSuccess;
+  return *e = reinterpret_cast<hipEvent_t>(make(Event{g_device, nullptr})), hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
-hipError_t hipEventDestroy(hipEvent_t e) { return delete E(e), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return free(E(e)), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   if (E(e)->device != (s ? S(s)->device : g_device)) return hipErrorInvalidHandle;
   return E(e)->recorded = S(s), hipSuccess;

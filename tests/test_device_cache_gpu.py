@@ -84,8 +84,9 @@ def test_cached_buffers_give_the_same_results(gpu):
 
 @pytest.mark.parametrize("n", [3, 43, 44, 90])
 def test_read_back_round_trips(gpu, n):
-    """States of one pinned chunk (2 MiB) or less, just above, and of many
-    chunks (several host threads) come back exactly as they were set."""
+    """States of one pinned chunk (2 MiB) or less, of a few chunks (4 and 5 MB:
+    one thread) and of many (several host threads) come back exactly as they
+    were set."""
     m = meshgen.hex_cube(n, 0.0)
     rng = np.random.default_rng(n)
     dm = gpu.DeviceMesh(m)
@@ -105,3 +106,22 @@ def test_read_back_round_trips(gpu, n):
     gpu.set_device_cache(0)  # gives the idle chunks back
     gpu.set_device_cache(CAP)
     np.testing.assert_array_equal(g.get_state()["sol"], sol)
+
+
+@pytest.mark.parametrize("n_nodes", [65515, 65516, 65517, 196608, 262144])
+def test_read_back_at_the_chunk_borders(gpu, n_nodes):
+    """The state, six tets' subgrid velocities (576 bytes) and the error flag,
+    each rounded up to 64 bytes, in one chunk of 2 MiB: 65,516 nodes fill it.
+    Then three and four whole chunks of states (the smallest sizes with a second
+    thread)."""
+    m = meshgen.tet_cube(1)
+    m = meshgen.Mesh(np.vstack([m.coords, np.full((n_nodes - 8, 3), 2.0)]), m.conn)  # nodes of no element
+    g = gpu.VMSSolver(gpu.DeviceMesh(m), meshgen.BoundaryConditions(), rho=1.0, mu=0.01, inv_eps=1.0, c1=4.0, c2=2.0,
+                      dt=0.01)
+    rng = np.random.default_rng(n_nodes)
+    sol, sdus = rng.normal(size=(n_nodes, 4)), rng.normal(size=12 * m.n_elems)
+    g.set_state(sol, sdus)
+    for _ in range(2):
+        got = g.get_state()
+        np.testing.assert_array_equal(got[0], sol)
+        np.testing.assert_array_equal(np.ravel(got[1]), sdus)

@@ -127,3 +127,21 @@ def test_log_of_a_union_member_waits_for_the_union(stub):
     assert calls[1][0] == "read", calls
     u.remove(g)
     """)
+
+
+@pytest.mark.parametrize("n_nodes", [100, 65516, 65517, 400000])
+def test_read_back_without_host_memory(stub, n_nodes):
+    """No exception for want of host memory leaves a C entry or ends a helper
+    thread: the state comes back all the same."""
+    _run(stub, f"""
+    g, sol = vms({n_nodes})
+    out = np.zeros_like(sol)
+    read = lambda: femx.load().femx_vms_get_state(g._h, out.ctypes.data_as(C.POINTER(C.c_double)), None, None)
+    for _ in range(3):
+        stub.stub_limits(99, 99, 0)
+        status = read()
+        stub.stub_limits(99, 99, -1)
+        assert status == 0
+        np.testing.assert_array_equal(out, sol)
+        out[:] = 0.0
+    """)
