@@ -142,9 +142,9 @@ struct DeviceGuard {
 
 // ------------------------------------------------------------ read-back
 // Copies device arrays to the caller's (pageable) host arrays after the work
-// queued on st, and waits for them.  A plain hipMemcpy to pageable memory
-// blocks per array and moves about 4 (several outputs repacked on the host)
-// to 15 GB/s; here the arrays pass through a few pinned chunks: small ones
+// queued on st (a stream of device), and waits for them.  A plain hipMemcpy to
+// pageable memory blocks per array and moves about 4 (several outputs repacked
+// on the host) to 15 GB/s; here the arrays pass through a few pinned chunks: small ones
 // all together under one wait, large ones by several host threads, each
 // moving its chunks' bytes to the caller while the other threads' chunks are
 // in flight.  The chunks come from a bounded per-device pool shared by all
@@ -154,7 +154,7 @@ struct ReadPiece {
   const void *src;
   size_t bytes;
 };
-femx_status read_back(hipStream_t st, const ReadPiece *p, int n);
+femx_status read_back(int device, hipStream_t st, const ReadPiece *p, int n);
 
 // -------------------------------------------------------------- the mesh
 // Device layout (one MI355X holds meshes of tens of millions of elements):

@@ -281,13 +281,11 @@ hipError_t read_pieces(hipStream_t st, int d, const ReadPiece *p, int n, std::at
 }
 }  // namespace
 
-femx_status read_back(hipStream_t st, const ReadPiece *p, int n) {
+femx_status read_back(int d, hipStream_t st, const ReadPiece *p, int n) {
   size_t total = 0;
   for (int i = 0; i < n; i++) total += (p[i].bytes + 63) & ~size_t(63);
   // chunks and events of the stream's device, whatever the caller's current
   // one is: an event is recorded on streams of its own device only
-  int d = 0;
-  FEMX_HIP(hipStreamGetDevice(st, &d));
   const DeviceGuard guard(d);
   Pin c;
   bool direct = d < 0 || d >= CACHE_DEVICES;

@@ -1375,7 +1375,7 @@ extern "C" femx_status femx_ins_get_state(femx_ins *s, double *phi, double *phi_
   if (phi) rb[nrb++] = {phi, dphi, sizeof(double) * N};
   if (vel) rb[nrb++] = {vel, dvel, sizeof(double) * 3 * N};
   if (phi_dot) rb[nrb++] = {phi_dot, s->phid.p, sizeof(double) * N};
-  return read_back(s->st, rb, nrb);
+  return read_back(s->mesh->device, s->st, rb, nrb);
 }
 
 extern "C" femx_status femx_ins_get_system(femx_ins *s, int *row_ptr, int *col, double *val, double *rhs,

@@ -1455,7 +1455,7 @@ femx_status flush_pressure(femx_supg *s) {
 femx_status read_checked(femx_supg *s, ReadPiece *p, int n) {
   int e = 0;
   p[n] = {&e, s->bc.err.p, sizeof(int)};
-  const femx_status r = read_back(s->st, p, n + 1);
+  const femx_status r = read_back(s->mesh->device, s->st, p, n + 1);
   if (r != FEMX_OK) return r;
   if (e) return set_error("Could not find time in femUtils::interpTableData."), FEMX_ERR_BC;
   return FEMX_OK;
