@@ -116,9 +116,9 @@ __device__ __forceinline__ void block_store(const double (&acc)[J], int cnt, dou
 __device__ __forceinline__ double wave_total(const double *part, int i, int nb) {
   const int lane = threadIdx.x & 63;
   const double *p = part + (long)i * nb;
-  // per chunk of 1024 partials: all loads first, then the lane's sum in the
+  // per chunk of 64 K partials: all loads first, then the lane's sum in the
   // order b = lane, lane + 64, ... (any nb: the solve's first reduction has
-  // one partial per block of all rows)
+  // one partial per workgroup of its kernel)
   constexpr int K = MAXNB / 64;
   double s = 0.0;
   for (int c0 = 0; c0 < nb; c0 += 64 * K) {
