@@ -1672,28 +1672,46 @@ extern "C" femx_status femx_supg_get_state(femx_supg *s, double *sol, double *pr
   femx_status r = flush_pressure(s);
   if (r != FEMX_OK) return r;
   // what is asked for, in the caller's layouts, in one staging array kept by
-  // the handle: [N][3] then E values per element field
+  // the handle: [N][3] then E values per element field.  Where the device has
+  // no room for it, the state is packed on the host and the fields pass through
+  // an array of E values one by one
+  double *outs[3] = {pres, lam, regime};
+  DevBuf<double> *srcs[3] = {&s->pres, &s->lam, &s->regime};
   size_t len = 0, off = 0;
-  for (double *o : {pres, lam, regime}) len += o ? m.E : 0;
+  for (double *o : outs) len += o ? m.E : 0;
   len += sol ? 3 * (size_t)m.N : 0;
-  if (s->scratch.n < len && (r = s->scratch.alloc(len)) != FEMX_OK) return r;
+  const bool staged = s->scratch.n >= len || s->scratch.alloc(len) == FEMX_OK;
+  if (!staged) (void)hipGetLastError();
   ReadPiece rb[5];
   int nrb = 0;
-  if (sol) {
+  if (sol && staged) {
     pack3<<<grid_for(3L * m.N, 256), 256, 0, s->st>>>(m.N, reinterpret_cast<const double *>(s->U[s->cur].p),
                                                       s->scratch.p);
     FEMX_HIP(hipGetLastError());
     rb[nrb++] = {sol, s->scratch.p, 3 * (size_t)m.N * sizeof(double)};
     off = 3 * (size_t)m.N;
+  } else if (sol) {
+    std::vector<double4> h(m.N);
+    const ReadPiece all = {h.data(), s->U[s->cur].p, m.N * sizeof(double4)};
+    if ((r = read_back(m.device, s->st, &all, 1)) != FEMX_OK) return r;
+    for (int n = 0; n < m.N; n++) {
+      sol[3L * n] = h[n].x;
+      sol[3L * n + 1] = h[n].y;
+      sol[3L * n + 2] = h[n].z;
+    }
   }
-  double *outs[3] = {pres, lam, regime};
-  DevBuf<double> *srcs[3] = {&s->pres, &s->lam, &s->regime};
   for (int k = 0; k < 3; k++) {
     if (!outs[k]) continue;
+    if (!staged && s->scratch.n < (size_t)m.E && (r = s->scratch.alloc(m.E)) != FEMX_OK) return r;
     block_to_orig<<<grid_for(m.E, 256), 256, 0, s->st>>>(m.E, m.blk.d_perm.p, srcs[k]->p, s->scratch.p + off);
     FEMX_HIP(hipGetLastError());
     rb[nrb++] = {outs[k], s->scratch.p + off, m.E * sizeof(double)};
-    off += m.E;
+    if (staged) {
+      off += m.E;
+    } else {
+      if ((r = read_back(m.device, s->st, rb, nrb)) != FEMX_OK) return r;
+      nrb = 0;
+    }
   }
   if (time) *time = s->time;
   return read_checked(s, rb, nrb);

@@ -24,7 +24,7 @@ struct Event {
 };
 thread_local int g_device = 0;
 std::atomic<int> g_streams{0}, g_pinned{1 << 30}, g_threads{1 << 30};
-std::atomic<long> g_new_max{-1};
+std::atomic<long> g_new_max{-1}, g_device_max{-1};
 std::mutex g_mu;
 char g_log[1 << 20];
 int g_log_len = 0;
@@ -58,6 +58,8 @@ void stub_limits(int pinned, int threads, long new_max) {
   g_threads = threads;
   g_new_max = new_max;
 }
+// the largest device allocation that succeeds (-1: any)
+void stub_device_max(long bytes) { g_device_max = bytes; }
 int stub_log(char *out, int n) {
   std::lock_guard<std::mutex> lk(g_mu);
   const int len = g_log_len;
@@ -76,7 +78,11 @@ hipError_t hipSetDevice(int d) {
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stub error"; }
-hipError_t hipMalloc(void **p, size_t n) { return *p = calloc(n ? n : 1, 1), hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) {
+  const long max = g_device_max.load();
+  if (max >= 0 && n > (size_t)max) return *p = nullptr, hipErrorOutOfMemory;
+  return *p = calloc(n ? n : 1, 1), hipSuccess;
+}
 hipError_t hipFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   if (!take(g_pinned)) return hipErrorOutOfMemory;

@@ -18,6 +18,7 @@ import ctypes as C, sys, threading
 import numpy as np
 stub = C.CDLL({stub!r}, mode=C.RTLD_GLOBAL)
 stub.stub_limits.argtypes = [C.c_int, C.c_int, C.c_long]
+stub.stub_device_max.argtypes = [C.c_long]
 sys.path.insert(0, {root!r})
 from femorph_amd import femx, meshgen
 from femorph_amd.mesh import BoundaryConditions, Mesh
@@ -144,4 +145,31 @@ def test_read_back_without_host_memory(stub, n_nodes):
         assert status == 0
         np.testing.assert_array_equal(out, sol)
         out[:] = 0.0
+    """)
+
+
+@pytest.mark.parametrize("n", [7, 44])
+def test_supg_state_without_room_for_its_staging(stub, n):
+    """A SUPG state is read where the device has no room left for the array
+    that all of it would pass through, and its fields where there is room for
+    one of them; without any, the fields are refused."""
+    _run(stub, f"""
+    m = meshgen.hex_cube({n}, 0.0)
+    g = femx.SUPGSolver(femx.DeviceMesh(m), BoundaryConditions(), rho=1.0, mu=0.01, alpha=1.0, cI=4.0, dt=0.01)
+    sol = np.random.default_rng(1).normal(size=(m.n_nodes, 3))
+    g.set_state(sol)
+    out = np.zeros_like(sol)
+    p = out.ctypes.data_as(C.POINTER(C.c_double))
+    stub.stub_device_max(0)
+    assert femx.load().femx_supg_get_state(g._h, p, None, None, None, None) == 0
+    np.testing.assert_array_equal(out, sol)
+    try:
+        g.get_state()
+        assert False
+    except femx.FemxError as e:
+        assert "hipMalloc" in str(e)
+    stub.stub_device_max(2 * 8 * m.n_elems)
+    np.testing.assert_array_equal(g.get_state()["sol"], sol)
+    stub.stub_device_max(-1)
+    assert femx.load().femx_supg_get_state(g._h, p, None, None, None, None) == 0
     """)
