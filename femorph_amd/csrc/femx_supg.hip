@@ -202,9 +202,9 @@ __device__ __forceinline__ void supg_node(const double F[3], double4 fprev, doub
 //    of one z = +-1/sqrt 3, and hold the element's fields and sums for that z
 //    only.  With one lane per element the same math needed 256 VGPRs, two
 //    waves per SIMD (316 us).
-// Per hexa8 element-step 2 x 2,000 wave-lane instructions against 6,650 node
-// by node; the block kernel at 2.1M hexa 356 -> 277 us mixed, at 85k hexa 47 ->
-// 31 us FP64.
+// Per hexa8 element-step 2 x 2,200 wave-lane instructions against 6,650 node
+// by node; with it the block kernel at 2.1M hexa went from 356 to 277 us mixed
+// (250 now), at 85k hexa from 47 to 31 us FP64 (28).
 // The other lane's value: a DPP quad permute (1, 0, 3, 2).
 __device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
 __device__ __forceinline__ float pair_swap(float v) { return __int_as_float(pair_swap(__float_as_int(v))); }
