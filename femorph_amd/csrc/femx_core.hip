@@ -242,8 +242,9 @@ bool piece(const ReadPiece *p, int n, size_t k, ReadPiece &q) {
   return false;
 }
 
-// Pieces taken from a shared counter: the thread's two chunks alternate, so that the next piece is in flight while one is copied
-// out.  Where no pinned memory is to be had the pieces are copied directly.
+// Pieces taken from a shared counter: the thread's two chunks alternate, so
+// that the next piece is in flight while one is copied out.  Where no pinned
+// memory is to be had the pieces are copied directly.
 hipError_t read_pieces(hipStream_t st, int d, const ReadPiece *p, int n, std::atomic<size_t> &next) {
   Pin c[2];
   ReadPiece in_c[2], q;

@@ -310,9 +310,8 @@ femx_status femx_supg_finish(femx_supg *s, int *steps_done);
  * all members, each by its own number of steps; bit for bit each handle
  * stepped on its own.  Members: FEMX_MIXED hexa8 with B-hat, no fixed DOFs,
  * no diagnostics, more than one element block, and their first step run on
- * their own.  A member's union steps
- * count as enqueued steps of its own: after femx_supg_union_remove,
- * femx_supg_finish checks them for the exit condition (a step past one
+ * their own.  A member's union steps count as enqueued steps of its own:
+ * after femx_supg_union_remove, femx_supg_finish checks them for the exit condition (a step past one
  * whose max |u| exceeded EXITCOND does not run) and femx_supg_get_state
  * reads the state.  While in a union a handle is not stepped, set, read or
  * switched to diagnostics on its own, but for femx_supg_get_log, which waits
@@ -396,9 +395,8 @@ femx_status femx_ffd_morph(const femx_ffd_box *box, int n_points, const double *
  * `n_points` DEVICE-resident points, `coords` [n][3] in and `disp` [n][3]
  * out (device pointers; they may be the same), enqueued on `stream` (a
  * hipStream_t; NULL = the null stream) without allocating, copying or
- * synchronising.  The box and
- * its displacement list are host data, at most 64 displaced control points
- * (13 control points per axis, as femx_ffd_morph).  The control-point
+ * synchronising.  The box and its displacement list are host data, at most 64
+ * displaced control points (13 control points per axis, as femx_ffd_morph).  The control-point
  * lattice goes to a fixed device array of 52,728 bytes per GPU, held until
  * the process ends and shared by every call on that GPU: calls that overlap
  * on one GPU (other streams, other threads) race on it.  The result equals
